@@ -8,18 +8,17 @@
 // C := ((P0 + P1) + ...) + (alpha*op(A)*op(B) + beta*C).
 //
 // Design (MI355X / CDNA4):
-//  * v_mfma_f64_16x16x4_f64.  A workgroup of 4 wave64s owns a 128x128 tile
-//    of C; each wave owns 64x64 = 4x4 MFMA blocks (64 accumulators per lane).
-//  * K advances in stages of 16.  A and B stage tiles are held in LDS as
-//    [k][m] and [k][n] (m / n fastest), double-buffered: the next stage's
-//    global loads are issued before the current stage's MFMAs and written to
-//    the other buffer afterwards, one barrier per stage.
+//  * v_mfma_f64_16x16x4_f64.  A workgroup of 8 wave64s owns a 128x128 tile
+//    of C, each wave 64x32 = 4x2 MFMA blocks; smaller products take 64x64 or
+//    32x32 tiles (pick_tile).
+//  * K advances in stages of 16, loaded direct-to-LDS into a double buffer:
+//    the next stage's loads are issued before the current stage's MFMAs, one
+//    barrier per stage.  Operands that cannot be loaded so are staged through
+//    registers by 4-wave workgroups.
 //  * Transposes are fused into the loads: an operand is either contiguous
 //    along m/n (A as stored, B^T) or along k (A^T, B as stored); both map to
-//    coalesced global reads, and the LDS image is identical, so the MFMA
-//    loop is the same for all four cases.
-//  * LDS addresses are XOR-swizzled per k row, so both the transposing
-//    stores (16 k rows, one column) and the MFMA operand reads (16
+//    coalesced global reads.
+//  * LDS addresses are XOR-swizzled, so that the MFMA operand reads (16
 //    consecutive m or n, two k rows per half wave) hit distinct banks.
 //  * Tiles are visited XCD-contiguously (workgroup b runs on XCD b % 8) and
 //    in groups of 16 tile-rows, so the tiles resident on one XCD share A and
@@ -38,15 +37,34 @@ namespace {
 
 using namespace ca3::gemm;
 
+// Workgroup -> tile origin.  Workgroup b runs on XCD b % 8; tile indices are
+// made XCD-contiguous (gridDim.x is a multiple of 8), so that the workgroups
+// behind one L2 share panels.  False for the workgroups beyond the last tile.
+// The results are put in scalar registers: the quotients come from the vector
+// ALU, and addresses or loop bounds that stay there cost the main loop vector
+// registers and masked branches.
+template <class TL>
+__device__ __forceinline__ bool locate(const GemmArgs &g, int *m0, int *n0)
+{
+    const int tiles = ((g.M + TL::BM - 1) / TL::BM) * ((g.N + TL::BN - 1) / TL::BN);
+    const int nb = gridDim.x;
+    const int t = (blockIdx.x & 7) * (nb >> 3) + (blockIdx.x >> 3);
+    if (t >= tiles) return false;
+    int tm, tn;
+    tile_coords<TL>(t, 1, g.M, g.N, &tm, &tn, g.group);        // nb = 1: no XCD remap here
+    *m0 = __builtin_amdgcn_readfirstlane(tm * TL::BM);
+    *n0 = __builtin_amdgcn_readfirstlane(tn * TL::BN);
+    return true;
+}
+
 template <int TA, int TB, class TL>
 __global__ __launch_bounds__(TL::THREADS, TL::MIN_BLOCKS) void dgemm_kernel(GemmArgs g)
 {
     __shared__ double As[2][kBK * TL::BM];
     __shared__ double Bs[2][kBK * TL::BN];
 
-    int tm, tn;
-    tile_coords<TL>(blockIdx.x, gridDim.x, g.M, g.N, &tm, &tn, g.group);
-    const int m0 = tm * TL::BM, n0 = tn * TL::BN;
+    int m0, n0;
+    if (!locate<TL>(g, &m0, &n0)) return;
 
     // A as stored (TA = 0) is contiguous along m; B as stored (TB = 0) is
     // contiguous along k, B^T along n.
@@ -55,60 +73,34 @@ __global__ __launch_bounds__(TL::THREADS, TL::MIN_BLOCKS) void dgemm_kernel(Gemm
     la.init(g.A, g.lda, m0, g.M);
     lb.init(g.B, g.ldb, n0, g.N);
 
-    f64x4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
-
+    f64x4 acc[TL::FI][TL::FJ];
+    zero(acc);
     mainloop<TL>(la, lb, 0, g.K, m0 + TL::BM <= g.M && n0 + TL::BN <= g.N, As, Bs, acc);
-
     epilogue<TL>(g, m0, n0, acc);
 }
 
-// The 128 x 128 tile with direct-to-LDS stages for its whole k-stages (the
-// k tail through the register-staged checked path).  WA / WB: 4 for 16-byte
-// loads of an operand, 1 for 4-byte loads.  Edge
-// tiles load copies of their last row / column in place of the missing
-// ones; with 16-byte loads that needs an even count of existing rows
-// (columns) where the operand is contiguous along m (n), otherwise the tile
-// runs the checked path throughout.  Same products in the same order as
-// dgemm_kernel<TA, TB, Tile128>.
-template <int TA, int TB, int WA, int WB>
-__global__ __launch_bounds__(kThreads, 2) void dgemm_dtl_kernel(GemmArgs g)
+// The same product with direct-to-LDS stages; needs k >= 16 and edges that
+// can be loaded so (dtl_edge_ok).  WA / WB: 4 for 16-byte loads of an operand,
+// 1 for 4-byte loads.  The same products in the same order as dgemm_kernel,
+// whatever the tile.  WPE: waves per SIMD to leave registers for.
+template <int TA, int TB, int WA, int WB, class TL, int WPE>
+__global__ __launch_bounds__(TL::THREADS, WPE) void dgemm_dtl_kernel(GemmArgs g)
 {
-    __shared__ __attribute__((aligned(1024))) double A0[kBK * kBM], A1[kBK * kBM];
-    __shared__ __attribute__((aligned(1024))) double B0[kBK * kBN], B1[kBK * kBN];
+    __shared__ __attribute__((aligned(1024))) double A0[kBK * TL::BM], A1[kBK * TL::BM];
+    __shared__ __attribute__((aligned(1024))) double B0[kBK * TL::BN], B1[kBK * TL::BN];
 
-    int tm, tn;
-    tile_coords<Tile128>(blockIdx.x, gridDim.x, g.M, g.N, &tm, &tn, g.group);
-    const int m0 = tm * kBM, n0 = tn * kBN;
+    int m0, n0;
+    if (!locate<TL>(g, &m0, &n0)) return;
+    const int mn = min(TL::BM, g.M - m0), nn = min(TL::BN, g.N - n0);
 
-    f64x4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
-
-    int kt0 = 0;
-    const int mn = min(kBM, g.M - m0), nn = min(kBN, g.N - n0);
-    if ((TA || WA == 1 || (mn & 1) == 0) && (!TB || WB == 1 || (nn & 1) == 0) && g.K >= kBK) {
-        DtlLoader<!TA, WA> da;
-        DtlLoader<TB, WB> db;
-        da.init(g.A, g.lda, m0, mn);
-        db.init(g.B, g.ldb, n0, nn);
-        const int nfull = g.K / kBK;
-        mainloop_dtl<!TA, TB>(da, db, g.lda, g.ldb, nfull, A0, A1, B0, B1, acc);
-        kt0 = nfull * kBK;
-    }
-    if (kt0 < g.K) {
-        OperandLoader<!TA> la;
-        OperandLoader<TB> lb;
-        la.init(g.A, g.lda, m0, g.M);
-        lb.init(g.B, g.ldb, n0, g.N);
-        mainloop_checked(la, lb, kt0, g.K, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
-    }
-    epilogue(g, m0, n0, acc);
+    f64x4 acc[TL::FI][TL::FJ];
+    zero(acc);
+    DtlLoader<!TA, WA, TL::BM, TL::NW> da;
+    DtlLoader<TB, WB, TL::BN, TL::NW> db;
+    da.init(g.A, g.lda, m0, mn);
+    db.init(g.B, g.ldb, n0, nn);
+    mainloop_dtl<TL>(da, db, g.lda, g.ldb, 0, g.K, A0, A1, B0, B1, acc);
+    epilogue<TL>(g, m0, n0, acc, dtl_shift<!TA, WA>(mn), dtl_shift<TB, WB>(nn));
 }
 
 // One problem of a batched launch (rank r's product C := sum over its
@@ -116,7 +108,6 @@ __global__ __launch_bounds__(kThreads, 2) void dgemm_dtl_kernel(GemmArgs g)
 // linear tile indices [base, base + tiles_m tiles_n).
 struct BatchProb {
     int M, N, nseg;
-    int dtl;                                   // bit s: segment s may take the direct-to-LDS stages
     int64_t base;
     double *C;
     int64_t ldc;
@@ -135,7 +126,9 @@ struct BatchProb {
 // on the first, 1 after), the bits of one dgemm_dtl_kernel<0, 0> launch
 // per segment.  Otherwise all segments accumulate in registers and the tile
 // is stored once (C = the sum), the bits of the persistent grouped kernel.
-template <bool PER_SEG>
+// DTL: every segment of every problem can take the direct-to-LDS stages;
+// otherwise all are register-staged (the two in one kernel spill).
+template <bool PER_SEG, bool DTL>
 __global__ __launch_bounds__(kThreads, 2) void dgemm_batch_kernel(const BatchProb *__restrict__ probs, int nprob,
                                                                     int64_t total, int group)
 {
@@ -168,30 +161,23 @@ __global__ __launch_bounds__(kThreads, 2) void dgemm_batch_kernel(const BatchPro
     f64x4 acc[4][4];
     for (int s = 0; s < P.nseg; ++s) {
         if (PER_SEG || s == 0) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+            zero(acc);
         }
         const int K = P.k[s];
-        int kt0 = 0;
         int sm0 = m0, sn0 = n0, smn = mn, snn = nn;
         asm volatile("" : "+s"(sm0), "+s"(sn0), "+s"(smn), "+s"(snn));
-        if (((P.dtl >> s) & 1) && (smn & 1) == 0 && K >= kBK) {
+        if (DTL) {
             DtlLoader<1, 4> da;
             DtlLoader<0, 4> db;
             da.init(P.A[s], P.lda[s], sm0, smn);
             db.init(P.B[s], P.ldb[s], sn0, snn);
-            const int nfull = K / kBK;
-            mainloop_dtl<1, 0>(da, db, P.lda[s], P.ldb[s], nfull, A0, A1, B0, B1, acc);
-            kt0 = nfull * kBK;
-        }
-        if (kt0 < K) {
+            mainloop_dtl<Tile128>(da, db, P.lda[s], P.ldb[s], 0, K, A0, A1, B0, B1, acc);
+        } else {
             OperandLoader<1> la;
             OperandLoader<0> lb;
             la.init(P.A[s], P.lda[s], sm0, P.M);
             lb.init(P.B[s], P.ldb[s], sn0, P.N);
-            mainloop_checked(la, lb, kt0, K, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
+            mainloop(la, lb, 0, K, smn == kBM && snn == kBN, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
         }
         if (PER_SEG) {
             // the epilogue's addresses are the same on every segment: keep
@@ -204,25 +190,26 @@ __global__ __launch_bounds__(kThreads, 2) void dgemm_batch_kernel(const BatchPro
             g.C = C;
             g.ldc = ldc;
             g.beta = s ? 1.0 : 0.0;
-            epilogue(g, em0, en0, acc);
+            epilogue(g, em0, en0, acc, DTL ? dtl_shift<1, 4>(mn) : -2);
         }
     }
     if (!PER_SEG) {
-        if (P.nseg == 0) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
-        }
-        epilogue(g, m0, n0, acc);             // alpha = 1, beta = 0: C = the sum as accumulated
+        if (P.nseg == 0) zero(acc);
+        epilogue(g, m0, n0, acc, DTL ? dtl_shift<1, 4>(mn) : -2);       // alpha = 1, beta = 0: C = the sum as accumulated
     }
 }
 
-template <int TA, int TB, int WA, int WB>
+template <class TL>
+int grid_of(const GemmArgs &g)
+{
+    const int64_t wgs = (int64_t) ((g.M + TL::BM - 1) / TL::BM) * ((g.N + TL::BN - 1) / TL::BN);
+    return (int) ((wgs + 7) / 8 * 8);
+}
+
+template <int TA, int TB, int WA, int WB, class TL, int WPE>
 int launch_dtl(const GemmArgs &g)
 {
-    const int tiles = ((g.M + kBM - 1) / kBM) * ((g.N + kBN - 1) / kBN);
-    dgemm_dtl_kernel<TA, TB, WA, WB><<<tiles, kThreads, 0, ca3::stream()>>>(g);
+    dgemm_dtl_kernel<TA, TB, WA, WB, TL, WPE><<<grid_of<TL>(g), TL::THREADS, 0, ca3::stream()>>>(g);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return ca3::fail(e, "dgemm_dtl_kernel");
     return HIP_PROXY_OK;
@@ -231,30 +218,62 @@ int launch_dtl(const GemmArgs &g)
 template <int TA, int TB, class TL>
 int launch_tile(const GemmArgs &g)
 {
-    const int tiles = ((g.M + TL::BM - 1) / TL::BM) * ((g.N + TL::BN - 1) / TL::BN);
-    dgemm_kernel<TA, TB, TL><<<tiles, TL::THREADS, 0, ca3::stream()>>>(g);
+    dgemm_kernel<TA, TB, TL><<<grid_of<TL>(g), TL::THREADS, 0, ca3::stream()>>>(g);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return ca3::fail(e, "dgemm_kernel");
     return HIP_PROXY_OK;
 }
 
-// Workgroup tile: 128 x 128 (4 waves, two workgroups per CU) unless
-// CA3DMM_DGEMM_TILE selects 256x128 or 128x256 (8 waves, one per CU).
-// The 128 x 128 tile loads its whole k-stages direct-to-LDS (6-16 % faster
-// than register staging, same bits) with 16-byte loads, whatever the
-// operand's leading dimension and its address modulo 16 bytes: gfx950
-// serves 16-byte global loads from 8-byte aligned addresses (the compiler
-// itself emits them for such pointers), so a leading dimension of 1333
-// only splits some loads over two cache lines.
-// CA3DMM_DGEMM_LOADS=reg keeps the register-staged stages throughout;
-// CA3DMM_DGEMM_LOADS=dword takes 4-byte loads for both operands (a test
-// form); CA3DMM_DGEMM_LOADS=aligned takes 16-byte loads only for 16-byte
-// aligned operands with even leading dimensions, 4-byte loads for other
-// operands contiguous along m or n, and register staging otherwise.
-int tile_choice()
+// CA3DMM_DGEMM_TILE: the workgroup tile, the library's choice unless it names
+// one.  CA3DMM_DGEMM_LOADS=reg keeps the register-staged stages throughout;
+// =dword takes 4-byte loads for both operands (a test form); =aligned takes
+// 16-byte loads only for 16-byte aligned operands with even leading
+// dimensions, 4-byte loads for other operands contiguous along m or n, and
+// register staging otherwise.  By default whole k-stages are loaded
+// direct-to-LDS (6-16 % faster than register staging, same bits) with 16-byte
+// loads, whatever the operand's leading dimension and its address modulo 16
+// bytes: gfx950 serves 16-byte global loads from 8-byte aligned addresses (the
+// compiler itself emits them for such pointers), so a leading dimension of
+// 1333 only splits some loads over two cache lines.
+enum TileChoice { kTileAuto, kTile128, kTile256x128, kTile128x256, kTile64, kTile32 };
+
+TileChoice tile_choice()
 {
+    static const struct { const char *name; TileChoice tile; } names[] = {
+        {"128x128", kTile128}, {"256x128", kTile256x128}, {"128x256", kTile128x256}, {"64x64", kTile64},
+        {"32x32", kTile32}};
     const char *v = getenv("CA3DMM_DGEMM_TILE");
-    return (v && !strcmp(v, "256x128")) ? 1 : (v && !strcmp(v, "128x256")) ? 2 : 0;
+    for (const auto &t : names)
+        if (v && !strcmp(v, t.name)) return t.tile;
+    return kTileAuto;
+}
+
+// The direct-to-LDS tile for an M x N product from K.  A CU that holds w
+// workgroups takes about a + b w microseconds per 16-deep stage: a is what
+// the stage's latency leaves exposed, b the MFMAs of one tile (measured at
+// 64 x 64 x 2000 to 8192^3; the sum is within a few percent of the runs
+// below).  A smaller tile spreads a small product over more CUs and wastes
+// less on edges and on the last round, but moves more bytes per flop, so it
+// has to be 8 % better to be taken.  Microseconds, 128 / 64 / 32 wide:
+//   600^3  78 / 26 / 16.5    1000^3  125 / 41 / 42    1000 x 2000 x 1000
+//   125 / 71.8 / 76.8    2000^3  247 / 263 / 287    3000^3  1053 / 868 / 976
+//   10000 x 10000 x 500  1515 / 1737 / 1826    8192^3  15150 / 18830 / 21150
+TileChoice pick_tile(int64_t M, int64_t N, int64_t K)
+{
+    static const struct { TileChoice tile; int bm; double a, b; } tiles[] = {
+        {kTile128, 128, 0.15, 1.80}, {kTile64, 64, 0.20, 0.47}, {kTile32, 32, 0.09, 0.135}};
+    const int64_t cus = ca3::cu_count();
+    TileChoice best = kTile128;
+    double t = 0.0;
+    for (const auto &c : tiles) {
+        const int64_t wgs = ((M + c.bm - 1) / c.bm) * ((N + c.bm - 1) / c.bm);
+        const double us = (double) ((K + kBK - 1) / kBK) * (c.a + c.b * (double) ((wgs + cus - 1) / cus));
+        if (c.tile == kTile128 || us < 0.92 * t) {
+            best = c.tile;
+            t = us;
+        }
+    }
+    return best;
 }
 
 // The direct-to-LDS load width of an operand (4 or 1 words), 0 for none
@@ -271,18 +290,27 @@ int dtl_words(const double *P, int64_t ld, bool xc, LoadMode mode)
 template <int TA, int TB>
 int launch(const GemmArgs &g)
 {
-    const int tc = tile_choice();
+    const TileChoice tc = tile_choice();
     const LoadMode mode = load_mode();
-    if (tc == 0 && mode != kLoadsReg) {
-        const int wa = dtl_words(g.A, g.lda, !TA, mode), wb = dtl_words(g.B, g.ldb, TB, mode);
-        if (wa == 4 && wb == 4) return launch_dtl<TA, TB, 4, 4>(g);
-        if (wa == 4 && wb == 1) return launch_dtl<TA, TB, 4, 1>(g);
-        if (wa == 1 && wb == 4) return launch_dtl<TA, TB, 1, 4>(g);
-        if (wa == 1 && wb == 1) return launch_dtl<TA, TB, 1, 1>(g);
+    const bool reg_tile = tc == kTile256x128 || tc == kTile128x256;
+    const int wa = dtl_words(g.A, g.lda, !TA, mode), wb = dtl_words(g.B, g.ldb, TB, mode);
+    // a single row (column) contiguous along m (n) has no pair to load
+    const bool edges = (TA || wa == 1 || g.M > 1) && (!TB || wb == 1 || g.N > 1);
+    if (!reg_tile && wa && wb && edges && g.K >= kBK) {
+        if (wa == 4 && wb == 4) {
+            switch (tc == kTileAuto ? pick_tile(g.M, g.N, g.K) : tc) {
+            case kTile64: return launch_dtl<TA, TB, 4, 4, Tile64, 4>(g);
+            case kTile32: return launch_dtl<TA, TB, 4, 4, Tile32, 4>(g);
+            default: return launch_dtl<TA, TB, 4, 4, Tile128w8, 4>(g);
+            }
+        }
+        if (wa == 4) return launch_dtl<TA, TB, 4, 1, Tile128, 2>(g);
+        if (wb == 4) return launch_dtl<TA, TB, 1, 4, Tile128, 2>(g);
+        return launch_dtl<TA, TB, 1, 1, Tile128, 2>(g);
     }
     switch (tc) {
-    case 1: return launch_tile<TA, TB, Tile256x128>(g);
-    case 2: return launch_tile<TA, TB, Tile128x256>(g);
+    case kTile256x128: return launch_tile<TA, TB, Tile256x128>(g);
+    case kTile128x256: return launch_tile<TA, TB, Tile128x256>(g);
     default: return launch_tile<TA, TB, Tile128>(g);
     }
 }
@@ -338,7 +366,7 @@ struct BatchPlan {
     int nprob = 0;
     int64_t total = 0;
     int group = 16;
-    bool per_segment = true;
+    bool per_segment = true, dtl = false;
 };
 
 int build_batch(const std::vector<Problem> &probs, bool per_segment, BatchPlan **out)
@@ -346,6 +374,7 @@ int build_batch(const std::vector<Problem> &probs, bool per_segment, BatchPlan *
     *out = nullptr;
     std::vector<BatchProb> h;
     int64_t base = 0;
+    bool all_dtl = true;
     const gemm::LoadMode mode = gemm::load_mode();
     for (const Problem &q : probs) {
         if (q.M <= 0 || q.N <= 0) continue;
@@ -363,8 +392,8 @@ int build_batch(const std::vector<Problem> &probs, bool per_segment, BatchPlan *
             b.A[s] = g.A; b.B[s] = g.B;
             b.lda[s] = g.lda; b.ldb[s] = g.ldb;
             b.k[s] = g.k;
-            if (dtl_words(g.A, g.lda, true, mode) == 4 && dtl_words(g.B, g.ldb, false, mode) == 4)
-                b.dtl |= 1 << s;
+            all_dtl = all_dtl && dtl_words(g.A, g.lda, true, mode) == 4 && dtl_words(g.B, g.ldb, false, mode) == 4 &&
+                      g.k >= gemm::kBK && q.M > 1;
         }
         h.push_back(b);
         base += (int64_t) ((q.M + gemm::kBM - 1) / gemm::kBM) * ((q.N + gemm::kBN - 1) / gemm::kBN);
@@ -372,6 +401,7 @@ int build_batch(const std::vector<Problem> &probs, bool per_segment, BatchPlan *
     if ((base + 7) / 8 * 8 > INT_MAX) return ca3::fail_msg(HIP_PROXY_ERR_UNSUPP, "dgemm batch: %lld tiles", (long long) base);
     auto *p = new BatchPlan;
     p->per_segment = per_segment;
+    p->dtl = all_dtl;
     p->nprob = (int) h.size();
     p->total = base;
     const char *v = getenv("CA3DMM_DGEMM_GROUP");
@@ -395,10 +425,9 @@ int run_batch(BatchPlan *p, int group)
     if (p->total == 0) return HIP_PROXY_OK;
     const int grid = (int) ((p->total + 7) / 8 * 8);
     const int G = (group >= 1 && group <= 256) ? group : p->group;
-    if (p->per_segment)
-        dgemm_batch_kernel<true><<<grid, gemm::kThreads, 0, ca3::stream()>>>(p->d, p->nprob, p->total, G);
-    else
-        dgemm_batch_kernel<false><<<grid, gemm::kThreads, 0, ca3::stream()>>>(p->d, p->nprob, p->total, G);
+    auto *kernel = p->per_segment ? (p->dtl ? dgemm_batch_kernel<true, true> : dgemm_batch_kernel<true, false>)
+                                  : (p->dtl ? dgemm_batch_kernel<false, true> : dgemm_batch_kernel<false, false>);
+    kernel<<<grid, gemm::kThreads, 0, ca3::stream()>>>(p->d, p->nprob, p->total, G);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return ca3::fail(e, "dgemm_batch_kernel");
     return ca3::finish();

@@ -23,19 +23,28 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 constexpr int kBM = 128, kBN = 128, kBK = 16, kThreads = 256;
 constexpr int kMaxFoldSrc = 8;
 
-// Workgroup tile BM x BN of C: waves of 64 x 64 (4 x 4 MFMA blocks each),
-// WM along m and WN along n.  128 x 128 (4 waves, two workgroups per CU)
-// is the default; 256 x 128 and 128 x 256 use 8 waves, one workgroup per CU.
-template <int BM_, int BN_>
+// Workgroup tile BM x BN of C: WM x WN waves along m and n, each of FI x FJ
+// MFMA blocks.  Register-staged kernels: 128 x 128 with 4 waves of 64 x 64
+// (two workgroups per CU), 256 x 128 and 128 x 256 with 8 waves (one per CU).
+// Direct-to-LDS kernels: Tile128w8, 8 waves of 64 x 32, whose 122 vector
+// registers leave room for four waves per SIMD (8192^3 TN 15.1 ms; the 4
+// waves of 64 x 64, two per SIMD, 15.45 ms; 10000 x 10000 x 500 1.52 / 1.59
+// ms); Tile64 (8 waves of 32 x 16) and Tile32 (4 waves of 16 x 16) for
+// products whose 128 x 128 tiles leave CUs idle.
+template <int BM_, int BN_, int WM_ = BM_ / 64, int WN_ = BN_ / 64>
 struct TileShape {
     static constexpr int BM = BM_, BN = BN_;
-    static constexpr int WM = BM / 64, WN = BN / 64;
+    static constexpr int WM = WM_, WN = WN_;
+    static constexpr int FI = BM / WM / 16, FJ = BN / WN / 16;
     static constexpr int NW = WM * WN, THREADS = 64 * NW;
     static constexpr int MIN_BLOCKS = THREADS == 256 ? 2 : 1;     // per CU, for __launch_bounds__
 };
 using Tile128 = TileShape<128, 128>;
 using Tile256x128 = TileShape<256, 128>;
 using Tile128x256 = TileShape<128, 256>;
+using Tile128w8 = TileShape<128, 128, 2, 4>;
+using Tile64 = TileShape<64, 64, 2, 4>;
+using Tile32 = TileShape<32, 32, 2, 2>;
 
 struct GemmArgs {
     int M, N, K;
@@ -51,6 +60,15 @@ struct GemmArgs {
     const double *P[kMaxFoldSrc];
     int64_t ldp[kMaxFoldSrc];
 };
+
+template <int FI, int FJ>
+__device__ __forceinline__ void zero(f64x4 (&acc)[FI][FJ])
+{
+#pragma unroll
+    for (int i = 0; i < FI; ++i)
+#pragma unroll
+        for (int j = 0; j < FJ; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+}
 
 // XOR swizzle of column x within LDS row kk (see dgemm.hip header).
 __device__ __forceinline__ int swz(int kk, int x)
@@ -168,7 +186,7 @@ struct OperandLoader {
 // k-slices [KS0, KS1) of the 16 k-steps of MFMAs on the LDS stage (4 x
 // v_mfma_f64_16x16x4 k-slices in all).
 template <class TL = Tile128, int KS0 = 0, int KS1 = kBK / 4>
-__device__ __forceinline__ void stage_mfma(const double *As, const double *Bs, f64x4 (&acc)[4][4])
+__device__ __forceinline__ void stage_mfma(const double *As, const double *Bs, f64x4 (&acc)[TL::FI][TL::FJ])
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = wave % TL::WM, wn = wave / TL::WM;
@@ -176,15 +194,15 @@ __device__ __forceinline__ void stage_mfma(const double *As, const double *Bs, f
 #pragma unroll
     for (int ks = KS0; ks < KS1; ++ks) {
         const int kk = ks * 4 + (lane >> 4);
-        double a[4], b[4];
+        double a[TL::FI], b[TL::FJ];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = As[kk * TL::BM + swz(kk, wm * 64 + i * 16 + li)];
+        for (int i = 0; i < TL::FI; ++i) a[i] = As[kk * TL::BM + swz(kk, (wm * TL::FI + i) * 16 + li)];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) b[j] = Bs[kk * TL::BN + swz(kk, wn * 64 + j * 16 + li)];
+        for (int j = 0; j < TL::FJ; ++j) b[j] = Bs[kk * TL::BN + swz(kk, (wn * TL::FJ + j) * 16 + li)];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < TL::FI; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < TL::FJ; ++j)
                 acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j], a[i], acc[i][j], 0, 0, 0);
     }
 }
@@ -201,7 +219,7 @@ struct LdsPair {
 // As / Bs: double[2][16 * BM] (or LdsPair), As[i] = stage buffer i.
 template <class TL = Tile128, class LA, class LB, class BA, class BB>
 __device__ __forceinline__ void mainloop_checked(LA &la, LB &lb, int kbeg, int kend, BA As, BB Bs,
-                                                 f64x4 (&acc)[4][4])
+                                                 f64x4 (&acc)[TL::FI][TL::FJ])
 {
     if (kend <= kbeg) return;
     const int nk = (kend - kbeg + kBK - 1) / kBK;
@@ -234,7 +252,7 @@ __device__ __forceinline__ void mainloop_checked(LA &la, LB &lb, int kbeg, int k
 // k-steps in the same order, so results do not depend on the path.
 template <class TL = Tile128, class LA, class LB, class BA, class BB>
 __device__ __forceinline__ void mainloop(LA &la, LB &lb, int kbeg, int kend, bool interior, BA As, BB Bs,
-                                         f64x4 (&acc)[4][4])
+                                         f64x4 (&acc)[TL::FI][TL::FJ])
 {
     const int nfull = (interior && kend > kbeg) ? (kend - kbeg) / kBK : 0;
     if (nfull > 0) {
@@ -264,15 +282,13 @@ __device__ __forceinline__ void mainloop(LA &la, LB &lb, int kbeg, int kend, boo
 }
 
 // ---------------------------------------------------------------------
-// Direct-to-LDS stages (whole k-stages of the 128 x 128 DGEMM, 16-byte
-// aligned operands with even leading dimensions): global_load_lds_dwordx4
-// writes lane l's 16 bytes (two doubles) at M0 + 16 l, so one wave
-// instruction fills a 1 KB LDS block; a stage of an operand is 16 blocks
-// (16 k x 128 x), four per wave.  No staging registers and no LDS stores:
-// the loads of stage z + 1 are issued once stage z's operands are read
-// from LDS, and have stage z's MFMAs to land.  Layouts (d = one double):
-//   XC = 1 (contiguous along x): block = one k row of 128 x; 16-byte chunk
-//     c of row k holds x = 2 (c ^ fx(k)), +1 with fx(k) = 8 (k & 1);
+// Direct-to-LDS stages: global_load_lds_dwordx4 writes lane l's 16 bytes
+// (two doubles) at M0 + 16 l, so one wave instruction fills a 1 KB LDS
+// block; a stage of a W-wide operand is W / 8 blocks (16 k x W), dealt to
+// the waves.  No staging registers and no LDS stores.  Layouts (d = one
+// double):
+//   XC = 1 (contiguous along x): k rows of W x, one after the other; 16-byte
+//     chunk c of row k holds x = 2 (c ^ fx(k)), +1 with fx(k) = 8 (k & 1);
 //   XC = 0 (contiguous along k): block = 8 x lines of 16 k; chunk c of line
 //     x holds k = 2 (c ^ hx(x)), +1 with hx(x) = (x >> 1) & 7.
 // Each lane fetches the global chunk its LDS slot holds, so the reads stay
@@ -280,28 +296,47 @@ __device__ __forceinline__ void mainloop(LA &la, LB &lb, int kbeg, int kend, boo
 // distinct banks per 32 lanes.  The k-slices of the MFMAs are those of
 // stage_mfma, so both paths add the same products in the same order.
 // ---------------------------------------------------------------------
-template <int XC>
+template <int XC, int W = 128>
 __device__ __forceinline__ int dtl_index(int k, int x)
 {
-    if (XC) return k * 128 + 2 * ((x >> 1) ^ ((k & 1) << 3)) + (x & 1);
+    if (XC) return k * W + 2 * ((x >> 1) ^ ((k & 1) << 3)) + (x & 1);
     return x * 16 + 2 * ((k >> 1) ^ ((x >> 1) & 7)) + (k & 1);
 }
 
-// Edge tiles: only xn <= 128 x of the tile exist.  A lane whose slot holds
-// an x >= xn loads the last existing x instead, so every load stays inside
-// the operand; those LDS rows hold copies whose products land in C rows or
-// columns the epilogue never stores.  Addresses are a wave-uniform base per
-// block (scalar registers) plus a 32-bit lane offset, which requires
-// 7 * ld * 8 + 128 < 2^32 bytes for XC = 0 (dtl_ld_ok).
+// Edge tiles: only xn <= W x of the tile exist.  A lane whose slot holds an
+// x >= xn loads the last existing x (or x pair) instead, so every load stays
+// inside the operand; those LDS rows hold copies whose products land in C
+// rows or columns the epilogue never stores.  For XC = 1 and odd xn the
+// last chunk holds the pair (xn - 2, xn - 1), one x lower than its slot
+// says: the products of x = xn - 1 come out in row (column) xn of the tile,
+// and the epilogue stores that one in place of row xn - 1 (dtl_shift).
+// Addresses are a wave-uniform base per block (scalar registers) plus a
+// 32-bit lane offset, which requires 7 * ld * 8 + 128 < 2^32 bytes
+// (dtl_ld_ok).
 //
 // WORDS = 4: one 16-byte load per lane and block (global_load_lds_dwordx4)
 // of a double pair, from an 8-byte aligned address (an odd ld or an
 // operand 8 bytes past a 16-byte boundary splits some loads over two
-// cache lines); for XC = 1 it needs an even xn (a chunk holds an x pair).
-// WORDS = 1: four 4-byte loads per lane and block (global_load_lds_dword,
-// lane l of load q lands at M0 + 256 q + 4 l), for any xn; the LDS image
-// is the same.
+// cache lines); for XC = 1 a lone x (xn = 1) needs the x before it (x0 > 0).
+// WORDS = 1 (W = 128 only): four 4-byte loads per lane and block
+// (global_load_lds_dword, lane l of load q lands at M0 + 256 q + 4 l), for
+// any xn, every x in its own slot; otherwise the same LDS image.
 __host__ __device__ constexpr bool dtl_ld_ok(int64_t ld) { return ld >= 0 && ld <= (int64_t) 1 << 26; }
+
+// Whether a tile edge of xn existing x from x0 can be loaded.
+template <int XC, int WORDS>
+__device__ __forceinline__ bool dtl_edge_ok(int x0, int xn)
+{
+    return !XC || WORDS == 1 || xn > 1 || x0 > 0;
+}
+
+// The x of the tile whose products appear one row (column) further on (see
+// above), or -2 for none.
+template <int XC, int WORDS>
+__device__ __forceinline__ int dtl_shift(int xn)
+{
+    return (XC && WORDS == 4 && (xn & 1)) ? xn - 1 : -2;
+}
 
 // Load forms of the direct-to-LDS stages (CA3DMM_DGEMM_LOADS): 16-byte
 // loads from any 8-byte aligned operand (default); "aligned": 16-byte
@@ -311,25 +346,31 @@ __host__ __device__ constexpr bool dtl_ld_ok(int64_t ld) { return ld >= 0 && ld 
 enum LoadMode { kLoads16, kLoadsAligned, kLoadsDword, kLoadsReg };
 LoadMode load_mode();
 
-template <int XC, int WORDS = 4>
+template <int XC_, int WORDS = 4, int W = 128, int NW = 4>
 struct DtlLoader;
 
-template <int XC>
-struct DtlLoader<XC, 4> {
-    const double *base[4];   // block i of this wave for k0 = 0 (wave-uniform)
-    uint32_t off[4];         // this lane's byte offset from base[i]
+template <int XC_, int W, int NW>
+struct DtlLoader<XC_, 4, W, NW> {
+    static constexpr int XC = XC_, WORDS = 4;
+    static constexpr int NB = W / (8 * NW);  // blocks per wave
+    static constexpr int RPB = 128 / W;      // XC: k rows per block
+    const double *base[NB];  // block i of this wave for k0 = 0 (wave-uniform)
+    uint32_t off[NB];        // this lane's byte offset from base[i]
 
-    __device__ __forceinline__ void init(const double *M, int64_t ld, int x0, int xn = 128)
+    __device__ __forceinline__ void init(const double *M, int64_t ld, int x0, int xn = W)
     {
         const int lane = threadIdx.x & 63;
         const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int b = 4 * w + i;
+        for (int i = 0; i < NB; ++i) {
+            const int b = NB * w + i;
             if (XC) {
-                // k row b of the stage; chunk c of the row holds x = 2c, 2c + 1
-                base[i] = M + x0 + (int64_t) b * ld;
-                off[i] = 16u * (uint32_t) min(lane ^ ((b & 1) << 3), (xn >> 1) - 1);
+                // k rows RPB b .. of the stage; chunk c of a row holds x = 2c, 2c + 1
+                const int kr = lane / (W / 2), k = RPB * b + kr;
+                const int x = min(2 * ((lane % (W / 2)) ^ ((k & 1) << 3)), xn - 2);
+                const int back = xn == 1;           // the pair (x0 - 1, x0)
+                base[i] = M + (x0 - back) + (int64_t) (RPB * b) * ld;
+                off[i] = (uint32_t) ((int64_t) kr * ld * 8) + 8u * (uint32_t) (x + back);
             } else {
                 // lines x = 8b .. 8b + 7 of the tile; the lane's k pair is
                 // fixed by its slot (line xl), the line read is x <= xn - 1
@@ -340,15 +381,15 @@ struct DtlLoader<XC, 4> {
         }
     }
 
-    // issue the stage starting at koff (elements) into S (16 x 128 doubles)
+    // issue the stage starting at koff (elements) into S (16 x W doubles)
     __device__ __forceinline__ void issue(int64_t koff, double *S) const
     {
         const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < NB; ++i) {
             const char *g = reinterpret_cast<const char *>(base[i] + koff) + (uint64_t) off[i];
             __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *) g,
-                                             (void __attribute__((address_space(3))) *) (S + (4 * w + i) * 128),
+                                             (void __attribute__((address_space(3))) *) (S + (NB * w + i) * 128),
                                              16, 0, 0);
         }
     }
@@ -359,8 +400,9 @@ struct DtlLoader<XC, 4> {
 // chunk c = 16 q + (l >> 2).  The offsets are rebuilt per stage from a few
 // lane constants (the vector ALU is idle under the MFMAs), so the loader
 // holds as many registers as the 16-byte one.
-template <int XC>
-struct DtlLoader<XC, 1> {
+template <int XC_>
+struct DtlLoader<XC_, 1, 128, 4> {
+    static constexpr int XC = XC_, WORDS = 1;
     const double *M;
     int64_t ld;
     int x0, xn;
@@ -407,32 +449,49 @@ struct DtlLoader<XC, 1> {
     }
 };
 
-template <int XCA, int XCB>
-__device__ __forceinline__ void stage_mfma_dtl(const double *As, const double *Bs, f64x4 (&acc)[4][4])
+// The MFMAs of one stage.  lo > 0 (a stage that overlaps the one before it):
+// the k below lo of the stage count as zero in both operands.
+template <int XCA, int XCB, class TL = Tile128, bool TAIL = false>
+__device__ __forceinline__ void stage_mfma_dtl(const double *As, const double *Bs, f64x4 (&acc)[TL::FI][TL::FJ],
+                                               int lo = 0)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
+    int tid = threadIdx.x;
+    if (TAIL) asm volatile("" : "+v"(tid));      // no address of the tail is computed before the main loop
+    const int lane = tid & 63, wave = tid >> 6;
+    const int wm = wave % TL::WM, wn = wave / TL::WM;
     const int li = lane & 15;
 #pragma unroll
     for (int ks = 0; ks < kBK / 4; ++ks) {
+        if (TAIL && ks * 4 + 4 <= lo) continue;
         const int kk = ks * 4 + (lane >> 4);
-        double a[4], b[4];
+        double a[TL::FI], b[TL::FJ];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = As[dtl_index<XCA>(kk, wm * 64 + i * 16 + li)];
+        for (int i = 0; i < TL::FI; ++i) {
+            a[i] = As[dtl_index<XCA, TL::BM>(kk, (wm * TL::FI + i) * 16 + li)];
+            if (TAIL) a[i] = kk >= lo ? a[i] : 0.0;
+        }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) b[j] = Bs[dtl_index<XCB>(kk, wn * 64 + j * 16 + li)];
+        for (int j = 0; j < TL::FJ; ++j) {
+            b[j] = Bs[dtl_index<XCB, TL::BN>(kk, (wn * TL::FJ + j) * 16 + li)];
+            if (TAIL) b[j] = kk >= lo ? b[j] : 0.0;
+        }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < TL::FI; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < TL::FJ; ++j)
                 acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j], a[i], acc[i][j], 0, 0, 0);
     }
 }
 
-// The whole 16-deep k-stages [0, nfull * 16) of an interior 128 x 128 tile
-// through the direct-to-LDS double buffer (koff(k) = k * ld for XC = 1, k
-// for XC = 0); nothing is loaded for nfull = 0.  Ends with a barrier, after
-// which the caller runs the k tail, if any, through mainloop_checked.
+// k in [kbeg, kend) of a TL tile through a double buffer of direct-to-LDS
+// stages, one in flight under the MFMAs of the other.  Needs kend >= 16
+// (whatever kbeg) and kbeg, kend in scalar registers.  The k left over after
+// the whole 16-deep stages are the last ones of a stage that starts at kend -
+// 16 and is prefetched like the others: it reads some k a second time, which
+// then count as zero.  (A separate bounds-checked stage cost a whole exposed
+// load latency.)  The products are added in the order of k either way, so
+// results do not depend on the path.  Ends with a barrier after which the
+// buffers are free.
 //
 // The two buffers of each operand must be distinct __shared__ arrays and
 // the loop is unrolled by two so that every access names its array at
@@ -440,57 +499,77 @@ __device__ __forceinline__ void stage_mfma_dtl(const double *As, const double *B
 // touch the buffer the DMA of stage z + 1 writes.  With one array indexed
 // by the stage's parity it cannot tell, and makes the first LDS read after
 // each DMA wait for it, which exposes the whole load latency every stage.
-template <int XCA, int XCB, int WA, int WB>
-__device__ __forceinline__ void mainloop_dtl(const DtlLoader<XCA, WA> &la, const DtlLoader<XCB, WB> &lb, int64_t lda,
-                                             int64_t ldb, int nfull, double *A0, double *A1, double *B0,
-                                             double *B1, f64x4 (&acc)[4][4])
+// Rings of three and four stages were slower at every size tried (8192^3
+// 16.4 and 16.9 ms against 15.1): their LDS costs the second workgroup per
+// CU, and other workgroups' waves hide the latency better than depth does.
+template <class TL, class LA, class LB>
+__device__ __forceinline__ void mainloop_dtl(const LA &la, const LB &lb, int64_t lda, int64_t ldb, int kbeg, int kend,
+                                             double *A0, double *A1, double *B0, double *B1,
+                                             f64x4 (&acc)[TL::FI][TL::FJ])
 {
-    auto koff = [](int xc, int64_t ld, int k0) -> int64_t { return xc ? (int64_t) k0 * ld : (int64_t) k0; };
-    // own loads of the stage have landed (vmcnt counts the LDS DMA), then
-    // every wave's; every wave has also finished reading the previous stage
+    constexpr int XCA = LA::XC, XCB = LB::XC;
+    const int nfull = (kend - kbeg) / kBK, rem = (kend - kbeg) % kBK;
+    const int ns = nfull + (rem > 0);
+    auto issue = [&](int z, double *SA, double *SB) __attribute__((always_inline)) {
+        const int64_t k0 = min(kbeg + z * kBK, kend - kBK);
+        la.issue(XCA ? k0 * lda : k0, SA);
+        lb.issue(XCB ? k0 * ldb : k0, SB);
+    };
+    // own loads of the stage have landed (vmcnt counts the LDS DMA) and own
+    // reads of the stage before it are done, then every wave's
     auto publish = []() __attribute__((always_inline)) {
-        __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0); expcnt (6:4) and lgkmcnt (11:8) not waited on
+        __builtin_amdgcn_s_waitcnt(0x0070);     // vmcnt(0) lgkmcnt(0); expcnt (6:4) not waited on
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
-    if (nfull > 0) {
-        la.issue(koff(XCA, lda, 0), A0);
-        lb.issue(koff(XCB, ldb, 0), B0);
+    if (ns > 0) issue(0, A0, B0);
+    for (int z = 0; z < nfull; z += 2) {
+        publish();                              // stage z in buffer 0
+        if (z + 1 < ns) issue(z + 1, A1, B1);
+        stage_mfma_dtl<XCA, XCB, TL>(A0, B0, acc);
+        if (z + 1 >= nfull) break;
+        publish();                              // stage z + 1 in buffer 1
+        if (z + 2 < ns) issue(z + 2, A0, B0);
+        stage_mfma_dtl<XCA, XCB, TL>(A1, B1, acc);
     }
-    for (int kt = 0; kt < nfull; kt += 2) {
-        publish();                              // stage kt in buffer 0
-        if (kt + 1 < nfull) {
-            la.issue(koff(XCA, lda, (kt + 1) * kBK), A1);
-            lb.issue(koff(XCB, ldb, (kt + 1) * kBK), B1);
-        }
-        stage_mfma_dtl<XCA, XCB>(A0, B0, acc);
-        if (kt + 1 >= nfull) break;
-        publish();                              // stage kt + 1 in buffer 1
-        if (kt + 2 < nfull) {
-            la.issue(koff(XCA, lda, (kt + 2) * kBK), A0);
-            lb.issue(koff(XCB, ldb, (kt + 2) * kBK), B0);
-        }
-        stage_mfma_dtl<XCA, XCB>(A1, B1, acc);
+    if (rem > 0) {
+        publish();
+        stage_mfma_dtl<XCA, XCB, TL, true>(nfull & 1 ? A1 : A0, nfull & 1 ? B1 : B0, acc, kBK - rem);
     }
-    __syncthreads();                            // the buffers are free for the caller's tail
+    __syncthreads();
 }
 
-// C := fold(P) + (alpha*acc + beta*C) for the tile at (m0, n0).
+// C := fold(P) + (alpha*acc + beta*C) for the tile at (m0, n0).  ms, ns_:
+// dtl_shift of the tile's rows and columns.
 template <class TL = Tile128>
-__device__ __forceinline__ void epilogue(const GemmArgs &g, int m0, int n0, const f64x4 (&acc)[4][4])
+__device__ __forceinline__ void epilogue(const GemmArgs &g, int m0, int n0, const f64x4 (&acc)[TL::FI][TL::FJ],
+                                         int ms = -2, int ns_ = -2)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = wave % TL::WM, wn = wave / TL::WM;
+    // opaque, so that no row, column or address below is computed before the
+    // main loop and held in vector registers across it
+    m0 = __builtin_amdgcn_readfirstlane(m0);
+    n0 = __builtin_amdgcn_readfirstlane(n0);
+    ms = __builtin_amdgcn_readfirstlane(ms);
+    ns_ = __builtin_amdgcn_readfirstlane(ns_);
+    asm volatile("" : "+s"(m0), "+s"(n0), "+s"(ms), "+s"(ns_));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = m0 + wm * 64 + i * 16 + (lane & 15);
+    for (int i = 0; i < TL::FI; ++i) {
+        int rt = (wm * TL::FI + i) * 16 + (lane & 15);
+        if (rt == ms) continue;
+        rt -= (rt == ms + 1);
+        const int row = m0 + rt;
         if (row >= g.M) continue;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < TL::FJ; ++j) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int col = n0 + wn * 64 + j * 16 + 4 * r + (lane >> 4);
+                int ct = (wn * TL::FJ + j) * 16 + 4 * r + (lane >> 4);
+                if (ct == ns_) continue;
+                ct -= (ct == ns_ + 1);
+                const int col = n0 + ct;
                 if (col >= g.N) continue;
                 double *c = g.C + (int64_t) col * g.ldc + row;
                 double v = ca3::mul_rn(g.alpha, acc[i][j][r]);

@@ -72,16 +72,15 @@ __global__ __launch_bounds__(kThreads, 2) void gram_partial_kernel(GramArgs g)
         for (int j = 0; j < 4; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
     const bool interior = (ti + 1) * kBM <= g.n && (tj + 1) * kBN <= g.n;
     int kt0 = kbeg;
-    if (W > 0 && kend - kbeg >= kBK) {
+    if (W > 0 && g.k >= kBK) {
         // whole stages direct-to-LDS (kbeg is a multiple of 16, so the panels
         // keep A's alignment; edge tiles load copies of their last line in
         // place of the missing ones); the same products in the same order
         DtlLoader<0, 4> da, db;
-        da.init(g.A + kbeg, g.lda, ti * kBM, min(kBM, g.n - ti * kBM));
-        db.init(g.A + kbeg, g.lda, tj * kBN, min(kBN, g.n - tj * kBN));
-        const int nfull = (kend - kbeg) / kBK;
-        mainloop_dtl<0, 0>(da, db, g.lda, g.lda, nfull, A0, A1, B0, B1, acc);
-        kt0 = kbeg + nfull * kBK;
+        da.init(g.A, g.lda, ti * kBM, min(kBM, g.n - ti * kBM));
+        db.init(g.A, g.lda, tj * kBN, min(kBN, g.n - tj * kBN));
+        mainloop_dtl<Tile128>(da, db, g.lda, g.lda, kbeg, kend, A0, A1, B0, B1, acc);
+        kt0 = kend;
     }
     if (kt0 < kend) mainloop(la, lb, kt0, kend, interior, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
     // store the full 128 x 128 partial (rows fastest)
