@@ -27,6 +27,7 @@
 #include <climits>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 
 #include "ca3dmm_ext.h"
 #include "dgemm_tile.h"
@@ -37,24 +38,42 @@ namespace {
 
 using namespace ca3::gemm;
 
-// Workgroup -> tile origin.  Workgroup b runs on XCD b % 8; tile indices are
-// made XCD-contiguous (gridDim.x is a multiple of 8), so that the workgroups
-// behind one L2 share panels.  False for the workgroups beyond the last tile.
-// The results are put in scalar registers: the quotients come from the vector
-// ALU, and addresses or loop bounds that stay there cost the main loop vector
-// registers and masked branches.
+// Workgroup -> tile origin, k range and k split.  Workgroup b runs on XCD
+// b % 8; logical ids are made XCD-contiguous (gridDim.x is a multiple of 8),
+// tiles fastest, so that the workgroups behind one L2 share the panels of
+// neighbouring tiles and, split, of one k range.  False for the workgroups
+// beyond the last tile.  The results are put in scalar registers: the
+// quotients come from the vector ALU, and addresses or loop bounds that stay
+// there cost the main loop vector registers and masked branches.
 template <class TL>
-__device__ __forceinline__ bool locate(const GemmArgs &g, int *m0, int *n0)
+__device__ __forceinline__ bool locate(const GemmArgs &g, int *m0, int *n0, int *kbeg, int *kend, int *split)
 {
     const int tiles = ((g.M + TL::BM - 1) / TL::BM) * ((g.N + TL::BN - 1) / TL::BN);
     const int nb = gridDim.x;
     const int t = (blockIdx.x & 7) * (nb >> 3) + (blockIdx.x >> 3);
-    if (t >= tiles) return false;
+    if (t >= tiles * g.ksplit) return false;
+    const int s = g.ksplit > 1 ? t / tiles : 0;
     int tm, tn;
-    tile_coords<TL>(t, 1, g.M, g.N, &tm, &tn, g.group);        // nb = 1: no XCD remap here
+    tile_coords<TL>(t - s * tiles, 1, g.M, g.N, &tm, &tn, g.group);    // nb = 1: no XCD remap here
     *m0 = __builtin_amdgcn_readfirstlane(tm * TL::BM);
     *n0 = __builtin_amdgcn_readfirstlane(tn * TL::BN);
+    *split = __builtin_amdgcn_readfirstlane(s);
+    *kbeg = *split * g.kstep;
+    *kend = min(g.K, *kbeg + g.kstep);
     return true;
+}
+
+// The epilogue of one split: the product itself, or with ksplit > 1 the bare
+// sum over the split's k range.  (The arguments are passed one by one: a
+// modified copy of g would live in scratch memory, and with it every loop
+// bound read from it.)
+template <class TL>
+__device__ __forceinline__ void store_split(const GemmArgs &g, int split, int m0, int n0,
+                                            const f64x4 (&acc)[TL::FI][TL::FJ], int ms = -2, int ns = -2)
+{
+    const bool whole = g.ksplit == 1;
+    epilogue_to<TL>(g, whole ? g.C : g.part + (int64_t) split * g.M * g.N, whole ? g.ldc : (int64_t) g.M,
+                    whole ? g.alpha : 1.0, whole ? g.beta : 0.0, whole ? g.nsrc : 0, m0, n0, acc, ms, ns);
 }
 
 template <int TA, int TB, class TL>
@@ -63,8 +82,8 @@ __global__ __launch_bounds__(TL::THREADS, TL::MIN_BLOCKS) void dgemm_kernel(Gemm
     __shared__ double As[2][kBK * TL::BM];
     __shared__ double Bs[2][kBK * TL::BN];
 
-    int m0, n0;
-    if (!locate<TL>(g, &m0, &n0)) return;
+    int m0, n0, kbeg, kend, split;
+    if (!locate<TL>(g, &m0, &n0, &kbeg, &kend, &split)) return;
 
     // A as stored (TA = 0) is contiguous along m; B as stored (TB = 0) is
     // contiguous along k, B^T along n.
@@ -75,8 +94,8 @@ __global__ __launch_bounds__(TL::THREADS, TL::MIN_BLOCKS) void dgemm_kernel(Gemm
 
     f64x4 acc[TL::FI][TL::FJ];
     zero(acc);
-    mainloop<TL>(la, lb, 0, g.K, m0 + TL::BM <= g.M && n0 + TL::BN <= g.N, As, Bs, acc);
-    epilogue<TL>(g, m0, n0, acc);
+    mainloop<TL>(la, lb, kbeg, kend, m0 + TL::BM <= g.M && n0 + TL::BN <= g.N, As, Bs, acc);
+    store_split<TL>(g, split, m0, n0, acc);
 }
 
 // The same product with direct-to-LDS stages; needs k >= 16 and edges that
@@ -89,8 +108,8 @@ __global__ __launch_bounds__(TL::THREADS, WPE) void dgemm_dtl_kernel(GemmArgs g)
     __shared__ __attribute__((aligned(1024))) double A0[kBK * TL::BM], A1[kBK * TL::BM];
     __shared__ __attribute__((aligned(1024))) double B0[kBK * TL::BN], B1[kBK * TL::BN];
 
-    int m0, n0;
-    if (!locate<TL>(g, &m0, &n0)) return;
+    int m0, n0, kbeg, kend, split;
+    if (!locate<TL>(g, &m0, &n0, &kbeg, &kend, &split)) return;
     const int mn = min(TL::BM, g.M - m0), nn = min(TL::BN, g.N - n0);
 
     f64x4 acc[TL::FI][TL::FJ];
@@ -99,8 +118,41 @@ __global__ __launch_bounds__(TL::THREADS, WPE) void dgemm_dtl_kernel(GemmArgs g)
     DtlLoader<TB, WB, TL::BN, TL::NW> db;
     da.init(g.A, g.lda, m0, mn);
     db.init(g.B, g.ldb, n0, nn);
-    mainloop_dtl<TL>(da, db, g.lda, g.ldb, 0, g.K, A0, A1, B0, B1, acc);
-    epilogue<TL>(g, m0, n0, acc, dtl_shift<!TA, WA>(mn), dtl_shift<TB, WB>(nn));
+    mainloop_dtl<TL>(da, db, g.lda, g.ldb, kbeg, kend, A0, A1, B0, B1, acc);
+    store_split<TL>(g, split, m0, n0, acc, dtl_shift<!TA, WA>(mn), dtl_shift<TB, WB>(nn));
+}
+
+// C := fold(P) + (alpha * (sum of the splits' partial products) + beta * C).
+// 64 entries per workgroup; wave w adds the splits [w ksplit / 4, (w + 1)
+// ksplit / 4) in order and the four sums are added as (0 + 1) + (2 + 3): a
+// fixed order, and enough loads in flight for a small C with many splits.
+__global__ __launch_bounds__(256) void dgemm_reduce_kernel(GemmArgs g)
+{
+    __shared__ double part[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t size = (int64_t) g.M * g.N, e = (int64_t) blockIdx.x * 64 + lane;
+    const int t0 = w * g.ksplit / 4, t1 = (w + 1) * g.ksplit / 4;
+    double s = 0.0;
+    if (e < size && t0 < t1) {
+        const double *p = g.part + e;
+        s = p[t0 * size];
+#pragma unroll 4
+        for (int t = t0 + 1; t < t1; ++t) s = ca3::add_rn(s, p[t * size]);
+    }
+    part[w][lane] = s;
+    __syncthreads();
+    if (w > 0 || e >= size) return;
+    s = ca3::add_rn(ca3::add_rn(part[0][lane], part[1][lane]), ca3::add_rn(part[2][lane], part[3][lane]));
+    const int64_t col = e / g.M, row = e - col * g.M;
+    double *c = g.C + col * g.ldc + row;
+    double v = ca3::mul_rn(g.alpha, s);
+    if (g.beta != 0.0) v = ca3::add_rn(v, ca3::mul_rn(g.beta, *c));
+    if (g.nsrc > 0) {
+        double f = g.P[0][col * g.ldp[0] + row];
+        for (int t = 1; t < g.nsrc; ++t) f = ca3::add_rn(f, g.P[t][col * g.ldp[t] + row]);
+        v = ca3::add_rn(f, v);
+    }
+    *c = v;
 }
 
 // One problem of a batched launch (rank r's product C := sum over its
@@ -202,7 +254,7 @@ __global__ __launch_bounds__(kThreads, 2) void dgemm_batch_kernel(const BatchPro
 template <class TL>
 int grid_of(const GemmArgs &g)
 {
-    const int64_t wgs = (int64_t) ((g.M + TL::BM - 1) / TL::BM) * ((g.N + TL::BN - 1) / TL::BN);
+    const int64_t wgs = (int64_t) ((g.M + TL::BM - 1) / TL::BM) * ((g.N + TL::BN - 1) / TL::BN) * g.ksplit;
     return (int) ((wgs + 7) / 8 * 8);
 }
 
@@ -248,32 +300,84 @@ TileChoice tile_choice()
     return kTileAuto;
 }
 
-// The direct-to-LDS tile for an M x N product from K.  A CU that holds w
-// workgroups takes about a + b w microseconds per 16-deep stage: a is what
-// the stage's latency leaves exposed, b the MFMAs of one tile (measured at
-// 64 x 64 x 2000 to 8192^3; the sum is within a few percent of the runs
-// below).  A smaller tile spreads a small product over more CUs and wastes
-// less on edges and on the last round, but moves more bytes per flop, so it
-// has to be 8 % better to be taken.  Microseconds, 128 / 64 / 32 wide:
+// How an M x N product from K is cut: the direct-to-LDS tile, and the number
+// of ranges its k is split into.
+//
+// A CU that holds w workgroups takes about a + b w microseconds per 16-deep
+// stage: a is what the stage's latency leaves exposed, b the MFMAs of one tile
+// (measured at 64 x 64 x 2000 to 8192^3; the sum is within a few percent of
+// the runs below).  A smaller tile spreads a small product over more CUs and
+// wastes less on edges and on the last round, but moves more bytes per flop,
+// so it has to be 8 % better to be taken.  Microseconds, 128 / 64 / 32 wide:
 //   600^3  78 / 26 / 16.5    1000^3  125 / 41 / 42    1000 x 2000 x 1000
 //   125 / 71.8 / 76.8    2000^3  247 / 263 / 287    3000^3  1053 / 868 / 976
 //   10000 x 10000 x 500  1515 / 1737 / 1826    8192^3  15150 / 18830 / 21150
-TileChoice pick_tile(int64_t M, int64_t N, int64_t K)
+//
+// Splits are tried at 1, 2, 4 and 8 workgroups per CU, each split at least
+// four stages long and all partial products within the buffer; one costs a
+// second launch (about 6 us) and writing and reading the partials, and has to
+// be 10 % better than none.
+struct Cut {
+    TileChoice tile;
+    int ksplit, stages;                        // stages: 16-deep k-stages per split
+};
+
+constexpr size_t kSplitBytes = (size_t) 64 << 20;
+
+Cut pick_cut(int64_t M, int64_t N, int64_t K, bool may_split)
 {
     static const struct { TileChoice tile; int bm; double a, b; } tiles[] = {
         {kTile128, 128, 0.15, 1.80}, {kTile64, 64, 0.20, 0.47}, {kTile32, 32, 0.09, 0.135}};
-    const int64_t cus = ca3::cu_count();
-    TileChoice best = kTile128;
-    double t = 0.0;
+    const int64_t cus = ca3::cu_count(), stages = (K + kBK - 1) / kBK;
+    Cut best = {kTile128, 1, (int) stages}, split = best;
+    double t = 0.0, ts = 0.0;
     for (const auto &c : tiles) {
         const int64_t wgs = ((M + c.bm - 1) / c.bm) * ((N + c.bm - 1) / c.bm);
-        const double us = (double) ((K + kBK - 1) / kBK) * (c.a + c.b * (double) ((wgs + cus - 1) / cus));
+        const double us = (double) stages * (c.a + c.b * (double) ((wgs + cus - 1) / cus));
         if (c.tile == kTile128 || us < 0.92 * t) {
-            best = c.tile;
+            best.tile = c.tile;
             t = us;
         }
+        for (int r = 1; may_split && r <= 8; r *= 2) {
+            int64_t s = std::min(r * cus / wgs, std::min(stages / 4, (int64_t) (kSplitBytes / 8) / (M * N)));
+            if (s < 2) continue;
+            const int64_t len = (stages + s - 1) / s;
+            s = (stages + len - 1) / len;
+            const double cost = 6.0 + (double) len * (c.a + c.b * (double) ((wgs * s + cus - 1) / cus)) +
+                                (double) (2 * s + 1) * M * N * 8.0 / 4e6;
+            if (s > 1 && (ts == 0.0 || cost < ts)) {
+                split = {c.tile, (int) s, (int) len};
+                ts = cost;
+            }
+        }
     }
-    return best;
+    return ts > 0.0 && ts < 0.9 * t ? split : best;
+}
+
+// The partial products of split calls: one buffer per device, allocated at the
+// first split call and kept.  The mutex is held from before the first to after
+// the second launch of a call, so that calls of several threads, which share
+// the device's stream, do not use it across each other.
+std::mutex g_split_mu;
+double *g_split_buf[16];
+
+// The device's buffer; null where there is none to use: the product then runs
+// unsplit.  Under stream capture that is always so (the captured launches may
+// be replayed beside later calls).
+double *split_buffer()
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ca3::stream(), &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+        (void) hipGetLastError();
+        return nullptr;
+    }
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) return nullptr;
+    if (!g_split_buf[dev] && hipMalloc((void **) &g_split_buf[dev], kSplitBytes) != hipSuccess) {
+        (void) hipGetLastError();              // the failed allocation is not an error of the call
+        g_split_buf[dev] = nullptr;
+    }
+    return g_split_buf[dev];
 }
 
 // The direct-to-LDS load width of an operand (4 or 1 words), 0 for none
@@ -288,7 +392,7 @@ int dtl_words(const double *P, int64_t ld, bool xc, LoadMode mode)
 }
 
 template <int TA, int TB>
-int launch(const GemmArgs &g)
+int launch(const GemmArgs &g, TileChoice best)
 {
     const TileChoice tc = tile_choice();
     const LoadMode mode = load_mode();
@@ -298,7 +402,7 @@ int launch(const GemmArgs &g)
     const bool edges = (TA || wa == 1 || g.M > 1) && (!TB || wb == 1 || g.N > 1);
     if (!reg_tile && wa && wb && edges && g.K >= kBK) {
         if (wa == 4 && wb == 4) {
-            switch (tc == kTileAuto ? pick_tile(g.M, g.N, g.K) : tc) {
+            switch (tc == kTileAuto ? best : tc) {
             case kTile64: return launch_dtl<TA, TB, 4, 4, Tile64, 4>(g);
             case kTile32: return launch_dtl<TA, TB, 4, 4, Tile32, 4>(g);
             default: return launch_dtl<TA, TB, 4, 4, Tile128w8, 4>(g);
@@ -317,7 +421,7 @@ int launch(const GemmArgs &g)
 
 int run(hip_proxy_enum_t transA, hip_proxy_enum_t transB, int m, int n, int k, double alpha,
         const double *A, int ldA, const double *B, int ldB, double beta, double *C, int ldC,
-        int nsrc, const double *const *P, const int *ldp)
+        int nsrc, const double *const *P, const int *ldp, bool may_split)
 {
     const int ta = (transA != HipNoTrans), tb = (transB != HipNoTrans);
     if (m < 0 || n < 0 || k < 0) return ca3::fail_msg(HIP_PROXY_ERR_ARG, "dgemm: negative size");
@@ -344,11 +448,26 @@ int run(hip_proxy_enum_t transA, hip_proxy_enum_t transB, int m, int n, int k, d
         g.P[t] = P[t];
         g.ldp[t] = ldp[t];
     }
+    std::unique_lock<std::mutex> lk(g_split_mu, std::defer_lock);
+    Cut cut = pick_cut(m, n, k, may_split);
+    if (cut.ksplit > 1) {
+        lk.lock();
+        g.part = split_buffer();
+        if (!g.part) cut = pick_cut(m, n, k, false);
+    }
+    g.ksplit = cut.ksplit;
+    g.kstep = std::max(1, cut.stages) * kBK;
     int rc;
-    if (!ta && !tb) rc = launch<0, 0>(g);
-    else if (!ta && tb) rc = launch<0, 1>(g);
-    else if (ta && !tb) rc = launch<1, 0>(g);
-    else rc = launch<1, 1>(g);
+    if (!ta && !tb) rc = launch<0, 0>(g, cut.tile);
+    else if (!ta && tb) rc = launch<0, 1>(g, cut.tile);
+    else if (ta && !tb) rc = launch<1, 0>(g, cut.tile);
+    else rc = launch<1, 1>(g, cut.tile);
+    if (!rc && g.ksplit > 1) {
+        dgemm_reduce_kernel<<<(unsigned) (((int64_t) m * n + 63) / 64), 256, 0, ca3::stream()>>>(g);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) rc = ca3::fail(e, "dgemm_reduce_kernel");
+    }
+    if (lk.owns_lock()) lk.unlock();
     if (rc) return rc;
     return ca3::finish();
 }
@@ -433,6 +552,12 @@ int run_batch(BatchPlan *p, int group)
     return ca3::finish();
 }
 
+int round_product(int m, int n, int k, const double *A, int lda, const double *B, int ldb, double beta, double *C,
+                  int ldc)
+{
+    return ::run(HipNoTrans, HipNoTrans, m, n, k, 1.0, A, lda, B, ldb, beta, C, ldc, 0, nullptr, nullptr, false);
+}
+
 void destroy_batch(BatchPlan *p)
 {
     if (!p) return;
@@ -459,7 +584,7 @@ int hip_dgemm(hip_proxy_enum_t transA, hip_proxy_enum_t transB, const int m, con
               const int k, const double alpha, const double *A, const int ldA, const double *B,
               const int ldB, const double beta, double *C, const int ldC)
 {
-    return run(transA, transB, m, n, k, alpha, A, ldA, B, ldB, beta, C, ldC, 0, nullptr, nullptr);
+    return run(transA, transB, m, n, k, alpha, A, ldA, B, ldB, beta, C, ldC, 0, nullptr, nullptr, true);
 }
 
 int hip_dgemm_fold(hip_proxy_enum_t transA, hip_proxy_enum_t transB, const int m, const int n,
@@ -467,7 +592,7 @@ int hip_dgemm_fold(hip_proxy_enum_t transA, hip_proxy_enum_t transB, const int m
                    const double *B, const int ldB, const double beta, double *C, const int ldC,
                    int nsrc, const double *const *P, const int *ldp)
 {
-    return run(transA, transB, m, n, k, alpha, A, ldA, B, ldB, beta, C, ldC, nsrc, P, ldp);
+    return run(transA, transB, m, n, k, alpha, A, ldA, B, ldB, beta, C, ldC, nsrc, P, ldp, true);
 }
 
 }  // extern "C"

@@ -59,6 +59,10 @@ struct GemmArgs {
     int nsrc;                       // partial-C fold in the epilogue
     const double *P[kMaxFoldSrc];
     int64_t ldp[kMaxFoldSrc];
+    // ksplit > 1: the workgroups of split s accumulate k in [s kstep, (s + 1)
+    // kstep) and store the bare sum to part + s M N (leading dimension M)
+    int ksplit, kstep;
+    double *part;
 };
 
 template <int FI, int FJ>
@@ -540,11 +544,13 @@ __device__ __forceinline__ void mainloop_dtl(const LA &la, const LB &lb, int64_t
     __syncthreads();
 }
 
-// C := fold(P) + (alpha*acc + beta*C) for the tile at (m0, n0).  ms, ns_:
-// dtl_shift of the tile's rows and columns.
-template <class TL = Tile128>
-__device__ __forceinline__ void epilogue(const GemmArgs &g, int m0, int n0, const f64x4 (&acc)[TL::FI][TL::FJ],
-                                         int ms = -2, int ns_ = -2)
+// C := fold(P) + (alpha*acc + beta*C) for the tile at (m0, n0), with the
+// first nsrc partials of g.P.  ms, ns_: dtl_shift of the tile's rows and
+// columns.
+template <class TL>
+__device__ __forceinline__ void epilogue_to(const GemmArgs &g, double *C, int64_t ldc, double alpha, double beta,
+                                            int nsrc, int m0, int n0, const f64x4 (&acc)[TL::FI][TL::FJ], int ms,
+                                            int ns_)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = wave % TL::WM, wn = wave / TL::WM;
@@ -571,18 +577,25 @@ __device__ __forceinline__ void epilogue(const GemmArgs &g, int m0, int n0, cons
                 ct -= (ct == ns_ + 1);
                 const int col = n0 + ct;
                 if (col >= g.N) continue;
-                double *c = g.C + (int64_t) col * g.ldc + row;
-                double v = ca3::mul_rn(g.alpha, acc[i][j][r]);
-                if (g.beta != 0.0) v = ca3::add_rn(v, ca3::mul_rn(g.beta, *c));
-                if (g.nsrc > 0) {
+                double *c = C + (int64_t) col * ldc + row;
+                double v = ca3::mul_rn(alpha, acc[i][j][r]);
+                if (beta != 0.0) v = ca3::add_rn(v, ca3::mul_rn(beta, *c));
+                if (nsrc > 0) {
                     double s = g.P[0][(int64_t) col * g.ldp[0] + row];
-                    for (int t = 1; t < g.nsrc; ++t) s = ca3::add_rn(s, g.P[t][(int64_t) col * g.ldp[t] + row]);
+                    for (int t = 1; t < nsrc; ++t) s = ca3::add_rn(s, g.P[t][(int64_t) col * g.ldp[t] + row]);
                     v = ca3::add_rn(s, v);
                 }
                 *c = v;
             }
         }
     }
+}
+
+template <class TL = Tile128>
+__device__ __forceinline__ void epilogue(const GemmArgs &g, int m0, int n0, const f64x4 (&acc)[TL::FI][TL::FJ],
+                                         int ms = -2, int ns_ = -2)
+{
+    epilogue_to<TL>(g, g.C, g.ldc, g.alpha, g.beta, g.nsrc, m0, n0, acc, ms, ns_);
 }
 
 }  // namespace gemm

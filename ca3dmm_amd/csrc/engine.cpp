@@ -1481,9 +1481,9 @@ int sim_products(ca3dmm_sim *S, void *const *dst_C, const int *ldC)
             const int lk = ce->k_displs[off + 1] - ce->k_displs[off];
             const ca3dmm_engine_p ea = S->eng[cannon_member(P, r, row, off)];
             const ca3dmm_engine_p eb = S->eng[cannon_member(P, r, off, col)];
-            rc = hip_dgemm(HipNoTrans, HipNoTrans, Am, Bn, lk, 1.0, (const double *) ea->A_2dmm_d,
-                           std::max(1, Am), (const double *) eb->B_2dmm_d, std::max(1, lk), s == 0 ? 0.0 : 1.0,
-                           C, std::max(1, Am));
+            rc = ca3::grouped::round_product(Am, Bn, lk, (const double *) ea->A_2dmm_d, std::max(1, Am),
+                                             (const double *) eb->B_2dmm_d, std::max(1, lk), s == 0 ? 0.0 : 1.0, C,
+                                             std::max(1, Am));
         }
     }
     if (rc) return rc;

@@ -100,7 +100,7 @@ void store_tuning_ozaki(const std::string &sig, const OzTuning &t);
 // launch of the direct-to-LDS DGEMM (dgemm.hip): one workgroup per
 // 128 x 128 tile of every problem, its k-segments in order.  per_segment:
 // each segment is added to C as its own product (beta 0 on the first, 1
-// after), so C gets the bits of one hip_dgemm call per segment; otherwise
+// after), so C gets the bits of one round_product per segment; otherwise
 // the segments accumulate in registers and C is stored once, the bits of
 // the persistent grouped kernel.  Segments may have k = 0; folds are not
 // part of it.  The load form (CA3DMM_DGEMM_LOADS) and the tile-row group
@@ -110,6 +110,11 @@ struct BatchPlan;
 int build_batch(const std::vector<Problem> &probs, bool per_segment, BatchPlan **out);
 int run_batch(BatchPlan *p, int group = 0);
 void destroy_batch(BatchPlan *p);
+
+// One segment of one problem as a launch of its own (beta 0 or 1), its k never
+// split over workgroups: the bits of the batched launch.
+int round_product(int m, int n, int k, const double *A, int lda, const double *B, int ldb, double beta, double *C,
+                  int ldc);
 
 // A whole enqueued sequence (every kernel `body` launches on the library
 // stream) captured once into a hipGraph and replayed.  body must not

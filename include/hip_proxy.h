@@ -105,7 +105,11 @@ int hip_dcopy(const int n, const double *x, const int incx, double *y, const int
 
 /* cuda_proxy.h:92-97 (cuda_cublas_dgemm, cuda_proxy.cu:211-230):
  * column-major C := alpha*op(A)*op(B) + beta*C, FP64 MFMA, all four
- * transA/transB cases (HipNoTrans / HipTrans). */
+ * transA/transB cases (HipNoTrans / HipTrans).  The sums run in a fixed order
+ * that depends on m, n and k alone.  Where C is small and k long, k is split
+ * over workgroups, whose partial sums pass through a device buffer of 64 MiB
+ * that the library allocates once and keeps; without it, and under stream
+ * capture, the same product runs unsplit. */
 int hip_dgemm(hip_proxy_enum_t transA, hip_proxy_enum_t transB,
               const int m, const int n, const int k, const double alpha,
               const double *A, const int ldA, const double *B, const int ldB,
