@@ -28,6 +28,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 #include "ca3dmm_ext.h"
 #include "dgemm_tile.h"
@@ -169,23 +170,23 @@ struct BatchProb {
     int k[ca3::grouped::kMaxSeg];
 };
 
-// Every problem's 128 x 128 tiles in one launch, one workgroup per tile
-// (gridDim.x = total tiles rounded up to a multiple of 8).  Linear tile
-// indices are laid out XCD-contiguously over the whole batch, so each XCD
-// works through its own problems' panels; inside a problem tiles are
-// walked in groups of `group` tile-rows.  A tile's segments run in order.
+// Every problem's tiles in one launch, one workgroup per tile (gridDim.x =
+// total tiles rounded up to a multiple of 8).  Linear tile indices are laid
+// out XCD-contiguously over the whole batch, so each XCD works through its
+// own problems' panels; inside a problem tiles are walked in groups of
+// `group` tile-rows.  A tile's segments run in order.
 // PER_SEG: each segment is its own product added by the epilogue (beta 0
 // on the first, 1 after), the bits of one dgemm_dtl_kernel<0, 0> launch
 // per segment.  Otherwise all segments accumulate in registers and the tile
 // is stored once (C = the sum), the bits of the persistent grouped kernel.
 // DTL: every segment of every problem can take the direct-to-LDS stages;
 // otherwise all are register-staged (the two in one kernel spill).
-template <bool PER_SEG, bool DTL>
-__global__ __launch_bounds__(kThreads, 2) void dgemm_batch_kernel(const BatchProb *__restrict__ probs, int nprob,
-                                                                    int64_t total, int group)
+template <bool PER_SEG, bool DTL, class TL, int WPE>
+__global__ __launch_bounds__(TL::THREADS, WPE) void dgemm_batch_kernel(const BatchProb *__restrict__ probs, int nprob,
+                                                                      int64_t total, int group)
 {
-    __shared__ __attribute__((aligned(1024))) double A0[kBK * kBM], A1[kBK * kBM];
-    __shared__ __attribute__((aligned(1024))) double B0[kBK * kBN], B1[kBK * kBN];
+    __shared__ __attribute__((aligned(1024))) double A0[kBK * TL::BM], A1[kBK * TL::BM];
+    __shared__ __attribute__((aligned(1024))) double B0[kBK * TL::BN], B1[kBK * TL::BN];
 
     const int64_t nb = gridDim.x;
     int64_t t = blockIdx.x;
@@ -199,9 +200,9 @@ __global__ __launch_bounds__(kThreads, 2) void dgemm_batch_kernel(const BatchPro
     }
     const BatchProb &P = probs[lo];
     int tm, tn;
-    tile_coords<Tile128>((int) (t - P.base), 1, P.M, P.N, &tm, &tn, group);   // nb = 1: no XCD remap here
-    const int m0 = tm * kBM, n0 = tn * kBN;
-    const int mn = min(kBM, P.M - m0), nn = min(kBN, P.N - n0);
+    tile_coords<TL>((int) (t - P.base), 1, P.M, P.N, &tm, &tn, group);   // nb = 1: no XCD remap here
+    const int m0 = __builtin_amdgcn_readfirstlane(tm * TL::BM), n0 = __builtin_amdgcn_readfirstlane(tn * TL::BN);
+    const int mn = min(TL::BM, P.M - m0), nn = min(TL::BN, P.N - n0);
 
     GemmArgs g;
     g.M = P.M; g.N = P.N;
@@ -210,26 +211,24 @@ __global__ __launch_bounds__(kThreads, 2) void dgemm_batch_kernel(const BatchPro
     g.beta = 0.0;
     g.C = P.C; g.ldc = P.ldc;
     g.nsrc = 0;
-    f64x4 acc[4][4];
+    f64x4 acc[TL::FI][TL::FJ];
     for (int s = 0; s < P.nseg; ++s) {
-        if (PER_SEG || s == 0) {
-            zero(acc);
-        }
+        if (PER_SEG || s == 0) zero(acc);
         const int K = P.k[s];
         int sm0 = m0, sn0 = n0, smn = mn, snn = nn;
         asm volatile("" : "+s"(sm0), "+s"(sn0), "+s"(smn), "+s"(snn));
-        if (DTL) {
-            DtlLoader<1, 4> da;
-            DtlLoader<0, 4> db;
+        if constexpr (DTL) {
+            DtlLoader<1, 4, TL::BM, TL::NW> da;
+            DtlLoader<0, 4, TL::BN, TL::NW> db;
             da.init(P.A[s], P.lda[s], sm0, smn);
             db.init(P.B[s], P.ldb[s], sn0, snn);
-            mainloop_dtl<Tile128>(da, db, P.lda[s], P.ldb[s], 0, K, A0, A1, B0, B1, acc);
+            mainloop_dtl<TL>(da, db, P.lda[s], P.ldb[s], 0, K, A0, A1, B0, B1, acc);
         } else {
-            OperandLoader<1> la;
-            OperandLoader<0> lb;
+            OperandLoader<1, TL::BM, TL::THREADS> la;
+            OperandLoader<0, TL::BN, TL::THREADS> lb;
             la.init(P.A[s], P.lda[s], sm0, P.M);
             lb.init(P.B[s], P.ldb[s], sn0, P.N);
-            mainloop(la, lb, 0, K, smn == kBM && snn == kBN, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
+            mainloop<TL>(la, lb, 0, K, smn == TL::BM && snn == TL::BN, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
         }
         if (PER_SEG) {
             // the epilogue's addresses are the same on every segment: keep
@@ -242,12 +241,12 @@ __global__ __launch_bounds__(kThreads, 2) void dgemm_batch_kernel(const BatchPro
             g.C = C;
             g.ldc = ldc;
             g.beta = s ? 1.0 : 0.0;
-            epilogue(g, em0, en0, acc, DTL ? dtl_shift<1, 4>(mn) : -2);
+            epilogue<TL>(g, em0, en0, acc, DTL ? dtl_shift<1, 4>(mn) : -2);
         }
     }
     if (!PER_SEG) {
         if (P.nseg == 0) zero(acc);
-        epilogue(g, m0, n0, acc, DTL ? dtl_shift<1, 4>(mn) : -2);       // alpha = 1, beta = 0: C = the sum as accumulated
+        epilogue<TL>(g, m0, n0, acc, DTL ? dtl_shift<1, 4>(mn) : -2);       // alpha = 1, beta = 0: C = the sum
     }
 }
 
@@ -317,6 +316,14 @@ TileChoice tile_choice()
 // four stages long and all partial products within the buffer; one costs a
 // second launch (about 6 us) and writing and reading the partials, and has to
 // be 10 % better than none.
+struct TileCost {
+    TileChoice tile;
+    int bm;
+    double a, b;
+};
+constexpr TileCost kTileCosts[] = {
+    {kTile128, 128, 0.15, 1.80}, {kTile64, 64, 0.20, 0.47}, {kTile32, 32, 0.09, 0.135}};
+
 struct Cut {
     TileChoice tile;
     int ksplit, stages;                        // stages: 16-deep k-stages per split
@@ -326,12 +333,10 @@ constexpr size_t kSplitBytes = (size_t) 64 << 20;
 
 Cut pick_cut(int64_t M, int64_t N, int64_t K, bool may_split)
 {
-    static const struct { TileChoice tile; int bm; double a, b; } tiles[] = {
-        {kTile128, 128, 0.15, 1.80}, {kTile64, 64, 0.20, 0.47}, {kTile32, 32, 0.09, 0.135}};
     const int64_t cus = ca3::cu_count(), stages = (K + kBK - 1) / kBK;
     Cut best = {kTile128, 1, (int) stages}, split = best;
     double t = 0.0, ts = 0.0;
-    for (const auto &c : tiles) {
+    for (const TileCost &c : kTileCosts) {
         const int64_t wgs = ((M + c.bm - 1) / c.bm) * ((N + c.bm - 1) / c.bm);
         const double us = (double) stages * (c.a + c.b * (double) ((wgs + cus - 1) / cus));
         if (c.tile == kTile128 || us < 0.92 * t) {
@@ -486,13 +491,13 @@ struct BatchPlan {
     int64_t total = 0;
     int group = 16;
     bool per_segment = true, dtl = false;
+    TileChoice tile = kTile128;                // register-staged plans: always 128 x 128
 };
 
 int build_batch(const std::vector<Problem> &probs, bool per_segment, BatchPlan **out)
 {
     *out = nullptr;
     std::vector<BatchProb> h;
-    int64_t base = 0;
     bool all_dtl = true;
     const gemm::LoadMode mode = gemm::load_mode();
     for (const Problem &q : probs) {
@@ -502,7 +507,6 @@ int build_batch(const std::vector<Problem> &probs, bool per_segment, BatchPlan *
         BatchProb b;
         memset(&b, 0, sizeof(b));
         b.M = q.M; b.N = q.N; b.nseg = q.nseg;
-        b.base = base;
         b.C = q.C; b.ldc = q.ldc;
         for (int s = 0; s < q.nseg; ++s) {
             const Seg &g = q.seg[s];
@@ -515,12 +519,39 @@ int build_batch(const std::vector<Problem> &probs, bool per_segment, BatchPlan *
                       g.k >= gemm::kBK && q.M > 1;
         }
         h.push_back(b);
-        base += (int64_t) ((q.M + gemm::kBM - 1) / gemm::kBM) * ((q.N + gemm::kBN - 1) / gemm::kBN);
+    }
+    // the tile whose rounds of workgroups cost least, by the rule of a single
+    // product: a CU takes a + b w per stage for its w workgroups, over the
+    // mean number of stages of a tile
+    TileChoice tile = kTile128;
+    int64_t base = 0;
+    double best = 0.0;
+    for (const TileCost &c : kTileCosts) {
+        int64_t wgs = 0, work = 0;
+        for (const BatchProb &b : h) {
+            const int64_t n = (int64_t) ((b.M + c.bm - 1) / c.bm) * ((b.N + c.bm - 1) / c.bm);
+            int64_t stages = 0;
+            for (int s = 0; s < b.nseg; ++s) stages += (b.k[s] + gemm::kBK - 1) / gemm::kBK;
+            wgs += n;
+            work += n * stages;
+        }
+        const double us = wgs ? (double) work / (double) wgs *
+                                    (c.a + c.b * (double) ((wgs + ca3::cu_count() - 1) / ca3::cu_count()))
+                              : 0.0;
+        if (c.tile != kTile128 && !(all_dtl && us < 0.92 * best)) continue;
+        tile = c.tile;
+        best = us;
+        base = 0;
+        for (BatchProb &b : h) {
+            b.base = base;
+            base += (int64_t) ((b.M + c.bm - 1) / c.bm) * ((b.N + c.bm - 1) / c.bm);
+        }
     }
     if ((base + 7) / 8 * 8 > INT_MAX) return ca3::fail_msg(HIP_PROXY_ERR_UNSUPP, "dgemm batch: %lld tiles", (long long) base);
     auto *p = new BatchPlan;
     p->per_segment = per_segment;
     p->dtl = all_dtl;
+    p->tile = tile;
     p->nprob = (int) h.size();
     p->total = base;
     const char *v = getenv("CA3DMM_DGEMM_GROUP");
@@ -544,9 +575,18 @@ int run_batch(BatchPlan *p, int group)
     if (p->total == 0) return HIP_PROXY_OK;
     const int grid = (int) ((p->total + 7) / 8 * 8);
     const int G = (group >= 1 && group <= 256) ? group : p->group;
-    auto *kernel = p->per_segment ? (p->dtl ? dgemm_batch_kernel<true, true> : dgemm_batch_kernel<true, false>)
-                                  : (p->dtl ? dgemm_batch_kernel<false, true> : dgemm_batch_kernel<false, false>);
-    kernel<<<grid, gemm::kThreads, 0, ca3::stream()>>>(p->d, p->nprob, p->total, G);
+    auto go = [&](auto per_seg) {
+        constexpr bool S = decltype(per_seg)::value;
+        hipStream_t st = ca3::stream();
+        if (!p->dtl) dgemm_batch_kernel<S, false, Tile128, 2><<<grid, 256, 0, st>>>(p->d, p->nprob, p->total, G);
+        else if (p->tile == kTile64)
+            dgemm_batch_kernel<S, true, Tile64, 4><<<grid, 512, 0, st>>>(p->d, p->nprob, p->total, G);
+        else if (p->tile == kTile32)
+            dgemm_batch_kernel<S, true, Tile32, 4><<<grid, 256, 0, st>>>(p->d, p->nprob, p->total, G);
+        else dgemm_batch_kernel<S, true, Tile128w8, 4><<<grid, 512, 0, st>>>(p->d, p->nprob, p->total, G);
+    };
+    if (p->per_segment) go(std::true_type{});
+    else go(std::false_type{});
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return ca3::fail(e, "dgemm_batch_kernel");
     return ca3::finish();

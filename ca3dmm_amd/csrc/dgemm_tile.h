@@ -19,6 +19,7 @@ namespace ca3 {
 namespace gemm {
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) double gdouble;     // in global memory (a pointer read from a table is generic)
 
 constexpr int kBM = 128, kBN = 128, kBK = 16, kThreads = 256;
 constexpr int kMaxFoldSrc = 8;
@@ -564,30 +565,64 @@ __device__ __forceinline__ void epilogue_to(const GemmArgs &g, double *C, int64_
 #pragma unroll
     for (int i = 0; i < TL::FI; ++i) {
         int rt = (wm * TL::FI + i) * 16 + (lane & 15);
-        if (rt == ms) continue;
+        const bool rok = rt != ms && m0 + rt - (rt == ms + 1) < g.M;
         rt -= (rt == ms + 1);
         const int row = m0 + rt;
-        if (row >= g.M) continue;
+        // a block row at a time, so that its loads of C and of the partials
+        // are in flight together (one by one, their latencies add up)
+        bool ok[TL::FJ][4];
+        int col[TL::FJ][4];
 #pragma unroll
-        for (int j = 0; j < TL::FJ; ++j) {
+        for (int j = 0; j < TL::FJ; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                int ct = (wn * TL::FJ + j) * 16 + 4 * r + (lane >> 4);
-                if (ct == ns_) continue;
-                ct -= (ct == ns_ + 1);
-                const int col = n0 + ct;
-                if (col >= g.N) continue;
-                double *c = C + (int64_t) col * ldc + row;
-                double v = ca3::mul_rn(alpha, acc[i][j][r]);
-                if (beta != 0.0) v = ca3::add_rn(v, ca3::mul_rn(beta, *c));
-                if (nsrc > 0) {
-                    double s = g.P[0][(int64_t) col * g.ldp[0] + row];
-                    for (int t = 1; t < nsrc; ++t) s = ca3::add_rn(s, g.P[t][(int64_t) col * g.ldp[t] + row]);
-                    v = ca3::add_rn(s, v);
-                }
-                *c = v;
+                const int ct = (wn * TL::FJ + j) * 16 + 4 * r + (lane >> 4);
+                col[j][r] = n0 + ct - (ct == ns_ + 1);
+                ok[j][r] = rok && ct != ns_ && col[j][r] < g.N;
             }
+        double v[TL::FJ][4], x[TL::FJ][4];
+        auto load = [&](const double *X, int64_t ldx) __attribute__((always_inline)) {
+            const gdouble *Xg = (const gdouble *) X;
+#pragma unroll
+            for (int j = 0; j < TL::FJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) x[j][r] = ok[j][r] ? Xg[(int64_t) col[j][r] * ldx + row] : 0.0;
+        };
+#pragma unroll
+        for (int j = 0; j < TL::FJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[j][r] = ca3::mul_rn(alpha, acc[i][j][r]);
+        if (beta != 0.0) {
+            load(C, ldc);
+#pragma unroll
+            for (int j = 0; j < TL::FJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[j][r] = ca3::add_rn(v[j][r], ca3::mul_rn(beta, x[j][r]));
         }
+        if (nsrc > 0) {
+            double s[TL::FJ][4];
+            load(g.P[0], g.ldp[0]);
+#pragma unroll
+            for (int j = 0; j < TL::FJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[j][r] = x[j][r];
+            for (int t = 1; t < nsrc; ++t) {
+                load(g.P[t], g.ldp[t]);
+#pragma unroll
+                for (int j = 0; j < TL::FJ; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s[j][r] = ca3::add_rn(s[j][r], x[j][r]);
+            }
+#pragma unroll
+            for (int j = 0; j < TL::FJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[j][r] = ca3::add_rn(s[j][r], v[j][r]);
+        }
+#pragma unroll
+        for (int j = 0; j < TL::FJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (ok[j][r]) ((gdouble *) C)[(int64_t) col[j][r] * ldc + row] = v[j][r];
     }
 }
 

@@ -97,8 +97,9 @@ bool lookup_tuning_ozaki(const std::string &sig, OzTuning *t);
 void store_tuning_ozaki(const std::string &sig, const OzTuning &t);
 
 // The same problems (every operand NN, as stored) as one non-persistent
-// launch of the direct-to-LDS DGEMM (dgemm.hip): one workgroup per
-// 128 x 128 tile of every problem, its k-segments in order.  per_segment:
+// launch of the direct-to-LDS DGEMM (dgemm.hip): one workgroup per tile of
+// every problem (128 x 128, or smaller where that leaves CUs idle), its
+// k-segments in order.  per_segment:
 // each segment is added to C as its own product (beta 0 on the first, 1
 // after), so C gets the bits of one round_product per segment; otherwise
 // the segments accumulate in registers and C is stored once, the bits of
