@@ -5,15 +5,14 @@
 // calls of examples/example_CholeskyQR.c:120-139.
 //
 //   hip_dpotrf(U)   blocked right-looking Cholesky A = R^T R over 64-wide
-//                   block columns: the diagonal block factored in LDS by one
-//                   workgroup, the block row R_jj^{-T} A_j,rest by forward
-//                   substitution (one wave per column), the trailing upper
-//                   triangle updated by the FP64 MFMA Gram (hip_dsyrk_gram,
-//                   alpha = -1, beta = 1).  The strictly lower part of A is
-//                   not touched.  Returns LAPACK's info (k+1 when the pivot k
-//                   is not > 0).
-//   hip_dtrtri_upper  R^{-1} for upper-triangular R: one workgroup per
-//                   column j solves R x = e_j by a column sweep in LDS.
+//                   block rows, two launches each: the block row (diagonal
+//                   block and R_jj^{-T} A_j,rest) and the FP64 MFMA update of
+//                   the trailing upper triangle.  The strictly lower part of
+//                   A is not touched.  Returns LAPACK's info (k+1 when the
+//                   pivot k is not > 0).
+//   hip_dtrtri_upper  R^{-1} for upper-triangular R: the 64 x 64 diagonal
+//                   blocks in one launch, then pairs of inverted blocks
+//                   joined by FP64 MFMA products, the block size doubling.
 //   hip_dtrsm(R,U,N,N)  B := alpha * B * R^{-1}: R^{-1} (trtri) followed by
 //                   one FP64 MFMA DGEMM per column block of the result, each
 //                   reading only the non-zero rows of R^{-1}; blocks are
@@ -22,101 +21,363 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 #include "ca3dmm_ext.h"
+#include "dgemm_tile.h"
 #include "hip_common.h"
 
 namespace {
 
-constexpr int kMaxN = 8192;            // potrf / trtri keep one column in LDS
+constexpr int kMaxN = 8192;            // the documented limit of the factorizations
 
-constexpr int kPb = 64;                // block width of the blocked Cholesky
+constexpr int kPb = 64;                // block width of the Cholesky and of the inverse
 
-// The jb x jb diagonal block at A(j0, j0) (its upper triangle) factored in
-// LDS: R_jj with R_jj^T R_jj = A_jj.  info: 0 written by the first block;
-// a later block does nothing once info is set, and writes j0 + k + 1 when
-// its pivot k is not > 0.
-__global__ __launch_bounds__(256) void potrf_diag_kernel(double *A, int64_t lda, int j0, int jb, int *info)
+__device__ __forceinline__ double readlane(double v, int lane)
 {
-    __shared__ double L[kPb][kPb + 1];     // L[j][i] = A(j0 + i, j0 + j), i <= j
-    __shared__ int bad;
-    const int t = threadIdx.x;
+    const uint64_t u = __double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readlane((int) (uint32_t) u, lane);
+    const uint32_t hi = __builtin_amdgcn_readlane((int) (uint32_t) (u >> 32), lane);
+    return __longlong_as_double((long long) (((uint64_t) hi << 32) | lo));
+}
+
+// v of lane I of the row of 16 lanes that the lane is in
+template <int I>
+__device__ __forceinline__ double row_lane(double v)
+{
+    const uint64_t u = (uint64_t) __double_as_longlong(v);
+    const int lo = (int) (uint32_t) u, hi = (int) (uint32_t) (u >> 32);
+    const uint32_t l = __builtin_amdgcn_update_dpp(lo, lo, 0x150 + I, 0xf, 0xf, true);     // row_newbcast:I
+    const uint32_t h = __builtin_amdgcn_update_dpp(hi, hi, 0x150 + I, 0xf, 0xf, true);
+    return __longlong_as_double((long long) (((uint64_t) h << 32) | l));
+}
+
+template <int I, int N, class F>
+__device__ __forceinline__ void unrolled(const F &f)
+{
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        unrolled<I + 1, N>(f);
+    }
+}
+
+// 16 steps of the factorization of the 16 x 16 block d, held by every row of
+// 16 lanes (lane = column, register = row), and of the columns r.  False if a
+// pivot is outside [2^-900, 2^900] (not positive ones among them): r is then
+// of no use.  The square root and its reciprocal come from Goldschmidt's
+// iteration, the quotients from the reciprocal and one correction, which
+// leaves them as the division would round them; no branch splits the chain,
+// so that a step's updates fill the next one's latencies.
+__device__ __forceinline__ bool eliminate16(double (&d)[16], double (&r)[16], bool first, int col)
+{
+    bool ok = true;
+    unrolled<0, 16>([&](auto K) {
+        constexpr int k = decltype(K)::value;
+        const double p = row_lane<k>(d[k]);
+        ok = ok && p >= 0x1p-900 && p <= 0x1p900;
+        const double y = __builtin_amdgcn_rsq(p);
+        double g = p * y, h = 0.5 * y, e = fma(-h, g, 0.5);
+        g = fma(g, e, g);
+        h = fma(h, e, h);
+        e = fma(-h, g, 0.5);
+        g = fma(g, e, g);
+        h = fma(h, e, h);
+        const double piv = fma(fma(-g, g, p), h, g);
+        double inv = h + h;
+        inv = fma(fma(-inv, piv, 1.0), inv, inv);
+        const double qd = d[k] * inv, qr = r[k] * inv;
+        d[k] = col == k ? piv : fma(fma(-qd, piv, d[k]), inv, qd);
+        r[k] = first && col == k ? piv : fma(fma(-qr, piv, r[k]), inv, qr);
+        unrolled<k + 1, 16>([&](auto I) {
+            constexpr int i = decltype(I)::value;
+            const double f = -row_lane<i>(d[k]);
+            d[i] = fma(f, d[k], d[i]);
+            r[i] = fma(f, r[k], r[i]);
+        });
+    });
+    return ok;
+}
+
+// Block row j0 of the factorization: R_jj of the jb x jb diagonal block and
+// X = R_jj^{-T} A(j0 : j0 + jb, c) for the columns c right of it, 64 columns
+// per workgroup.  Every workgroup factors the diagonal block itself, so that
+// the solve needs no second launch behind it; workgroup 0 stores it, to Rjj
+// (leading dimension 64) where other workgroups may still read A's.
+//
+// The block row is a 64 x 128 array in LDS.  16 rows at a time: lane = column,
+// the 16 rows in registers of two waves, which both also hold the 16 x 16
+// diagonal block, so that no barrier falls between two pivots; then the rows
+// below are updated by MFMAs.  The chain of 64 pivots (square root, quotient,
+// first update) bounds it.
+//
+// info: 0 written by the first block row; a later one does nothing once info
+// is set, and writes j0 + k + 1 when its pivot k is not > 0.
+__global__ __launch_bounds__(256) void potrf_row_kernel(double *A, int64_t lda, int j0, int jb, int n, double *Rjj,
+                                                        int *info)
+{
+    constexpr int LD = 2 * kPb + 1;
+    __shared__ double W[kPb][LD];           // W[i][j]: row i; columns j < 64 the diagonal block, then the 64 others
+    __shared__ int bad, plain;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     if (j0 > 0 && *info) return;
-    if (t == 0) bad = 0;
-    double *D = A + (int64_t) j0 * lda + j0;
-    for (int e = t; e < jb * jb; e += 256) {
-        const int i = e % jb, j = e / jb;
-        if (i <= j) L[j][i] = D[(int64_t) j * lda + i];
+    const int c0 = j0 + jb + (int) blockIdx.x * kPb, nc = min(kPb, n - c0);
+    double *D = A + (int64_t) j0 * lda + j0, *S = A + (int64_t) c0 * lda + j0;
+    if (t == 0) bad = plain = 0;
+    // beyond jb the identity, below the diagonal and beyond nc zeros
+#pragma unroll
+    for (int q = 0; q < kPb / 4; ++q) {
+        const int j = wave + 4 * q;
+        W[lane][j] = (lane <= j && j < jb) ? D[(int64_t) j * lda + lane] : (lane == j ? 1.0 : 0.0);
+        W[lane][kPb + j] = (lane < jb && j < nc) ? S[(int64_t) j * lda + lane] : 0.0;
     }
     __syncthreads();
-    for (int k = 0; k < jb; ++k) {
-        if (t == 0) {
-            const double d = L[k][k];
-            if (!(d > 0.0)) bad = k + 1;
-            else L[k][k] = sqrt(d);
+    for (int s = 0; s < kPb; s += 16) {
+        double r[16], d[16];
+        bool ok = true;
+        if (wave < 2) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                r[i] = W[s + i][t];
+                d[i] = W[s + i][s + (lane & 15)];
+            }
+            ok = eliminate16(d, r, (t & ~15) == s, lane & 15);
+            if (t == 0 && !ok) plain = 1;
+        }
+        __syncthreads();                   // both waves have read the diagonal block before one stores it
+        if (plain) {
+            // an extreme pivot in these 16 rows: the same steps in LDS, by
+            // square root and division
+            for (int k = s; k < s + 16; ++k) {
+                const double p = W[k][k];
+                __syncthreads();
+                if (!(p > 0.0)) {
+                    if (t == 0) bad = k + 1;
+                    break;
+                }
+                const double piv = sqrt(p);
+                if (t >= k && t < 2 * kPb) W[k][t] = t == k ? piv : W[k][t] / piv;
+                __syncthreads();
+                if (t > k && t < 2 * kPb)
+                    for (int i = k + 1; i < s + 16; ++i) W[i][t] = fma(-W[k][i], W[k][t], W[i][t]);
+                __syncthreads();
+            }
+            __syncthreads();
+            if (t == 0) plain = 0;
+        } else if (t >= s && wave < 2) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) W[s + i][t] = r[i];
         }
         __syncthreads();
         if (bad) break;
-        const double piv = L[k][k];
-        for (int j = k + 1 + t; j < jb; j += 256) L[j][k] = L[j][k] / piv;      // row k of R
-        __syncthreads();
-        // A(i, j) -= R(k, i) R(k, j), k < i <= j
-        const int r = jb - k - 1;
-        for (int e = t; e < r * r; e += 256) {
-            const int i = k + 1 + e % r, j = k + 1 + e / r;
-            if (i <= j) L[j][i] = fma(-L[i][k], L[j][k], L[j][i]);
-        }
+        // rows below: W(i, j) -= W(s : s + 16, i)^T W(s : s + 16, j) for the
+        // block rows bi and the blocks bj >= bi of each
+        const int s16 = s / 16;
+        int e = 0;
+        for (int bi = s16 + 1; bi < 4; ++bi)
+            for (int bj = bi; bj < 8; ++bj, ++e) {
+                if ((e & 3) != wave) continue;
+                const int l16 = lane & 15, h = lane >> 4;
+                ca3::gemm::f64x4 acc;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[v] = W[16 * bi + 4 * v + h][16 * bj + l16];
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks)
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-W[s + 4 * ks + h][16 * bi + l16],
+                                                               W[s + 4 * ks + h][16 * bj + l16], acc, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) W[16 * bi + 4 * v + h][16 * bj + l16] = acc[v];
+            }
         __syncthreads();
     }
-    for (int e = t; e < jb * jb; e += 256) {
-        const int i = e % jb, j = e / jb;
-        if (i <= j) D[(int64_t) j * lda + i] = L[j][i];
+    if (blockIdx.x == 0) {
+        const bool last = nc <= 0;
+        if (t == 0 && (j0 == 0 || bad)) *info = bad ? j0 + bad : 0;
+        for (int j = wave; !bad && j < jb; j += 4)
+            if (lane <= j) (last ? D : Rjj)[(int64_t) j * (last ? lda : kPb) + lane] = W[lane][j];
     }
-    if (t == 0 && (j0 == 0 || bad)) *info = bad ? j0 + bad : 0;
+    for (int j = wave; !bad && j < nc; j += 4)
+        if (lane < jb) S[(int64_t) j * lda + lane] = W[lane][kPb + j];
 }
 
-// Block row: X = R_jj^{-T} A(j0:j0+jb, c) for the columns c >= j0 + jb, in
-// place, by forward substitution; one wave per column, lane i holds row i.
-__global__ __launch_bounds__(256) void potrf_panel_kernel(double *A, int64_t lda, int j0, int jb, int n,
-                                                          const int *info)
+// The trailing update behind a block row of 64: C(i, j) -= X(:, i)^T X(:, j)
+// for i <= j < n, X of 64 rows, one 64 x 64 tile per workgroup, tiles of the
+// upper triangle only, C loaded under the products.  Workgroup 0 also puts
+// the factored diagonal block in its place.
+template <bool DTL>
+__global__ __launch_bounds__(512, 4) void potrf_update_kernel(const double *X, double *C, int64_t lda, int n,
+                                                             const double *Rjj, double *D, const int *info)
 {
-    __shared__ double R[kPb][kPb + 1];     // R[j][i] = R_jj(i, j)
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    using namespace ca3::gemm;
+    using TL = Tile64;
+    __shared__ __attribute__((aligned(1024))) double A0[kBK * TL::BM], A1[kBK * TL::BM];
+    __shared__ __attribute__((aligned(1024))) double B0[kBK * TL::BN], B1[kBK * TL::BN];
     if (*info) return;
-    const double *D = A + (int64_t) j0 * lda + j0;
-    for (int e = t; e < jb * jb; e += 256) {
-        const int i = e % jb, j = e / jb;
-        R[j][i] = (i <= j) ? D[(int64_t) j * lda + i] : 0.0;
+    // tile pairs ti <= tj, column by column of the triangle
+    int tj = (int) ((sqrtf(8.0f * (float) blockIdx.x + 1.0f) - 1.0f) * 0.5f);
+    while (tj * (tj + 1) / 2 > (int) blockIdx.x) --tj;
+    while ((tj + 1) * (tj + 2) / 2 <= (int) blockIdx.x) ++tj;
+    const int ti = (int) blockIdx.x - tj * (tj + 1) / 2;
+    const int m0 = __builtin_amdgcn_readfirstlane(ti * TL::BM), n0 = __builtin_amdgcn_readfirstlane(tj * TL::BN);
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int row0 = m0 + (wave % TL::WM) * (TL::BM / TL::WM) + (lane & 15);
+    const int col0 = n0 + (wave / TL::WM) * (TL::BN / TL::WN) + (lane >> 4);
+    double c[TL::FI][TL::FJ][4];
+#pragma unroll
+    for (int i = 0; i < TL::FI; ++i)
+#pragma unroll
+        for (int j = 0; j < TL::FJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = row0 + 16 * i, col = col0 + 16 * j + 4 * r;
+                c[i][j][r] = (row <= col && col < n) ? C[(int64_t) col * lda + row] : 0.0;
+            }
+    f64x4 acc[TL::FI][TL::FJ];
+    zero(acc);
+    if constexpr (DTL) {
+        DtlLoader<0, 4, TL::BM, TL::NW> da, db;
+        da.init(X, lda, m0, min(TL::BM, n - m0));
+        db.init(X, lda, n0, min(TL::BN, n - n0));
+        mainloop_dtl<TL>(da, db, lda, lda, 0, kPb, A0, A1, B0, B1, acc);
+    } else {
+        OperandLoader<0, TL::BM, TL::THREADS> la, lb;
+        la.init(X, lda, m0, n);
+        lb.init(X, lda, n0, n);
+        mainloop<TL>(la, lb, 0, kPb, m0 + TL::BM <= n && n0 + TL::BN <= n, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
     }
-    __syncthreads();
-    const int c = j0 + jb + blockIdx.x * 4 + wave;
-    if (c >= n) return;
-    double *col = A + (int64_t) c * lda + j0;
-    double x = lane < jb ? col[lane] : 0.0;
-    for (int i = 0; i < jb; ++i) {
-        // x_i is final once the rows above it are eliminated
-        const double xi = __shfl(x, i) / R[i][i];
-        if (lane == i) x = xi;
-        if (lane > i) x = fma(-R[lane][i], xi, x);
-    }
-    if (lane < jb) col[lane] = x;
+#pragma unroll
+    for (int i = 0; i < TL::FI; ++i)
+#pragma unroll
+        for (int j = 0; j < TL::FJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = row0 + 16 * i, col = col0 + 16 * j + 4 * r;
+                if (row <= col && col < n) C[(int64_t) col * lda + row] = ca3::add_rn(c[i][j][r], -acc[i][j][r]);
+            }
+    if (blockIdx.x == 0)
+        for (int e = t; e < kPb * kPb; e += TL::THREADS)
+            if (e % kPb <= e / kPb) D[(int64_t) (e / kPb) * lda + e % kPb] = Rjj[e];
 }
 
-// X = R^{-1}, both n x n upper triangular (ldx, ldr); one block per column.
-__global__ __launch_bounds__(256) void trtri_upper_kernel(const double *R, int64_t ldr, double *X, int64_t ldx, int n)
+// X = R^{-1} on the 64 x 64 diagonal blocks (the last may be smaller), one
+// workgroup each, the zeros below the diagonal included.  A wave sweeps 16
+// columns from the bottom row up, lane = row, so that a step is 16 independent
+// quotients and updates.
+__global__ __launch_bounds__(256) void trtri_diag_kernel(const double *R, int64_t ldr, double *X, int64_t ldx, int n)
 {
-    __shared__ double x[kMaxN];
-    const int j = blockIdx.x, t = threadIdx.x;
-    for (int p = t; p <= j; p += 256) x[p] = (p == j) ? 1.0 : 0.0;
-    __syncthreads();
-    for (int i = j; i >= 0; --i) {
-        const double xi = x[i] / R[(int64_t) i * ldr + i];
-        __syncthreads();
-        if (t == 0) x[i] = xi;
-        for (int p = t; p < i; p += 256) x[p] = fma(-R[(int64_t) i * ldr + p], xi, x[p]);
-        __syncthreads();
+    __shared__ double L[kPb][kPb + 1];     // L[j][i] = R(j0 + i, j0 + j), i <= j
+    const int j0 = (int) blockIdx.x * kPb, jb = min(kPb, n - j0);
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const double *D = R + (int64_t) j0 * ldr + j0;
+#pragma unroll
+    for (int q = 0; q < kPb / 4; ++q) {
+        const int j = wave + 4 * q;
+        L[j][lane] = (lane <= j && j < jb) ? D[(int64_t) j * ldr + lane] : (lane == j ? 1.0 : 0.0);
     }
-    for (int p = t; p < n; p += 256) X[(int64_t) j * ldx + p] = (p <= j) ? x[p] : 0.0;
+    __syncthreads();
+    const int w16 = __builtin_amdgcn_readfirstlane(wave * 16);
+    // quotients from the rounded reciprocal and one correction (the rounded
+    // quotient, where nothing leaves the normal range); by division where a
+    // diagonal entry is extreme
+    const double dl = L[lane][lane], rdiag = 1.0 / dl;
+    const bool normal = __all(fabs(dl) > 0x1p-500 && fabs(dl) < 0x1p500);
+    double x[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) x[q] = lane == w16 + q ? 1.0 : 0.0;
+    if (normal) {
+        for (int i = w16 + 15; i >= 0; --i) {
+            const double d = L[i][i], rd = readlane(rdiag, i), u = lane < i ? -L[i][lane] : 0.0;
+            double v[16], xi[16];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) v[q] = readlane(x[q], i);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const double v0 = v[q] * rd, v1 = fma(fma(-v0, d, v[q]), rd, v0);
+                xi[q] = v1 == v1 ? v1 : v0;            // v not finite
+            }
+#pragma unroll
+            for (int q = 0; q < 16; ++q) x[q] = lane < i ? fma(u, xi[q], x[q]) : (lane == i ? xi[q] : x[q]);
+        }
+    } else {
+        for (int i = w16 + 15; i >= 0; --i) {
+            const double d = L[i][i], u = lane < i ? -L[i][lane] : 0.0;
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const double xi = readlane(x[q], i) / d;
+                x[q] = lane < i ? fma(u, xi, x[q]) : (lane == i ? xi : x[q]);
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        const int j = w16 + q;
+        if (j < jb && lane < jb) X[(int64_t) (j0 + j) * ldx + j0 + lane] = lane <= j ? x[q] : 0.0;
+    }
+}
+
+// Joins pairs of inverted blocks: with R11 (s x s, at o = 2 s blockIdx.y) and
+// R22 (w x w) inverted in X, X12 = -X11 (R12 X22).  PART 0 forms the
+// transpose of T = R12 X22 in the place of X21 (w x s, zeroed at the end),
+// PART 1 the product of X11 with it.  Below the diagonal the 64 x 64 blocks
+// hold such products of earlier steps: k starts (ends) at the tile's first
+// row (last column), which passes over them and over the zeros.  With fewer
+// than 16 k the one stage starts before the block (o + s >= 64, so inside X
+// and R) and counts what it reads there as zero.
+template <int PART, bool DTL>
+__global__ __launch_bounds__(256, 4) void trtri_join_kernel(const double *R, int64_t ldr, double *X, int64_t ldx,
+                                                           int n, int s)
+{
+    using namespace ca3::gemm;
+    using TL = Tile32;
+    __shared__ __attribute__((aligned(1024))) double A0[kBK * TL::BM], A1[kBK * TL::BM];
+    __shared__ __attribute__((aligned(1024))) double B0[kBK * TL::BN], B1[kBK * TL::BN];
+    const int o = 2 * s * (int) blockIdx.y, w = min(s, n - o - s);
+    GemmArgs g;
+    g.M = PART ? s : w;
+    g.N = PART ? w : s;
+    g.K = g.M;
+    g.nsrc = 0;
+    g.alpha = PART ? -1.0 : 1.0;
+    g.beta = 0.0;
+    double *const X11 = X + (int64_t) o * ldx + o, *const X21 = X11 + s;
+    const double *const X22 = X11 + (int64_t) s * ldx + s;
+    g.A = PART ? X11 : X22;
+    g.lda = ldx;
+    g.B = PART ? X21 : R + (int64_t) (o + s) * ldr + o;
+    g.ldb = PART ? ldx : ldr;
+    g.C = PART ? X11 + (int64_t) s * ldx : X21;
+    g.ldc = ldx;
+    const int tiles_m = (g.M + TL::BM - 1) / TL::BM, tiles_n = (g.N + TL::BN - 1) / TL::BN;
+    if ((int) blockIdx.x >= tiles_m * tiles_n) return;
+    // the tiles with the longest k first
+    const int tm = (int) blockIdx.x / tiles_n;
+    const int m0 = __builtin_amdgcn_readfirstlane((PART ? tm : tiles_m - 1 - tm) * TL::BM);
+    const int n0 = __builtin_amdgcn_readfirstlane(((int) blockIdx.x % tiles_n) * TL::BN);
+    const int kbeg = PART ? m0 : 0, kend = PART ? s : min(w, m0 + TL::BM);
+    const int mn = min(TL::BM, g.M - m0), nn = min(TL::BN, g.N - n0);
+    f64x4 acc[TL::FI][TL::FJ];
+    zero(acc);
+    if constexpr (DTL) {
+        DtlLoader<PART, 4, TL::BM, TL::NW> da;
+        DtlLoader<1, 4, TL::BN, TL::NW> db;
+        da.init(g.A, g.lda, m0, mn);
+        db.init(g.B, g.ldb, n0, nn);
+        mainloop_dtl<TL>(da, db, g.lda, g.ldb, kbeg, kend, A0, A1, B0, B1, acc);
+        epilogue<TL>(g, m0, n0, acc, dtl_shift<PART, 4>(mn), dtl_shift<1, 4>(nn));
+    } else {
+        OperandLoader<PART, TL::BM, TL::THREADS> la;
+        OperandLoader<1, TL::BN, TL::THREADS> lb;
+        la.init(g.A, g.lda, m0, g.M);
+        lb.init(g.B, g.ldb, n0, g.N);
+        mainloop<TL>(la, lb, kbeg, kend, mn == TL::BM && nn == TL::BN, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
+        epilogue<TL>(g, m0, n0, acc);
+    }
+}
+
+// The strictly lower 64 x 64 blocks of X := 0, one workgroup per column.
+__global__ __launch_bounds__(256) void trtri_zero_kernel(double *X, int64_t ldx, int n)
+{
+    const int j = blockIdx.x;
+    for (int i = (j / kPb + 1) * kPb + (int) threadIdx.x; i < n; i += 256) X[(int64_t) j * ldx + i] = 0.0;
 }
 
 struct Ws {
@@ -159,22 +420,25 @@ int hip_dpotrf(const char uplo, const int n, double *A, const int ldA)
     if (n > kMaxN) return ca3::fail_msg(HIP_PROXY_ERR_UNSUPP, "dpotrf: n > %d", kMaxN);
     if (n == 0) return 0;
     int rc = 0;
-    int *dinfo = (int *) scratch(256, &rc);
+    int *dinfo = (int *) scratch(256 + sizeof(double) * kPb * kPb, &rc);
     if (rc) return rc;
+    double *Rjj = (double *) ((char *) dinfo + 256);
+    const bool dtl = ca3::gemm::dtl_ld_ok(ldA) && ca3::gemm::load_mode() == ca3::gemm::kLoads16;
     const int save = ca3::sync_mode();
     hip_proxy_set_sync(0);
     for (int j0 = 0; j0 < n && !rc; j0 += kPb) {
         const int jb = std::min(kPb, n - j0), nr = n - j0 - jb;
-        potrf_diag_kernel<<<1, 256, 0, ca3::stream()>>>(A, ldA, j0, jb, dinfo);
+        potrf_row_kernel<<<std::max(1, (nr + kPb - 1) / kPb), 256, 0, ca3::stream()>>>(A, ldA, j0, jb, n, Rjj, dinfo);
         hipError_t e = hipGetLastError();
-        if (e != hipSuccess) { rc = ca3::fail(e, "potrf_diag_kernel"); break; }
+        if (e != hipSuccess) { rc = ca3::fail(e, "potrf_row_kernel"); break; }
         if (nr == 0) break;
-        potrf_panel_kernel<<<(nr + 3) / 4, 256, 0, ca3::stream()>>>(A, ldA, j0, jb, n, dinfo);
+        // trailing upper triangle: A(r, r) -= X^T X, X = A(j0:j0+64, r)
+        double *X = A + (int64_t) (j0 + jb) * ldA + j0, *D = A + (int64_t) j0 * ldA + j0;
+        const int nt = (nr + kPb - 1) / kPb;
+        if (dtl) potrf_update_kernel<true><<<nt * (nt + 1) / 2, 512, 0, ca3::stream()>>>(X, X + jb, ldA, nr, Rjj, D, dinfo);
+        else potrf_update_kernel<false><<<nt * (nt + 1) / 2, 512, 0, ca3::stream()>>>(X, X + jb, ldA, nr, Rjj, D, dinfo);
         e = hipGetLastError();
-        if (e != hipSuccess) { rc = ca3::fail(e, "potrf_panel_kernel"); break; }
-        // trailing upper triangle: A(r, r) -= X^T X, X = A(j0:j0+jb, r)
-        double *X = A + (int64_t) (j0 + jb) * ldA + j0;
-        rc = hip_dsyrk_gram(nr, jb, -1.0, X, ldA, 1.0, A + (int64_t) (j0 + jb) * ldA + j0 + jb, ldA, 0);
+        if (e != hipSuccess) rc = ca3::fail(e, "potrf_update_kernel");
     }
     hip_proxy_set_sync(save);
     if (rc) return rc;
@@ -190,7 +454,23 @@ int hip_dtrtri_upper(const int n, const double *R, const int ldR, double *X, con
         return ca3::fail_msg(HIP_PROXY_ERR_ARG, "dtrtri: bad arguments");
     if (n > kMaxN) return ca3::fail_msg(HIP_PROXY_ERR_UNSUPP, "dtrtri: n > %d", kMaxN);
     if (n == 0) return HIP_PROXY_OK;
-    trtri_upper_kernel<<<n, 256, 0, ca3::stream()>>>(R, ldR, X, ldX, n);
+    const bool dtl = ca3::gemm::dtl_ld_ok(ldR) && ca3::gemm::dtl_ld_ok(ldX) &&
+                     ca3::gemm::load_mode() == ca3::gemm::kLoads16;
+    hipStream_t st = ca3::stream();
+    trtri_diag_kernel<<<(n + kPb - 1) / kPb, 256, 0, st>>>(R, ldR, X, ldX, n);
+    for (int s = kPb; s < n; s *= 2) {
+        // blocks of s joined in pairs; the last block may be alone or short
+        const int pairs = (n - s + 2 * s - 1) / (2 * s), tiles = s / 32;
+        const dim3 grid((unsigned) (tiles * tiles), (unsigned) pairs);
+        if (dtl) {
+            trtri_join_kernel<0, true><<<grid, 256, 0, st>>>(R, ldR, X, ldX, n, s);
+            trtri_join_kernel<1, true><<<grid, 256, 0, st>>>(R, ldR, X, ldX, n, s);
+        } else {
+            trtri_join_kernel<0, false><<<grid, 256, 0, st>>>(R, ldR, X, ldX, n, s);
+            trtri_join_kernel<1, false><<<grid, 256, 0, st>>>(R, ldR, X, ldX, n, s);
+        }
+    }
+    if (n > kPb) trtri_zero_kernel<<<n, 256, 0, st>>>(X, ldX, n);
     return ca3::finish();
 }
 
