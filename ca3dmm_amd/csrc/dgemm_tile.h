@@ -11,6 +11,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <climits>
 #include <cstdint>
 
 #include "hip_common.h"
@@ -496,7 +497,8 @@ __device__ __forceinline__ void stage_mfma_dtl(const double *As, const double *B
 // then count as zero.  (A separate bounds-checked stage cost a whole exposed
 // load latency.)  The products are added in the order of k either way, so
 // results do not depend on the path.  Ends with a barrier after which the
-// buffers are free.
+// buffers are free.  A wave takes no part in the products of whole stages that
+// start at kw or later (its operand is zero there).
 //
 // The two buffers of each operand must be distinct __shared__ arrays and
 // the loop is unrolled by two so that every access names its array at
@@ -510,7 +512,7 @@ __device__ __forceinline__ void stage_mfma_dtl(const double *As, const double *B
 template <class TL, class LA, class LB>
 __device__ __forceinline__ void mainloop_dtl(const LA &la, const LB &lb, int64_t lda, int64_t ldb, int kbeg, int kend,
                                              double *A0, double *A1, double *B0, double *B1,
-                                             f64x4 (&acc)[TL::FI][TL::FJ])
+                                             f64x4 (&acc)[TL::FI][TL::FJ], int kw = INT_MAX)
 {
     constexpr int XCA = LA::XC, XCB = LB::XC;
     const int nfull = (kend - kbeg) / kBK, rem = (kend - kbeg) % kBK;
@@ -532,11 +534,11 @@ __device__ __forceinline__ void mainloop_dtl(const LA &la, const LB &lb, int64_t
     for (int z = 0; z < nfull; z += 2) {
         publish();                              // stage z in buffer 0
         if (z + 1 < ns) issue(z + 1, A1, B1);
-        stage_mfma_dtl<XCA, XCB, TL>(A0, B0, acc);
+        if (kbeg + z * kBK < kw) stage_mfma_dtl<XCA, XCB, TL>(A0, B0, acc);
         if (z + 1 >= nfull) break;
         publish();                              // stage z + 1 in buffer 1
         if (z + 2 < ns) issue(z + 2, A0, B0);
-        stage_mfma_dtl<XCA, XCB, TL>(A1, B1, acc);
+        if (kbeg + (z + 1) * kBK < kw) stage_mfma_dtl<XCA, XCB, TL>(A1, B1, acc);
     }
     if (rem > 0) {
         publish();

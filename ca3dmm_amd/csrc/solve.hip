@@ -19,6 +19,7 @@
 //                   produced from the last to the first through a workspace,
 //                   so B can be overwritten in place.
 #include <algorithm>
+#include <climits>
 #include <cstring>
 #include <mutex>
 #include <type_traits>
@@ -380,6 +381,38 @@ __global__ __launch_bounds__(256) void trtri_zero_kernel(double *X, int64_t ldx,
     for (int i = (j / kPb + 1) * kPb + (int) threadIdx.x; i < n; i += 256) X[(int64_t) j * ldx + i] = 0.0;
 }
 
+// X := B R^{-1} for B of m x n and T = R^{-1}, zero below the diagonal: the
+// 128 x 128 tile at column n0 takes k in [0, min(n, n0 + 128)), and a wave
+// leaves out the stages behind its own last column.  All column blocks in one
+// launch: each by itself leaves part of the chip idle (30011 x 1999: 235 tiles
+// each) and reads B again.  Workgroup b runs on XCD b % 8, which works through
+// an eighth of the tile rows in groups of 32, the columns with the longest k
+// first, so that a group's rows of B stay in that XCD's L2 for all columns.
+__global__ __launch_bounds__(512, 4) void trmm_kernel(ca3::gemm::GemmArgs g)
+{
+    using namespace ca3::gemm;
+    using TL = Tile128w8;
+    __shared__ __attribute__((aligned(1024))) double A0[kBK * TL::BM], A1[kBK * TL::BM];
+    __shared__ __attribute__((aligned(1024))) double B0[kBK * TL::BN], B1[kBK * TL::BN];
+    const int tiles_m = (g.M + TL::BM - 1) / TL::BM, tiles_n = (g.N + TL::BN - 1) / TL::BN;
+    const int per_xcd = (tiles_m + 7) / 8, first = (int) (blockIdx.x & 7) * per_xcd;
+    const int rows = min(per_xcd, tiles_m - first), e = (int) (blockIdx.x >> 3);
+    if (e >= rows * tiles_n) return;
+    const int grp = e / (32 * tiles_n), r = e - grp * 32 * tiles_n, gsz = min(rows - 32 * grp, 32);
+    const int m0 = __builtin_amdgcn_readfirstlane((first + 32 * grp + r % gsz) * TL::BM);
+    const int n0 = __builtin_amdgcn_readfirstlane((tiles_n - 1 - r / gsz) * TL::BN);
+    const int kend = min(g.K, n0 + TL::BN), mn = min(TL::BM, g.M - m0);
+    const int wn = __builtin_amdgcn_readfirstlane((int) (threadIdx.x >> 6) / TL::WM);
+    f64x4 acc[TL::FI][TL::FJ];
+    zero(acc);
+    DtlLoader<1, 4, TL::BM, TL::NW> da;
+    DtlLoader<0, 4, TL::BN, TL::NW> db;
+    da.init(g.A, g.lda, m0, mn);
+    db.init(g.B, g.ldb, n0, min(TL::BN, g.N - n0));
+    mainloop_dtl<TL>(da, db, g.lda, g.ldb, 0, kend, A0, A1, B0, B1, acc, n0 + (wn + 1) * (TL::BN / TL::WN));
+    epilogue<TL>(g, m0, n0, acc, dtl_shift<1, 4>(mn));
+}
+
 struct Ws {
     void *p = nullptr;
     size_t bytes = 0;
@@ -521,6 +554,20 @@ int ca3::trsm_right_upper_out(int m, int n, const double *R, int ldR, const doub
     const int save = ca3::sync_mode();
     hip_proxy_set_sync(0);
     rc = hip_dtrtri_upper(n, R, ldR, Rinv, n);
+    const int64_t tiles = (int64_t) ((m + 127) / 128 + 7) / 8 * 8 * ((n + 127) / 128);
+    if (!rc && m > 1 && n >= gemm::kBK && tiles <= INT_MAX && gemm::dtl_ld_ok(ldB) && ((uintptr_t) B % 8) == 0 &&
+        gemm::load_mode() == gemm::kLoads16) {
+        gemm::GemmArgs g;
+        memset(&g, 0, sizeof(g));
+        g.M = m; g.N = n; g.K = n;
+        g.alpha = 1.0;
+        g.A = B; g.lda = ldB; g.B = Rinv; g.ldb = n; g.C = X; g.ldc = ldX;
+        trmm_kernel<<<(unsigned) tiles, 512, 0, ca3::stream()>>>(g);
+        hipError_t e = hipGetLastError();
+        hip_proxy_set_sync(save);
+        if (e != hipSuccess) return ca3::fail(e, "trmm_kernel");
+        return ca3::finish();
+    }
     // column block jb of X = B R^{-1} needs rows 0 .. end(jb) of R^{-1}
     const int nb = 128;
     for (int j0 = 0; !rc && j0 < n; j0 += nb) {

@@ -67,6 +67,26 @@ def test_inverse_of_extreme_diagonals(hip):
     assert np.array_equal(dX.numpy(), np.diag(1.0 / d))
 
 
+@pytest.mark.parametrize("m,n,pad", [(129, 16, 0), (300, 129, 1), (4097, 257, 0), (1000, 500, 3), (20001, 128, 0)])
+def test_orthogonalisation_of_odd_sizes(hip, monkeypatch, m, n, pad):
+    """Q = A R^{-1} in one launch agrees with the in-place form (one product
+    per column block), and Q R = A; kappa(A) is below 10."""
+    rnd = np.random.default_rng(m + n)
+    A = rnd.standard_normal((m, n))
+    out = []
+    for inplace in ("0", "1"):
+        monkeypatch.setenv("CA3DMM_CHOLQR_INPLACE", inplace)
+        dA, dR = _padded(hip, A, m + pad), hip.DeviceArray.filled((n, n), 0xFF)
+        info, passes = hip.cholesky_qr(m, n, dA, dR, variant=2)
+        assert info == 0 and passes == 2
+        out.append((dA.numpy(), dR.numpy()))
+    (Q, R), (Q1, R1) = out
+    assert np.abs(Q - Q1).max() <= 1e-13 and np.abs(R - R1).max() <= 1e-13 * np.abs(R1).max()
+    assert np.all(Q[m:] == 7.0)
+    assert np.linalg.norm(Q[:m] @ R - A) <= 1e-13 * np.linalg.norm(A)
+    assert np.linalg.norm(Q[:m].T @ Q[:m] - np.eye(n)) <= 1e-13 * n
+
+
 @pytest.mark.parametrize("n,at", [(64, 0), (100, 40), (200, 150), (130, 129)])
 def test_factor_with_extreme_pivots(hip, n, at):
     """Pivots outside the range of the iterated square root are taken by
