@@ -489,6 +489,16 @@ __device__ __forceinline__ void stage_mfma_dtl(const double *As, const double *B
     }
 }
 
+// Own loads of the stage have landed (vmcnt counts the LDS DMA) and own reads
+// of the stage before it are done, then every wave's.
+__device__ __forceinline__ void dtl_publish()
+{
+    __builtin_amdgcn_s_waitcnt(0x0070);         // vmcnt(0) lgkmcnt(0); expcnt (6:4) not waited on
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // k in [kbeg, kend) of a TL tile through a double buffer of direct-to-LDS
 // stages, one in flight under the MFMAs of the other.  Needs kend >= 16
 // (whatever kbeg) and kbeg, kend in scalar registers.  The k left over after
@@ -522,29 +532,37 @@ __device__ __forceinline__ void mainloop_dtl(const LA &la, const LB &lb, int64_t
         la.issue(XCA ? k0 * lda : k0, SA);
         lb.issue(XCB ? k0 * ldb : k0, SB);
     };
-    // own loads of the stage have landed (vmcnt counts the LDS DMA) and own
-    // reads of the stage before it are done, then every wave's
-    auto publish = []() __attribute__((always_inline)) {
-        __builtin_amdgcn_s_waitcnt(0x0070);     // vmcnt(0) lgkmcnt(0); expcnt (6:4) not waited on
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-    };
     if (ns > 0) issue(0, A0, B0);
     for (int z = 0; z < nfull; z += 2) {
-        publish();                              // stage z in buffer 0
+        dtl_publish();                              // stage z in buffer 0
         if (z + 1 < ns) issue(z + 1, A1, B1);
         if (kbeg + z * kBK < kw) stage_mfma_dtl<XCA, XCB, TL>(A0, B0, acc);
         if (z + 1 >= nfull) break;
-        publish();                              // stage z + 1 in buffer 1
+        dtl_publish();                              // stage z + 1 in buffer 1
         if (z + 2 < ns) issue(z + 2, A0, B0);
         if (kbeg + (z + 1) * kBK < kw) stage_mfma_dtl<XCA, XCB, TL>(A1, B1, acc);
     }
     if (rem > 0) {
-        publish();
+        dtl_publish();
         stage_mfma_dtl<XCA, XCB, TL, true>(nfull & 1 ? A1 : A0, nfull & 1 ? B1 : B0, acc, kBK - rem);
     }
     __syncthreads();
+}
+
+// The whole tile of acc to out, column by column (rows fastest).
+template <class TL>
+__device__ __forceinline__ void store_tile(double *out, const f64x4 (&acc)[TL::FI][TL::FJ])
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = wave % TL::WM, wn = wave / TL::WM;
+#pragma unroll
+    for (int i = 0; i < TL::FI; ++i)
+#pragma unroll
+        for (int j = 0; j < TL::FJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                out[((wn * TL::FJ + j) * 16 + 4 * r + (lane >> 4)) * TL::BM + (wm * TL::FI + i) * 16 + (lane & 15)] =
+                    acc[i][j][r];
 }
 
 // C := fold(P) + (alpha*acc + beta*C) for the tile at (m0, n0), with the

@@ -3,12 +3,13 @@
 // The reference computes B^T B in full through the general Cannon DGEMM
 // (src/ca3dmm.c:1172-1265) and the CholeskyQR driver uses it for
 // S = B^T B (examples/example_CholeskyQR.c:109-117, :160-168).  Here only
-// tiles (i <= j) of the upper triangle are computed: n(n+1)k flops instead
-// of 2n^2 k.  Tall-skinny inputs (k >> n, e.g. 2e6 x 512) give few tiles,
-// so k is split across workgroups; each split writes its partial tile and a
-// second kernel adds the partials in split order (deterministic) and writes
-// the upper triangle, optionally mirrored into the lower one.  Mirroring
-// copies values, so the result is exactly symmetric.
+// tiles (i <= j) of the upper triangle are computed, and in the tiles on the
+// diagonal only the 16 x 16 blocks (i <= j): n(n+1)k flops instead of 2n^2 k.
+// Tall-skinny inputs (k >> n, e.g. 2e6 x 512) give few tiles, so k is split
+// across workgroups; each split writes its partial tile and a second kernel
+// adds the partials in split order (deterministic) and writes the upper
+// triangle, optionally mirrored into the lower one.  Mirroring copies values,
+// so the result is exactly symmetric.
 #include <algorithm>
 #include <cstring>
 #include <mutex>
@@ -27,97 +28,191 @@ namespace {
 
 using namespace ca3::gemm;
 
+// Tile pairs (ti < tj) take k in ranges of step1, s1 of them, the tiles on the
+// diagonal ranges of step2, s2 of them.  Partials in P: pair p and range ks at
+// (ks noff + p), diagonal tile t at (noff s1 + ks ntile + t), in tiles.
 struct GramArgs {
-    int n, k, ntile, npairs, ksplit, kstep;
+    int n, k, ntile, noff, s1, step1, s2, step2;
     const double *A;
     int64_t lda;
-    double *P;      // partials: [ksplit][npairs][128 * 128]
+    double *P;
 };
 
-// pair index -> (ti, tj), ti <= tj, row-major over the upper triangle
+// pair index -> (ti, tj), ti < tj, row-major over the strict upper triangle
 __device__ __forceinline__ void pair_of(int p, int nt, int *ti, int *tj)
 {
     int i = 0, rem = p;
-    while (rem >= nt - i) { rem -= nt - i; ++i; }
+    while (rem >= nt - 1 - i) { rem -= nt - 1 - i; ++i; }
     *ti = i;
-    *tj = i + rem;
+    *tj = i + 1 + rem;
 }
 
-// W: 4 for 16-byte direct-to-LDS loads (A 16-byte aligned, even lda), 0 for
-// register-staged stages (both panels are k-contiguous, where 4-byte
-// direct-to-LDS loads lose to register staging).
-template <int W>
-__global__ __launch_bounds__(kThreads, 2) void gram_partial_kernel(GramArgs g)
+// A diagonal tile in direct-to-LDS stages: one panel is both operands, and the
+// 16 x 16 blocks on and above the diagonal (36 of 64 in a 128-wide tile) are
+// dealt to the 8 waves, which leaves the SIMDs the same number (9 each).  The
+// products of an entry and their order are those of mainloop_dtl.
+template <class TL>
+struct DiagTile {
+    static constexpr int NB = TL::BM / 16, BLOCKS = NB * (NB + 1) / 2;
+    static constexpr int MOST = (BLOCKS + TL::NW - 1) / TL::NW, LEAST = BLOCKS / TL::NW;
+    int bi[MOST], bj[MOST], count;
+    f64x4 acc[MOST];
+
+    __device__ __forceinline__ void init()
+    {
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        count = (BLOCKS - wave + TL::NW - 1) / TL::NW;
+#pragma unroll
+        for (int q = 0; q < MOST; ++q) {
+            const int p = min(wave + q * TL::NW, BLOCKS - 1);
+            int j = 0;
+            while ((j + 1) * (j + 2) / 2 <= p) ++j;
+            bi[q] = p - j * (j + 1) / 2;
+            bj[q] = j;
+            acc[q] = f64x4{0.0, 0.0, 0.0, 0.0};
+        }
+    }
+
+    template <bool TAIL = false>
+    __device__ __forceinline__ void mfma(const double *S, int lo = 0)
+    {
+        const int lane = threadIdx.x & 63, li = lane & 15;
+#pragma unroll
+        for (int ks = 0; ks < kBK / 4; ++ks) {
+            const int kk = ks * 4 + (lane >> 4);
+            const double *L = S + dtl_index<0, TL::BM>(kk, li);
+#pragma unroll
+            for (int q = 0; q < MOST; ++q) {
+                if (q >= LEAST && q >= count) continue;
+                double a = L[bi[q] * 256], b = L[bj[q] * 256];
+                if (TAIL) {
+                    a = kk >= lo ? a : 0.0;
+                    b = kk >= lo ? b : 0.0;
+                }
+                acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, acc[q], 0, 0, 0);
+            }
+        }
+    }
+
+    template <class LD>
+    __device__ __forceinline__ void run(const LD &ld, int kbeg, int kend, double *S0, double *S1)
+    {
+        const int nfull = (kend - kbeg) / kBK, rem = (kend - kbeg) % kBK, ns = nfull + (rem > 0);
+        auto issue = [&](int z, double *S) __attribute__((always_inline)) {
+            ld.issue(min(kbeg + z * kBK, kend - kBK), S);
+        };
+        if (ns > 0) issue(0, S0);
+        for (int z = 0; z < nfull; z += 2) {
+            dtl_publish();
+            if (z + 1 < ns) issue(z + 1, S1);
+            mfma(S0);
+            if (z + 1 >= nfull) break;
+            dtl_publish();
+            if (z + 2 < ns) issue(z + 2, S0);
+            mfma(S1);
+        }
+        if (rem > 0) {
+            dtl_publish();
+            mfma<true>(nfull & 1 ? S1 : S0, kBK - rem);
+        }
+    }
+
+    __device__ __forceinline__ void store(double *out) const
+    {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int q = 0; q < MOST; ++q) {
+            if (q >= count) continue;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                out[(bj[q] * 16 + 4 * r + (lane >> 4)) * TL::BM + bi[q] * 16 + (lane & 15)] = acc[q][r];
+        }
+    }
+};
+
+// One partial tile per workgroup.  DTL: 16-byte direct-to-LDS stages in 8-wave
+// workgroups; otherwise register-staged (both panels are k-contiguous, where
+// 4-byte direct-to-LDS loads lose to register staging), the same products in
+// the same order.
+template <class TL, bool DTL>
+__global__ __launch_bounds__(TL::THREADS, DTL ? 4 : 2) void gram_partial_kernel(GramArgs g)
 {
-    __shared__ __attribute__((aligned(1024))) double A0[kBK * kBM], A1[kBK * kBM];
-    __shared__ __attribute__((aligned(1024))) double B0[kBK * kBN], B1[kBK * kBN];
+    __shared__ __attribute__((aligned(1024))) double A0[kBK * TL::BM], A1[kBK * TL::BM];
+    __shared__ __attribute__((aligned(1024))) double B0[kBK * TL::BN], B1[kBK * TL::BN];
     // Workgroups are dealt round-robin over the 8 XCDs; the logical ids are
     // made XCD-contiguous (the grid is a multiple of 8) so that the pairs of
     // one k-range, which share their panels, run behind the same L2.
-    const int nb = gridDim.x, total = g.npairs * g.ksplit;
+    const int nb = gridDim.x, off = g.noff * g.s1;
     const int bid = (blockIdx.x & 7) * (nb >> 3) + (blockIdx.x >> 3);
-    if (bid >= total) return;
-    const int pair = bid % g.npairs, ks = bid / g.npairs;
-    int ti, tj;
-    pair_of(pair, g.ntile, &ti, &tj);
-    const int kbeg = ks * g.kstep, kend = min(g.k, kbeg + g.kstep);
-    // op(A) = A^T and op(B) = A: both panels are contiguous along k
-    OperandLoader<0> la, lb;
-    la.init(g.A, g.lda, ti * kBM, g.n);
-    lb.init(g.A, g.lda, tj * kBN, g.n);
-    f64x4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
-    const bool interior = (ti + 1) * kBM <= g.n && (tj + 1) * kBN <= g.n;
-    int kt0 = kbeg;
-    if (W > 0 && g.k >= kBK) {
-        // whole stages direct-to-LDS (kbeg is a multiple of 16, so the panels
-        // keep A's alignment; edge tiles load copies of their last line in
-        // place of the missing ones); the same products in the same order
-        DtlLoader<0, 4> da, db;
-        da.init(g.A, g.lda, ti * kBM, min(kBM, g.n - ti * kBM));
-        db.init(g.A, g.lda, tj * kBN, min(kBN, g.n - tj * kBN));
-        mainloop_dtl<Tile128>(da, db, g.lda, g.lda, kbeg, kend, A0, A1, B0, B1, acc);
-        kt0 = kend;
+    if (bid >= off + g.ntile * g.s2) return;
+    const bool diag = bid >= off;
+    int ti, tj, ks;
+    if (diag) {
+        ks = (bid - off) / g.ntile;
+        ti = tj = bid - off - ks * g.ntile;
+    } else {
+        ks = bid / g.noff;
+        pair_of(bid - ks * g.noff, g.ntile, &ti, &tj);
     }
-    if (kt0 < kend) mainloop(la, lb, kt0, kend, interior, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
-    // store the full 128 x 128 partial (rows fastest)
-    double *out = g.P + ((int64_t) ks * g.npairs + pair) * (kBM * kBN);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = wm * 64 + i * 16 + (lane & 15);
-                const int col = wn * 64 + j * 16 + 4 * r + (lane >> 4);
-                out[col * kBM + row] = acc[i][j][r];
-            }
+    const int step = diag ? g.step2 : g.step1;
+    const int kbeg = __builtin_amdgcn_readfirstlane(ks * step);
+    const int kend = __builtin_amdgcn_readfirstlane(min(g.k, kbeg + step));
+    const int m0 = __builtin_amdgcn_readfirstlane(ti * TL::BM), n0 = __builtin_amdgcn_readfirstlane(tj * TL::BN);
+    double *out = g.P + (int64_t) bid * (TL::BM * TL::BN);
+    // op(A) = A^T and op(B) = A: both panels are contiguous along k.  The
+    // splits start at multiples of 16, so the panels keep A's alignment; edge
+    // tiles load copies of their last line in place of the missing ones.
+    if constexpr (DTL) {
+        DtlLoader<0, 4, TL::BM, TL::NW> da;
+        da.init(g.A, g.lda, m0, min(TL::BM, g.n - m0));
+        if (diag) {
+            DiagTile<TL> tile;
+            tile.init();
+            tile.run(da, kbeg, kend, A0, A1);
+            tile.store(out);
+            return;
+        }
+        DtlLoader<0, 4, TL::BN, TL::NW> db;
+        db.init(g.A, g.lda, n0, min(TL::BN, g.n - n0));
+        f64x4 acc[TL::FI][TL::FJ];
+        zero(acc);
+        mainloop_dtl<TL>(da, db, g.lda, g.lda, kbeg, kend, A0, A1, B0, B1, acc);
+        store_tile<TL>(out, acc);
+    } else {
+        OperandLoader<0, TL::BM, TL::THREADS> la;
+        OperandLoader<0, TL::BN, TL::THREADS> lb;
+        la.init(g.A, g.lda, m0, g.n);
+        lb.init(g.A, g.lda, n0, g.n);
+        f64x4 acc[TL::FI][TL::FJ];
+        zero(acc);
+        mainloop<TL>(la, lb, kbeg, kend, m0 + TL::BM <= g.n && n0 + TL::BN <= g.n, LdsPair{A0, A1}, LdsPair{B0, B1},
+                     acc);
+        store_tile<TL>(out, acc);
+    }
 }
 
-__global__ __launch_bounds__(256) void gram_reduce_kernel(const double *__restrict__ P, int n, int ntile, int npairs,
-                                                          int ksplit, double alpha, double beta, double *C,
+template <int BM>
+__global__ __launch_bounds__(256) void gram_reduce_kernel(GramArgs g, double alpha, double beta, double *C,
                                                           int64_t ldc, int mirror)
 {
-    const int pair = blockIdx.y;
-    int ti, tj;
-    pair_of(pair, ntile, &ti, &tj);
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < kBM * kBN; e += gridDim.x * blockDim.x) {
-        const int row = e % kBM, col = e / kBM;
-        const int gi = ti * kBM + row, gj = tj * kBN + col;
-        if (gi >= n || gj >= n || gi > gj) continue;
-        double s = P[(int64_t) pair * (kBM * kBN) + e];
-        for (int ks = 1; ks < ksplit; ++ks) s = ca3::add_rn(s, P[((int64_t) ks * npairs + pair) * (kBM * kBN) + e]);
-        double *c = C + (int64_t) gj * ldc + gi;
-        double v = ca3::mul_rn(alpha, s);
-        if (beta != 0.0) v = ca3::add_rn(v, ca3::mul_rn(beta, *c));
-        *c = v;
-        if (mirror && gi != gj) C[(int64_t) gi * ldc + gj] = v;
-    }
+    const int p = blockIdx.y;
+    const bool diag = p >= g.noff;
+    int ti = p - g.noff, tj = ti;
+    if (!diag) pair_of(p, g.ntile, &ti, &tj);
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    const int row = e % BM, col = e / BM, gi = ti * BM + row, gj = tj * BM + col;
+    if (gi >= g.n || gj >= g.n || gi > gj) return;
+    const int ksplit = diag ? g.s2 : g.s1;
+    const int64_t step = (int64_t) (diag ? g.ntile : g.noff) * (BM * BM);
+    const double *q = g.P + (diag ? (int64_t) g.noff * g.s1 + ti : (int64_t) p) * (BM * BM) + e;
+    double s = *q;
+#pragma unroll 8
+    for (int ks = 1; ks < ksplit; ++ks) s = ca3::add_rn(s, q[ks * step]);
+    double *c = C + (int64_t) gj * ldc + gi;
+    double v = ca3::mul_rn(alpha, s);
+    if (beta != 0.0) v = ca3::add_rn(v, ca3::mul_rn(beta, *c));
+    *c = v;
+    if (mirror && gi != gj) C[(int64_t) gi * ldc + gj] = v;
 }
 
 struct Ws {
@@ -127,22 +222,63 @@ struct Ws {
 Ws g_gram_ws[16];
 std::mutex g_gram_mu;
 
-constexpr int kScratchTiles = 512;   // partial tiles the allocation-free entry can hold
+constexpr int kScratchTiles = 512;   // partial 128 x 128 tiles the allocation-free entry can hold
 double *g_scratch_ptr[16];          // device address of `scratch` per device (0: not looked up yet)
 
-// Tiles, k-split and k-range per split for n x n from k.  Enough workgroups
-// for one round of the chip at two per CU (at most kScratchTiles partial
-// tiles on a 256-CU part), stages of >= 1024 k, whole 16-k stages per split.
-void plan(int n, int k, GramArgs *g)
+// Tile width and k ranges for n x n from k, by the cost of a single product's
+// rule: a CU that holds w workgroups takes a + b w us per 16-deep stage, a
+// diagonal tile f of that b; the second launch and the partials cost what the
+// k split of a product does.  Diagonal tiles get longer ranges, so that all
+// workgroups end together.  Splits are at least four stages long and the
+// partials within the fixed scratch, unless the tiles alone exceed it (one
+// range each, then, as 128-wide tiles).
+struct Plan {
+    GramArgs g;
+    int bm, wgs;
+};
+
+Plan plan(int n, int k)
 {
-    memset(g, 0, sizeof(*g));
-    const int ntile = (n + kBM - 1) / kBM, npairs = ntile * (ntile + 1) / 2;
-    const int target = 2 * ca3::cu_count();
-    int ksplit = std::max(1, std::min(target / npairs, (k + 1023) / 1024));
-    if (k == 0) ksplit = 1;
-    const int kstep = std::max(kBK, ((k + ksplit - 1) / ksplit + kBK - 1) / kBK * kBK);
-    ksplit = std::max(1, (k + kstep - 1) / kstep);
-    g->n = n; g->k = k; g->ntile = ntile; g->npairs = npairs; g->ksplit = ksplit; g->kstep = kstep;
+    static const struct { int bm; double a, b, f; int most; } tiles[] = {
+        {128, 0.15, 1.80, 36.0 / 64, 2}, {64, 0.20, 0.47, 12.0 / 16, 4}};
+    const int cus = ca3::cu_count(), stages = (k + kBK - 1) / kBK, longest = std::max(1, stages / 4);
+    Plan best;
+    memset(&best, 0, sizeof(best));
+    double cost = 0.0;
+    for (const auto &t : tiles) {
+        const int ntile = (n + t.bm - 1) / t.bm;
+        const int64_t noff = (int64_t) ntile * (ntile - 1) / 2;
+        const int64_t cap = (int64_t) kScratchTiles * (128 / t.bm) * (128 / t.bm);
+        auto consider = [&](int64_t s1, int64_t s2) {
+            const int l1 = (int) ((stages + s1 - 1) / s1), l2 = (int) ((stages + s2 - 1) / s2);
+            s1 = l1 ? (stages + l1 - 1) / l1 : 1;
+            s2 = l2 ? (stages + l2 - 1) / l2 : 1;
+            const int64_t wgs = noff * s1 + ntile * s2;
+            const double w = (double) ((wgs + cus - 1) / cus);
+            const double us = std::max(noff ? l1 * (t.a + t.b * w) : 0.0, l2 * (t.a + t.b * t.f * w)) +
+                              (double) (2 * wgs) * t.bm * t.bm * 8.0 / 4e6;
+            if (best.bm && us >= (best.bm == t.bm ? 1.0 : 0.92) * cost) return;
+            cost = us;
+            best.bm = t.bm;
+            best.wgs = (int) wgs;
+            best.g.n = n; best.g.k = k; best.g.ntile = ntile; best.g.noff = (int) noff;
+            best.g.s1 = (int) s1; best.g.step1 = std::max(1, l1) * kBK;
+            best.g.s2 = (int) s2; best.g.step2 = std::max(1, l2) * kBK;
+        };
+        if (t.bm == 128 || noff + ntile <= cap) consider(1, 1);
+        for (int r = 1; r <= t.most; r *= 2) {
+            const int64_t slots = std::min((int64_t) r * cus, cap);
+            // the split that fills the slots with equally long ranges, and those around it
+            const int64_t even = (int64_t) ((double) slots / ((double) noff + t.f * ntile));
+            for (int64_t s1 = std::max<int64_t>(1, std::min<int64_t>(even, longest) - 1);
+                 s1 <= std::min<int64_t>(even + 1, longest) && noff * s1 + ntile <= slots; ++s1) {
+                const int64_t s2 = std::min((slots - noff * s1) / ntile, (int64_t) longest);
+                consider(s1, s2);
+                consider(s1, std::min(s2, std::max<int64_t>(1, (int64_t) ((double) s1 * t.f + 0.999))));
+            }
+        }
+    }
+    return best;
 }
 
 int check_args(int n, int k, const double *A, int ldA, const double *C, int ldC)
@@ -153,24 +289,33 @@ int check_args(int n, int k, const double *A, int ldA, const double *C, int ldC)
     return 0;
 }
 
-int launch(const GramArgs &g, double alpha, double beta, double *C, int ldC, int mirror)
+template <class TL, class TR>
+void launch_tile(const Plan &p, bool dtl, double alpha, double beta, double *C, int ldC, int mirror)
 {
     hipStream_t st = ca3::stream();
-    const int grid = (g.npairs * g.ksplit + 7) / 8 * 8;
+    const int grid = (p.wgs + 7) / 8 * 8;
+    if (dtl) gram_partial_kernel<TL, true><<<grid, TL::THREADS, 0, st>>>(p.g);
+    else gram_partial_kernel<TR, false><<<grid, TR::THREADS, 0, st>>>(p.g);
+    gram_reduce_kernel<TL::BM><<<dim3(TL::BM * TL::BM / 256, p.g.noff + p.g.ntile), 256, 0, st>>>(p.g, alpha, beta, C,
+                                                                                               ldC, mirror ? 1 : 0);
+}
+
+// Both launches; the caller holds g_gram_mu, so that calls of several threads,
+// which share the device's stream and the partials, do not mix theirs.
+int launch(const Plan &p, double alpha, double beta, double *C, int ldC, int mirror)
+{
     // 16-byte direct-to-LDS loads from any 8-byte aligned A (as the DGEMM;
     // CA3DMM_DGEMM_LOADS=aligned keeps them to 16-byte aligned A with even
     // lda, "reg" and "dword" stage through registers)
+    const GramArgs &g = p.g;
     const LoadMode mode = load_mode();
     const bool aligned16 = ((uintptr_t) g.A % 16) == 0 && (g.lda % 2) == 0;
-    if (dtl_ld_ok(g.lda) && ((uintptr_t) g.A % 8) == 0 && (mode == kLoads16 || (mode == kLoadsAligned && aligned16)))
-        gram_partial_kernel<4><<<grid, kThreads, 0, st>>>(g);
-    else
-        gram_partial_kernel<0><<<grid, kThreads, 0, st>>>(g);
+    const bool dtl = g.k >= kBK && dtl_ld_ok(g.lda) && ((uintptr_t) g.A % 8) == 0 &&
+                     (mode == kLoads16 || (mode == kLoadsAligned && aligned16));
+    if (p.bm == 128) launch_tile<Tile128w8, Tile128>(p, dtl, alpha, beta, C, ldC, mirror);
+    else launch_tile<Tile64, Tile64>(p, dtl, alpha, beta, C, ldC, mirror);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return ca3::fail(e, "gram_partial_kernel");
-    gram_reduce_kernel<<<dim3(16, g.npairs), 256, 0, st>>>(g.P, g.n, g.ntile, g.npairs, g.ksplit, alpha, beta, C,
-                                                          ldC, mirror ? 1 : 0);
-    return ca3::finish();
+    return e != hipSuccess ? ca3::fail(e, "gram kernels") : HIP_PROXY_OK;
 }
 
 }  // namespace
@@ -182,9 +327,8 @@ int hip_dsyrk_gram(const int n, const int k, const double alpha, const double *A
 {
     int rc = check_args(n, k, A, ldA, C, ldC);
     if (rc || n == 0) return rc;
-    GramArgs g;
-    plan(n, k, &g);
-    const size_t bytes = sizeof(double) * (size_t) g.ksplit * g.npairs * kBM * kBN;
+    Plan p = plan(n, k);
+    const size_t bytes = sizeof(double) * (size_t) p.wgs * p.bm * p.bm;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) dev = 0;
     Ws &w = g_gram_ws[dev & 15];
@@ -200,9 +344,10 @@ int hip_dsyrk_gram(const int n, const int k, const double alpha, const double *A
             CA3_CHECK(hipMalloc(&w.p, bytes));
             w.bytes = bytes;
         }
+        p.g.A = A; p.g.lda = ldA; p.g.P = (double *) w.p;
+        rc = launch(p, alpha, beta, C, ldC, mirror);
     }
-    g.A = A; g.lda = ldA; g.P = (double *) w.p;
-    return launch(g, alpha, beta, C, ldC, mirror);
+    return rc ? rc : ca3::finish();
 }
 
 int hip_dsyrk_gram_noalloc(const int n, const int k, const double alpha, const double *A, const int ldA,
@@ -210,30 +355,29 @@ int hip_dsyrk_gram_noalloc(const int n, const int k, const double alpha, const d
 {
     int rc = check_args(n, k, A, ldA, C, ldC);
     if (rc || n == 0) return rc;
-    GramArgs g;
-    plan(n, k, &g);
     static_assert(sizeof(scratch) == sizeof(double) * (size_t) kScratchTiles * kBM * kBN, "scratch size");
-    if ((int64_t) g.ksplit * g.npairs > kScratchTiles)
+    const int64_t nt = ((int64_t) n + kBM - 1) / kBM;
+    if (nt * (nt + 1) / 2 > kScratchTiles)
         return ca3::fail_msg(HIP_PROXY_ERR_ARG,
                              "gram_noalloc: n = %d, k = %d needs %lld partial 128 x 128 tiles; the fixed scratch "
-                             "holds %d (n <= 3968)", n, k, (long long) g.ksplit * g.npairs, kScratchTiles);
+                             "holds %d (n <= 3968)", n, k, (long long) (nt * (nt + 1) / 2), kScratchTiles);
+    Plan p = plan(n, k);
     int dev = 0;
     CA3_CHECK(hipGetDevice(&dev));
     if (dev < 0 || dev >= 16) return ca3::fail_msg(HIP_PROXY_ERR_UNSUPP, "gram_noalloc: device %d >= 16", dev);
-    double *ptr = nullptr;
     {
         std::lock_guard<std::mutex> lk(g_gram_mu);
         if (!g_scratch_ptr[dev]) {
             // once per device, with that device current: the host-side name
             // `scratch` is not a device address
-            void *p = nullptr;
-            CA3_CHECK(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-            g_scratch_ptr[dev] = (double *) p;
+            void *q = nullptr;
+            CA3_CHECK(hipGetSymbolAddress(&q, HIP_SYMBOL(scratch)));
+            g_scratch_ptr[dev] = (double *) q;
         }
-        ptr = g_scratch_ptr[dev];
+        p.g.A = A; p.g.lda = ldA; p.g.P = g_scratch_ptr[dev];
+        rc = launch(p, alpha, beta, C, ldC, mirror);
     }
-    g.A = A; g.lda = ldA; g.P = ptr;
-    return launch(g, alpha, beta, C, ldC, mirror);
+    return rc ? rc : ca3::finish();
 }
 
 }  // extern "C"
