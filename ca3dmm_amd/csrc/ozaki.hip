@@ -1113,8 +1113,7 @@ __global__ __launch_bounds__(256) void ozaki2_residue_kernel(const double *__res
 // entry s of C = op(A) op(B), i_s = (s 2654435761 + 2135587861) mod 2^32 mod
 // m and j_s = (s 2246822519 + 3266489917) mod 2^32 mod n, with a = |row i_s
 // of op(A)| and b = |column j_s of op(B)|: sum a b, sum a^2, sum b^2,
-// sum a, sum b, max a, max b (one workgroup per sample; an estimate, so the
-// summation order is free).
+// sum a, sum b, max a, max b (an estimate, so the summation order is free).
 constexpr int kSpreadSamples = 4096;
 
 __device__ __forceinline__ void spread_accumulate(double x, double y, double v[7])
@@ -1148,19 +1147,92 @@ __device__ __forceinline__ void spread_reduce_store(const double v[7], double *_
     }
     if (threadIdx.x < 7) out[threadIdx.x] = red[threadIdx.x][0];
 }
+
+// The statistics over one range of k, lane = sample, 256 samples per
+// workgroup.  An operand that is contiguous along m or n gives a lane one
+// double of a cache line per k, and the lines of one k are shared by all
+// samples: workgroup b runs on XCD b % 8, which takes all samples of a k
+// range together, so that its L2 serves the rest of a line.  (A workgroup per
+// sample, threads along k, fetched a line per double: at 5000 x 3001 x 4001
+// with both operands so 528 us and 230 KB for the host to take logarithms of;
+// now 158 and, for the exponents, 16.)  An operand contiguous along k (AK, BK) is read
+// a line at a time by its lane.  Partials: part[(range 7 + statistic) samples
+// + sample].
+template <bool AK, bool BK>
 __global__ __launch_bounds__(256) void ozaki_spread_kernel(const double *__restrict__ A, int64_t a_sl, int64_t a_sk,
                                                             int m, const double *__restrict__ B, int64_t b_sl,
-                                                            int64_t b_sk, int n, int k, double *__restrict__ out)
+                                                            int64_t b_sk, int n, int k, int kstep,
+                                                            double *__restrict__ part)
 {
-    const int s = blockIdx.x;
+    constexpr int GROUPS = kSpreadSamples / 256, U = 8;
+    const int e = (int) (blockIdx.x >> 3), range = (e / GROUPS) * 8 + (int) (blockIdx.x & 7);
+    const int s = (e % GROUPS) * 256 + (int) threadIdx.x;
+    const int k0 = range * kstep, k1 = min(k, k0 + kstep);
+    if (k0 >= k) return;
     const uint64_t i = (((uint64_t) s * 2654435761ull + 2135587861ull) & 0xffffffffull) % (uint64_t) m;
     const uint64_t j = (((uint64_t) s * 2246822519ull + 3266489917ull) & 0xffffffffull) % (uint64_t) n;
-    const double *a = A + (int64_t) i * a_sl;
-    const double *b = B + (int64_t) j * b_sl;
+    const int64_t ak = AK ? 1 : a_sk, bk = BK ? 1 : b_sk;
+    const double *a = A + (int64_t) i * a_sl + k0 * ak;
+    const double *b = B + (int64_t) j * b_sl + k0 * bk;
     double v[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int l = threadIdx.x; l < k; l += 256)
-        spread_accumulate(fabs(a[(int64_t) l * a_sk]), fabs(b[(int64_t) l * b_sk]), v);
-    spread_reduce_store(v, out + (int64_t) s * 7);
+    int l = k0;
+    for (; l + U <= k1; l += U, a += U * ak, b += U * bk) {
+        double x[U], y[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            x[u] = a[u * ak];
+            y[u] = b[u * bk];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) spread_accumulate(fabs(x[u]), fabs(y[u]), v);
+    }
+    for (; l < k1; ++l, a += ak, b += bk) spread_accumulate(fabs(*a), fabs(*b), v);
+#pragma unroll
+    for (int q = 0; q < 7; ++q) part[((int64_t) range * 7 + q) * kSpreadSamples + s] = v[q];
+}
+
+// The exponents L and Ls of spread_exponents over 64 samples per workgroup
+// (out[2 b], out[2 b + 1]; -inf where every line is empty): the partials of a
+// sample added over the k ranges, a quarter of them per wave.
+__global__ __launch_bounds__(256) void ozaki_spread_exponents_kernel(const double *__restrict__ part, int ranges,
+                                                                     double *__restrict__ out)
+{
+    __shared__ double red[4][7][64], top[2][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const double *p = part + (int64_t) blockIdx.x * 64 + lane;
+    double v[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int r = w * ranges / 4; r < (w + 1) * ranges / 4; ++r)
+#pragma unroll
+        for (int q = 0; q < 7; ++q) {
+            const double o = p[((int64_t) r * 7 + q) * kSpreadSamples];
+            v[q] = q >= 5 ? fmax(v[q], o) : v[q] + o;
+        }
+#pragma unroll
+    for (int q = 0; q < 7; ++q) red[w][q][lane] = v[q];
+    __syncthreads();
+    if (w > 0) return;
+#pragma unroll
+    for (int q = 0; q < 7; ++q)
+        for (int u = 1; u < 4; ++u) {
+            const double o = red[u][q][lane];
+            v[q] = q >= 5 ? fmax(v[q], o) : v[q] + o;
+        }
+    double l = -INFINITY, ls = -INFINITY;
+    if (v[1] > 0.0 && v[2] > 0.0) {                         // an empty line: nothing to lose
+        const double lg = log2(v[0]);                       // -inf for disjoint supports
+        const double x = 0.5 * log2(v[1]) + 0.5 * log2(v[2]) - lg, xs = log2(v[5] * v[4] + v[6] * v[3]) - lg;
+        l = l < x ? x : l;
+        ls = ls < xs ? xs : ls;
+    }
+    top[0][lane] = l;
+    top[1][lane] = ls;
+    __builtin_amdgcn_wave_barrier();
+    if (lane < 2) {
+        double t = -INFINITY;
+        for (int u = 0; u < 64; ++u) t = t < top[lane][u] ? top[lane][u] : t;
+        out[2 * blockIdx.x + lane] = t;
+    }
 }
 
 // The statistics of sampled entries of the grouped launch's problems (the
@@ -2601,19 +2673,32 @@ int hip_ozaki_choose(hip_proxy_enum_t transA, hip_proxy_enum_t transB, const int
     if (m == 0 || n == 0 || k == 0) return hip_ozaki_counts(0.0, 0.0, k, nslices, nmoduli);
     if (!A || ldA < std::max(1, ta ? k : m)) return ca3::fail_msg(HIP_PROXY_ERR_ARG, "ozaki_choose: bad A / ldA");
     if (!B || ldB < std::max(1, tb ? n : k)) return ca3::fail_msg(HIP_PROXY_ERR_ARG, "ozaki_choose: bad B / ldB");
+    // k ranges of at least 8, at most 128 of them: 2048 workgroups
+    int kstep = (std::max(8, (k + 127) / 128) + 7) / 8 * 8;
+    const int ranges = (k + kstep - 1) / kstep, blocks = kSpreadSamples / 64;
+    const size_t words = (size_t) kSpreadSamples * 7 * ranges;
     int rc = 0;
-    double *d = (double *) workspace((size_t) kSpreadSamples * 7 * sizeof(double), &rc);
+    double *d = (double *) workspace((words + 2 * blocks) * sizeof(double), &rc);
     if (rc) return rc;
     const int64_t a_sl = ta ? ldA : 1, a_sk = ta ? 1 : ldA;
     const int64_t b_sl = tb ? 1 : ldB, b_sk = tb ? ldB : 1;
     hipStream_t st = ca3::stream();
-    ozaki_spread_kernel<<<kSpreadSamples, 256, 0, st>>>(A, a_sl, a_sk, m, B, b_sl, b_sk, n, k, d);
-    std::vector<double> h((size_t) kSpreadSamples * 7);
-    hipError_t e = hipMemcpyAsync(h.data(), d, h.size() * sizeof(double), hipMemcpyDeviceToHost, st);
+    const int grid = (ranges + 7) / 8 * 8 * (kSpreadSamples / 256);
+    if (ta && tb) ozaki_spread_kernel<true, false><<<grid, 256, 0, st>>>(A, a_sl, a_sk, m, B, b_sl, b_sk, n, k, kstep, d);
+    else if (ta) ozaki_spread_kernel<true, true><<<grid, 256, 0, st>>>(A, a_sl, a_sk, m, B, b_sl, b_sk, n, k, kstep, d);
+    else if (tb) ozaki_spread_kernel<false, false><<<grid, 256, 0, st>>>(A, a_sl, a_sk, m, B, b_sl, b_sk, n, k, kstep, d);
+    else ozaki_spread_kernel<false, true><<<grid, 256, 0, st>>>(A, a_sl, a_sk, m, B, b_sl, b_sk, n, k, kstep, d);
+    ozaki_spread_exponents_kernel<<<blocks, 256, 0, st>>>(d, ranges, d + words);
+    double h[2 * (kSpreadSamples / 64)];
+    hipError_t e = hipMemcpyAsync(h, d + words, sizeof(h), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) return ca3::fail(e, "ozaki_choose");
-    double L = 0.0, Ls = 0.0;
-    spread_exponents(h.data(), kSpreadSamples, &L, &Ls);
+    double L = -INFINITY, Ls = -INFINITY;
+    for (int q = 0; q < blocks; ++q) {
+        L = std::max(L, h[2 * q]);
+        Ls = std::max(Ls, h[2 * q + 1]);
+    }
+    if (L == -INFINITY) L = Ls = 0.0;
     return hip_ozaki_counts(L, Ls, k, nslices, nmoduli);
 }
 
