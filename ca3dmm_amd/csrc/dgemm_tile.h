@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 #include <climits>
 #include <cstdint>
+#include <type_traits>
 
 #include "hip_common.h"
 
@@ -32,9 +33,13 @@ constexpr int kMaxFoldSrc = 8;
 // registers leave room for four waves per SIMD (8192^3 TN 15.1 ms; the 4
 // waves of 64 x 64, two per SIMD, 15.45 ms; 10000 x 10000 x 500 1.52 / 1.59
 // ms); Tile64 (8 waves of 32 x 16) and Tile32 (4 waves of 16 x 16) for
-// products whose 128 x 128 tiles leave CUs idle.
-template <int BM_, int BN_, int WM_ = BM_ / 64, int WN_ = BN_ / 64>
+// products whose 128 x 128 tiles leave CUs idle.  IL (Tile128e): a wave's
+// blocks lie WM (WN) blocks apart instead of side by side, so that the blocks
+// inside C of an edge tile are spread over all waves and SIMDs, and blocks
+// outside take no MFMAs.
+template <int BM_, int BN_, int WM_ = BM_ / 64, int WN_ = BN_ / 64, bool IL_ = false>
 struct TileShape {
+    static constexpr bool IL = IL_;
     static constexpr int BM = BM_, BN = BN_;
     static constexpr int WM = WM_, WN = WN_;
     static constexpr int FI = BM / WM / 16, FJ = BN / WN / 16;
@@ -45,6 +50,7 @@ using Tile128 = TileShape<128, 128>;
 using Tile256x128 = TileShape<256, 128>;
 using Tile128x256 = TileShape<128, 256>;
 using Tile128w8 = TileShape<128, 128, 2, 4>;
+using Tile128e = TileShape<128, 128, 2, 4, true>;
 using Tile64 = TileShape<64, 64, 2, 4>;
 using Tile32 = TileShape<32, 32, 2, 2>;
 
@@ -66,6 +72,12 @@ struct GemmArgs {
     int ksplit, kstep;
     double *part;
 };
+
+// First row (column) in the tile of a wave's block i (j).
+template <class TL>
+__device__ __forceinline__ int block_row(int wm, int i) { return (TL::IL ? i * TL::WM + wm : wm * TL::FI + i) * 16; }
+template <class TL>
+__device__ __forceinline__ int block_col(int wn, int j) { return (TL::IL ? j * TL::WN + wn : wn * TL::FJ + j) * 16; }
 
 template <int FI, int FJ>
 __device__ __forceinline__ void zero(f64x4 (&acc)[FI][FJ])
@@ -202,9 +214,9 @@ __device__ __forceinline__ void stage_mfma(const double *As, const double *Bs, f
         const int kk = ks * 4 + (lane >> 4);
         double a[TL::FI], b[TL::FJ];
 #pragma unroll
-        for (int i = 0; i < TL::FI; ++i) a[i] = As[kk * TL::BM + swz(kk, (wm * TL::FI + i) * 16 + li)];
+        for (int i = 0; i < TL::FI; ++i) a[i] = As[kk * TL::BM + swz(kk, block_row<TL>(wm, i) + li)];
 #pragma unroll
-        for (int j = 0; j < TL::FJ; ++j) b[j] = Bs[kk * TL::BN + swz(kk, (wn * TL::FJ + j) * 16 + li)];
+        for (int j = 0; j < TL::FJ; ++j) b[j] = Bs[kk * TL::BN + swz(kk, block_col<TL>(wn, j) + li)];
 #pragma unroll
         for (int i = 0; i < TL::FI; ++i)
 #pragma unroll
@@ -455,9 +467,26 @@ struct DtlLoader<XC_, 1, 128, 4> {
     }
 };
 
-// The MFMAs of one stage.  lo > 0 (a stage that overlaps the one before it):
-// the k below lo of the stage count as zero in both operands.
-template <int XCA, int XCB, class TL = Tile128, bool TAIL = false>
+// The blocks of this wave that lie inside an mn x nn edge tile (mn and nn with
+// the row or column that dtl_shift moves on), in scalar registers.
+struct Blocks {
+    int fi, fj;
+};
+
+template <class TL>
+__device__ __forceinline__ Blocks blocks_inside(int mn, int nn, int ms, int ns)
+{
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave % TL::WM, wn = wave / TL::WM;
+    const int rb = (min(mn + (ms >= 0), TL::BM) + 15) >> 4, cb = (min(nn + (ns >= 0), TL::BN) + 15) >> 4;
+    return Blocks{__builtin_amdgcn_readfirstlane((rb - wm + TL::WM - 1) / TL::WM),
+                  __builtin_amdgcn_readfirstlane((cb - wn + TL::WN - 1) / TL::WN)};
+}
+
+// The MFMAs of one stage on the wave's blocks i < FIV, j < FJV.  lo > 0
+// (a stage that overlaps the one before it): the k below lo of the stage count
+// as zero in both operands.
+template <int XCA, int XCB, class TL, int FIV, int FJV, bool TAIL = false>
 __device__ __forceinline__ void stage_mfma_dtl(const double *As, const double *Bs, f64x4 (&acc)[TL::FI][TL::FJ],
                                                int lo = 0)
 {
@@ -472,19 +501,19 @@ __device__ __forceinline__ void stage_mfma_dtl(const double *As, const double *B
         const int kk = ks * 4 + (lane >> 4);
         double a[TL::FI], b[TL::FJ];
 #pragma unroll
-        for (int i = 0; i < TL::FI; ++i) {
-            a[i] = As[dtl_index<XCA, TL::BM>(kk, (wm * TL::FI + i) * 16 + li)];
+        for (int i = 0; i < FIV; ++i) {
+            a[i] = As[dtl_index<XCA, TL::BM>(kk, block_row<TL>(wm, i) + li)];
             if (TAIL) a[i] = kk >= lo ? a[i] : 0.0;
         }
 #pragma unroll
-        for (int j = 0; j < TL::FJ; ++j) {
-            b[j] = Bs[dtl_index<XCB, TL::BN>(kk, (wn * TL::FJ + j) * 16 + li)];
+        for (int j = 0; j < FJV; ++j) {
+            b[j] = Bs[dtl_index<XCB, TL::BN>(kk, block_col<TL>(wn, j) + li)];
             if (TAIL) b[j] = kk >= lo ? b[j] : 0.0;
         }
 #pragma unroll
-        for (int i = 0; i < TL::FI; ++i)
+        for (int i = 0; i < FIV; ++i)
 #pragma unroll
-            for (int j = 0; j < TL::FJ; ++j)
+            for (int j = 0; j < FJV; ++j)
                 acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j], a[i], acc[i][j], 0, 0, 0);
     }
 }
@@ -507,8 +536,10 @@ __device__ __forceinline__ void dtl_publish()
 // then count as zero.  (A separate bounds-checked stage cost a whole exposed
 // load latency.)  The products are added in the order of k either way, so
 // results do not depend on the path.  Ends with a barrier after which the
-// buffers are free.  A wave takes no part in the products of whole stages that
-// start at kw or later (its operand is zero there).
+// buffers are free.
+//
+// A wave takes no part in the products of whole stages that start at kw or
+// later (its operand is zero there).
 //
 // The two buffers of each operand must be distinct __shared__ arrays and
 // the loop is unrolled by two so that every access names its array at
@@ -519,10 +550,10 @@ __device__ __forceinline__ void dtl_publish()
 // Rings of three and four stages were slower at every size tried (8192^3
 // 16.4 and 16.9 ms against 15.1): their LDS costs the second workgroup per
 // CU, and other workgroups' waves hide the latency better than depth does.
-template <class TL, class LA, class LB>
-__device__ __forceinline__ void mainloop_dtl(const LA &la, const LB &lb, int64_t lda, int64_t ldb, int kbeg, int kend,
-                                             double *A0, double *A1, double *B0, double *B1,
-                                             f64x4 (&acc)[TL::FI][TL::FJ], int kw = INT_MAX)
+template <class TL, int FIV, int FJV, class LA, class LB>
+__device__ __forceinline__ void mainloop_blocks(const LA &la, const LB &lb, int64_t lda, int64_t ldb, int kbeg,
+                                                int kend, double *A0, double *A1, double *B0, double *B1,
+                                                f64x4 (&acc)[TL::FI][TL::FJ], int kw = INT_MAX)
 {
     constexpr int XCA = LA::XC, XCB = LB::XC;
     const int nfull = (kend - kbeg) / kBK, rem = (kend - kbeg) % kBK;
@@ -536,17 +567,52 @@ __device__ __forceinline__ void mainloop_dtl(const LA &la, const LB &lb, int64_t
     for (int z = 0; z < nfull; z += 2) {
         dtl_publish();                              // stage z in buffer 0
         if (z + 1 < ns) issue(z + 1, A1, B1);
-        if (kbeg + z * kBK < kw) stage_mfma_dtl<XCA, XCB, TL>(A0, B0, acc);
+        if (kbeg + z * kBK < kw) stage_mfma_dtl<XCA, XCB, TL, FIV, FJV>(A0, B0, acc);
         if (z + 1 >= nfull) break;
         dtl_publish();                              // stage z + 1 in buffer 1
         if (z + 2 < ns) issue(z + 2, A0, B0);
-        if (kbeg + (z + 1) * kBK < kw) stage_mfma_dtl<XCA, XCB, TL>(A1, B1, acc);
+        if (kbeg + (z + 1) * kBK < kw) stage_mfma_dtl<XCA, XCB, TL, FIV, FJV>(A1, B1, acc);
     }
     if (rem > 0) {
         dtl_publish();
-        stage_mfma_dtl<XCA, XCB, TL, true>(nfull & 1 ? A1 : A0, nfull & 1 ? B1 : B0, acc, kBK - rem);
+        stage_mfma_dtl<XCA, XCB, TL, FIV, FJV, true>(nfull & 1 ? A1 : A0, nfull & 1 ? B1 : B0, acc, kBK - rem);
     }
     __syncthreads();
+}
+
+template <class TL, class LA, class LB>
+__device__ __forceinline__ void mainloop_dtl(const LA &la, const LB &lb, int64_t lda, int64_t ldb, int kbeg, int kend,
+                                             double *A0, double *A1, double *B0, double *B1,
+                                             f64x4 (&acc)[TL::FI][TL::FJ], int kw = INT_MAX)
+{
+    mainloop_blocks<TL, TL::FI, TL::FJ>(la, lb, lda, ldb, kbeg, kend, A0, A1, B0, B1, acc, kw);
+}
+
+// The same for a tile whose blocks may lie outside C (IL): one loop per number
+// of blocks, a wave's own (a branch around each MFMA would cost copies of the
+// accumulators); all loops issue the same loads and barriers.
+template <class TL, class LA, class LB>
+__device__ __forceinline__ void mainloop_edge(const LA &la, const LB &lb, int64_t lda, int64_t ldb, int kbeg,
+                                              int kend, double *A0, double *A1, double *B0, double *B1,
+                                              f64x4 (&acc)[TL::FI][TL::FJ], const Blocks &in)
+{
+    static_assert(TL::FI == 4 && TL::FJ == 2, "the wave shape these loops are for");
+    auto run = [&](auto FIV, auto FJV) __attribute__((always_inline)) {
+        mainloop_blocks<TL, decltype(FIV)::value, decltype(FJV)::value>(la, lb, lda, ldb, kbeg, kend, A0, A1, B0, B1,
+                                                                        acc);
+    };
+    using std::integral_constant;
+    const integral_constant<int, 4> four{};
+    const integral_constant<int, 3> three{};
+    const integral_constant<int, 2> two{};
+    const integral_constant<int, 1> one{};
+    if (in.fi <= 0 || in.fj <= 0) run(integral_constant<int, 0>{}, integral_constant<int, 0>{});
+    else if (in.fj > 1) {
+        if (in.fi > 3) run(four, two);
+        else if (in.fi > 2) run(three, two);
+        else run(two, two);
+    } else if (in.fi > 2) run(four, one);
+    else run(two, one);
 }
 
 // The whole tile of acc to out, column by column (rows fastest).
@@ -561,7 +627,7 @@ __device__ __forceinline__ void store_tile(double *out, const f64x4 (&acc)[TL::F
         for (int j = 0; j < TL::FJ; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                out[((wn * TL::FJ + j) * 16 + 4 * r + (lane >> 4)) * TL::BM + (wm * TL::FI + i) * 16 + (lane & 15)] =
+                out[(block_col<TL>(wn, j) + 4 * r + (lane >> 4)) * TL::BM + block_row<TL>(wm, i) + (lane & 15)] =
                     acc[i][j][r];
 }
 
@@ -584,7 +650,7 @@ __device__ __forceinline__ void epilogue_to(const GemmArgs &g, double *C, int64_
     asm volatile("" : "+s"(m0), "+s"(n0), "+s"(ms), "+s"(ns_));
 #pragma unroll
     for (int i = 0; i < TL::FI; ++i) {
-        int rt = (wm * TL::FI + i) * 16 + (lane & 15);
+        int rt = block_row<TL>(wm, i) + (lane & 15);
         const bool rok = rt != ms && m0 + rt - (rt == ms + 1) < g.M;
         rt -= (rt == ms + 1);
         const int row = m0 + rt;
@@ -596,7 +662,7 @@ __device__ __forceinline__ void epilogue_to(const GemmArgs &g, double *C, int64_
         for (int j = 0; j < TL::FJ; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int ct = (wn * TL::FJ + j) * 16 + 4 * r + (lane >> 4);
+                const int ct = block_col<TL>(wn, j) + 4 * r + (lane >> 4);
                 col[j][r] = n0 + ct - (ct == ns_ + 1);
                 ok[j][r] = rok && ct != ns_ && col[j][r] < g.N;
             }
