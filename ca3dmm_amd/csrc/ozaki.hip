@@ -69,6 +69,22 @@ __device__ __forceinline__ double oz_unscale(double v, int ea, int eb)
     return ldexp(v, ea + eb);
 }
 
+// use(load(i)) for i = first, first + S, ... below end, eight loads in flight.
+template <int S, class Load, class Use>
+__device__ __forceinline__ void strided(int first, int end, const Load &load, const Use &use)
+{
+    constexpr int U = 8;
+    int i = first;
+    for (; i + (U - 1) * S < end; i += U * S) {
+        double x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = load(i + u * S);
+#pragma unroll
+        for (int u = 0; u < U; ++u) use(x[u]);
+    }
+    for (; i < end; i += S) use(load(i));
+}
+
 // ---------------------------------------------------------------------
 // 1. line exponents
 // ---------------------------------------------------------------------
@@ -97,8 +113,9 @@ __device__ __forceinline__ void oz_max_body(int bx, int by, int gy, const double
             if (l >= lines) break;
             const double *xl = X + (int64_t) l * sl;
             unsigned long long m = 0;
-            for (int kk = k0 + lane; kk < k1; kk += 64)
-                m = max(m, (unsigned long long) __double_as_longlong(fabs(xl[kk])));
+            strided<64>(k0 + lane, k1, [&](int kk) { return xl[kk]; }, [&](double x) {
+                m = max(m, (unsigned long long) __double_as_longlong(fabs(x)));
+            });
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off));
             if (lane == 0 && m != 0) atomicMax(&mx[l], m);
@@ -108,8 +125,10 @@ __device__ __forceinline__ void oz_max_body(int bx, int by, int gy, const double
     __shared__ unsigned long long red[256];
     unsigned long long m = 0;
     const int myline = l0 + (t & 63);
-    for (int kk = k0 + (t >> 6); kk < k1; kk += 4)
-        if (myline < lines) m = max(m, (unsigned long long) __double_as_longlong(fabs(X[myline + (int64_t) kk * sk])));
+    if (myline < lines)
+        strided<4>(k0 + (t >> 6), k1, [&](int kk) { return X[myline + (int64_t) kk * sk]; }, [&](double x) {
+            m = max(m, (unsigned long long) __double_as_longlong(fabs(x)));
+        });
     red[t] = m;
     __syncthreads();
     if (t < 64) {
@@ -896,13 +915,17 @@ __device__ __forceinline__ uint32_t crt_pack4(int r0, int r1, int r2, int r3)
 // atomics: the sum does not depend on the order.
 __device__ __forceinline__ unsigned long long crt_norm_term(double x, int E)
 {
-    if (x == 0.0) return 0ull;
-    int ex;
-    const double f = frexp(fabs(x), &ex);
-    const unsigned long long m2 = (unsigned long long) ceil(f * 16.0) * (unsigned long long) ceil(f * 16.0);
+    const unsigned long long u = (unsigned long long) __double_as_longlong(x);
+    const unsigned hi = (unsigned) (u >> 32) & 0x7fffffffu, lo = (unsigned) u;
+    if ((hi | lo) == 0) return 0ull;
+    int ex = (int) (hi >> 20) - 1022;
+    // |frac| = 1.m / 2, so ceil(16 |frac|) = 8 + ceil(8 * 0.m), from the bits
+    unsigned m4 = 8u + ((hi >> 17) & 7u) + (((hi & 0x1ffffu) | lo) != 0);
+    if (hi < 0x100000u) m4 = (unsigned) ceil(frexp(fabs(x), &ex) * 16.0);      // subnormal
+    const unsigned m2 = m4 * m4;
     const int sh = 2 * (ex - E) + 32;                 // <= 32: ex <= E
-    if (sh >= 0) return m2 << sh;
-    return ((m2 - 1) >> min(-sh, 62)) + 1;
+    if (sh >= 0) return (unsigned long long) m2 << sh;
+    return ((m2 - 1) >> min(-sh, 31)) + 1;
 }
 
 __device__ __forceinline__ void oz2_norm_body(int bx, int by, int gy, const double *__restrict__ X, int lines,
@@ -925,7 +948,7 @@ __device__ __forceinline__ void oz2_norm_body(int bx, int by, int gy, const doub
             (void) frexp(__longlong_as_double((long long) mx[l]), &E);
             const double *xl = X + (int64_t) l * sl;
             unsigned long long acc = 0;
-            for (int kk = k0 + lane; kk < k1; kk += 64) acc += crt_norm_term(xl[kk], E);
+            strided<64>(k0 + lane, k1, [&](int kk) { return xl[kk]; }, [&](double x) { acc += crt_norm_term(x, E); });
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
             if (lane == 0 && acc != 0) atomicAdd(&S[l], acc);
@@ -938,7 +961,8 @@ __device__ __forceinline__ void oz2_norm_body(int bx, int by, int gy, const doub
     if (myline < lines && mx[myline] < kNonFiniteBits) {
         int E;
         (void) frexp(__longlong_as_double((long long) mx[myline]), &E);
-        for (int kk = k0 + (t >> 6); kk < k1; kk += 4) acc += crt_norm_term(X[myline + (int64_t) kk * sk], E);
+        strided<4>(k0 + (t >> 6), k1, [&](int kk) { return X[myline + (int64_t) kk * sk]; },
+                   [&](double x) { acc += crt_norm_term(x, E); });
     }
     red[t] = acc;
     __syncthreads();
@@ -1980,7 +2004,7 @@ int ozaki_core(int ta, int tb, int m, int n, int k, double alpha, const double *
     const int64_t a_sl = ta ? ldA : 1, a_sk = ta ? 1 : ldA;
     // op(B): line j, element (l, j): B[l + j*ldB] (no trans) or B[j + l*ldB]
     const int64_t b_sl = tb ? 1 : ldB, b_sk = tb ? ldB : 1;
-    const int ky = std::min(64, std::max(1, k / 512));
+    const int ky = std::min(64, std::max(1, k / 128));   // 128 k a workgroup: enough of them
     if (k > 0) {
         ozaki_max_kernel<<<dim3((m + 63) / 64, ky), 256, 0, st>>>(A, m, k, a_sl, a_sk, mxA);
         if (!gram) ozaki_max_kernel<<<dim3((n + 63) / 64, ky), 256, 0, st>>>(B, n, k, b_sl, b_sk, mxB);
@@ -2139,7 +2163,7 @@ int ozaki2_core(int ta, int tb, int m, int n, int k, double alpha, const double 
     fill_int_kernel<<<(4 * nl + 255) / 256, 256, 0, st>>>((int *) mx, 4 * nl, 0);
     const int64_t a_sl = ta ? ldA : 1, a_sk = ta ? 1 : ldA;
     const int64_t b_sl = tb ? 1 : ldB, b_sk = tb ? ldB : 1;
-    const int ky = std::min(64, std::max(1, k / 512));
+    const int ky = std::min(64, std::max(1, k / 128));   // 128 k a workgroup: enough of them
     if (k > 0) {
         ozaki_max_kernel<<<dim3((m + 63) / 64, ky), 256, 0, st>>>(A, m, k, a_sl, a_sk, mx);
         ozaki_max_kernel<<<dim3((n + 63) / 64, ky), 256, 0, st>>>(B, n, k, b_sl, b_sk, mx + Mp);
