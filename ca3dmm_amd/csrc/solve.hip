@@ -46,11 +46,8 @@ __device__ __forceinline__ double readlane(double v, int lane)
 template <int I>
 __device__ __forceinline__ double row_lane(double v)
 {
-    const uint64_t u = (uint64_t) __double_as_longlong(v);
-    const int lo = (int) (uint32_t) u, hi = (int) (uint32_t) (u >> 32);
-    const uint32_t l = __builtin_amdgcn_update_dpp(lo, lo, 0x150 + I, 0xf, 0xf, true);     // row_newbcast:I
-    const uint32_t h = __builtin_amdgcn_update_dpp(hi, hi, 0x150 + I, 0xf, 0xf, true);
-    return __longlong_as_double((long long) (((uint64_t) h << 32) | l));
+    return __longlong_as_double(__builtin_amdgcn_update_dpp((long long) 0, __double_as_longlong(v), 0x150 + I, 0xf, 0xf,
+                                                            true));                    // row_newbcast:I
 }
 
 template <int I, int N, class F>
@@ -65,10 +62,12 @@ __device__ __forceinline__ void unrolled(const F &f)
 // 16 steps of the factorization of the 16 x 16 block d, held by every row of
 // 16 lanes (lane = column, register = row), and of the columns r.  False if a
 // pivot is outside [2^-900, 2^900] (not positive ones among them): r is then
-// of no use.  The square root and its reciprocal come from Goldschmidt's
-// iteration, the quotients from the reciprocal and one correction, which
-// leaves them as the division would round them; no branch splits the chain,
-// so that a step's updates fill the next one's latencies.
+// of no use.  The steps eliminate with p_k = d_kk itself, d_i -= (d_k / p_k)_i
+// d_k, and the rows are divided by sqrt(p_k) at the end: a step's chain is then
+// a reciprocal (two Newton iterations) and a product, and the 16 square roots
+// (Goldschmidt's iteration) overlap.  Rounding: a multiplier carries 1.5 ulp at
+// most, where two rows divided by a rounded root carry two between them; the
+// final quotients are corrected to what the division would round them to.
 __device__ __forceinline__ bool eliminate16(double (&d)[16], double (&r)[16], bool first, int col)
 {
     bool ok = true;
@@ -76,7 +75,28 @@ __device__ __forceinline__ bool eliminate16(double (&d)[16], double (&r)[16], bo
         constexpr int k = decltype(K)::value;
         const double p = row_lane<k>(d[k]);
         ok = ok && p >= 0x1p-900 && p <= 0x1p900;
-        const double y = __builtin_amdgcn_rsq(p);
+        double y = __builtin_amdgcn_rcp(p);
+        y = fma(fma(-p, y, 1.0), y, y);
+        y = fma(fma(-p, y, 1.0), y, y);
+        const double w = d[k] * y;
+        unrolled<k + 1, 16>([&](auto I) {
+            constexpr int i = decltype(I)::value;
+            const double f = -row_lane<i>(w);
+            d[i] = fma(f, d[k], d[i]);
+            r[i] = fma(f, r[k], r[i]);
+        });
+        // r keeps pace with d: left to itself the compiler runs all of d first
+        // and holds 120 multipliers for r
+        unrolled<k + 1, 16>([&](auto I) {
+            double &ri = r[decltype(I)::value];
+            asm volatile("" : "+v"(ri));
+        });
+        double &dl = d[15];
+        asm volatile("" : "+v"(dl));
+    });
+    unrolled<0, 16>([&](auto K) {
+        constexpr int k = decltype(K)::value;
+        const double p = row_lane<k>(d[k]), y = __builtin_amdgcn_rsq(p);
         double g = p * y, h = 0.5 * y, e = fma(-h, g, 0.5);
         g = fma(g, e, g);
         h = fma(h, e, h);
@@ -86,15 +106,8 @@ __device__ __forceinline__ bool eliminate16(double (&d)[16], double (&r)[16], bo
         const double piv = fma(fma(-g, g, p), h, g);
         double inv = h + h;
         inv = fma(fma(-inv, piv, 1.0), inv, inv);
-        const double qd = d[k] * inv, qr = r[k] * inv;
-        d[k] = col == k ? piv : fma(fma(-qd, piv, d[k]), inv, qd);
-        r[k] = first && col == k ? piv : fma(fma(-qr, piv, r[k]), inv, qr);
-        unrolled<k + 1, 16>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            const double f = -row_lane<i>(d[k]);
-            d[i] = fma(f, d[k], d[i]);
-            r[i] = fma(f, r[k], r[i]);
-        });
+        const double q = r[k] * inv;
+        r[k] = first && col == k ? piv : fma(fma(-q, piv, r[k]), inv, q);
     });
     return ok;
 }
@@ -120,17 +133,29 @@ __global__ __launch_bounds__(256) void potrf_row_kernel(double *A, int64_t lda, 
     __shared__ double W[kPb][LD];           // W[i][j]: row i; columns j < 64 the diagonal block, then the 64 others
     __shared__ int bad, plain;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    if (j0 > 0 && *info) return;
+    const int failed = j0 > 0 ? *info : 0;   // looked at once the loads below are under way
     const int c0 = j0 + jb + (int) blockIdx.x * kPb, nc = min(kPb, n - c0);
     double *D = A + (int64_t) j0 * lda + j0, *S = A + (int64_t) c0 * lda + j0;
     if (t == 0) bad = plain = 0;
-    // beyond jb the identity, below the diagonal and beyond nc zeros
+    // beyond jb the identity, below the diagonal and beyond nc zeros (loaded
+    // from clamped places and selected afterwards: a load under a condition
+    // would be waited for by itself)
+    double dv[kPb / 4], sv[kPb / 4];
+    const double *Sc = nc > 0 ? S : D;
+    const int ri = min(lane, jb - 1), nl = max(nc, 1) - 1;
 #pragma unroll
     for (int q = 0; q < kPb / 4; ++q) {
         const int j = wave + 4 * q;
-        W[lane][j] = (lane <= j && j < jb) ? D[(int64_t) j * lda + lane] : (lane == j ? 1.0 : 0.0);
-        W[lane][kPb + j] = (lane < jb && j < nc) ? S[(int64_t) j * lda + lane] : 0.0;
+        dv[q] = D[(int64_t) min(j, jb - 1) * lda + ri];
+        sv[q] = Sc[(int64_t) min(j, nl) * lda + ri];
     }
+#pragma unroll
+    for (int q = 0; q < kPb / 4; ++q) {
+        const int j = wave + 4 * q;
+        W[lane][j] = lane <= j && j < jb ? dv[q] : lane == j ? 1.0 : 0.0;
+        W[lane][kPb + j] = lane < jb && j < nc ? sv[q] : 0.0;
+    }
+    if (failed) return;
     __syncthreads();
     for (int s = 0; s < kPb; s += 16) {
         double r[16], d[16];
@@ -212,7 +237,7 @@ __global__ __launch_bounds__(512, 4) void potrf_update_kernel(const double *X, d
     using TL = Tile64;
     __shared__ __attribute__((aligned(1024))) double A0[kBK * TL::BM], A1[kBK * TL::BM];
     __shared__ __attribute__((aligned(1024))) double B0[kBK * TL::BN], B1[kBK * TL::BN];
-    if (*info) return;
+    const int failed = *info;                // looked at before the stores
     // tile pairs ti <= tj, column by column of the triangle
     int tj = (int) ((sqrtf(8.0f * (float) blockIdx.x + 1.0f) - 1.0f) * 0.5f);
     while (tj * (tj + 1) / 2 > (int) blockIdx.x) --tj;
@@ -245,6 +270,7 @@ __global__ __launch_bounds__(512, 4) void potrf_update_kernel(const double *X, d
         lb.init(X, lda, n0, n);
         mainloop<TL>(la, lb, 0, kPb, m0 + TL::BM <= n && n0 + TL::BN <= n, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
     }
+    if (failed) return;
 #pragma unroll
     for (int i = 0; i < TL::FI; ++i)
 #pragma unroll
@@ -260,57 +286,61 @@ __global__ __launch_bounds__(512, 4) void potrf_update_kernel(const double *X, d
 }
 
 // X = R^{-1} on the 64 x 64 diagonal blocks (the last may be smaller), one
-// workgroup each, the zeros below the diagonal included.  A wave sweeps 16
-// columns from the bottom row up, lane = row, so that a step is 16 independent
+// workgroup each, the zeros below the diagonal included.  A wave sweeps 8
+// columns from the bottom row up, lane = row, so that a step is 8 independent
 // quotients and updates.
-__global__ __launch_bounds__(256) void trtri_diag_kernel(const double *R, int64_t ldr, double *X, int64_t ldx, int n)
+__global__ __launch_bounds__(64 * kPb / 8) void trtri_diag_kernel(const double *R, int64_t ldr, double *X, int64_t ldx, int n)
 {
     __shared__ double L[kPb][kPb + 1];     // L[j][i] = R(j0 + i, j0 + j), i <= j
     const int j0 = (int) blockIdx.x * kPb, jb = min(kPb, n - j0);
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const double *D = R + (int64_t) j0 * ldr + j0;
+    constexpr int NQ = 8;                  // columns per wave, waves 64 / 8
+    double v[NQ];
 #pragma unroll
-    for (int q = 0; q < kPb / 4; ++q) {
-        const int j = wave + 4 * q;
-        L[j][lane] = (lane <= j && j < jb) ? D[(int64_t) j * ldr + lane] : (lane == j ? 1.0 : 0.0);
+    for (int q = 0; q < NQ; ++q) v[q] = D[(int64_t) min(wave + 8 * q, jb - 1) * ldr + min(lane, jb - 1)];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int j = wave + 8 * q;
+        L[j][lane] = lane <= j && j < jb ? v[q] : lane == j ? 1.0 : 0.0;
     }
     __syncthreads();
-    const int w16 = __builtin_amdgcn_readfirstlane(wave * 16);
+    const int w0 = __builtin_amdgcn_readfirstlane(wave * NQ);
     // quotients from the rounded reciprocal and one correction (the rounded
     // quotient, where nothing leaves the normal range); by division where a
     // diagonal entry is extreme
     const double dl = L[lane][lane], rdiag = 1.0 / dl;
     const bool normal = __all(fabs(dl) > 0x1p-500 && fabs(dl) < 0x1p500);
-    double x[16];
+    double x[NQ];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) x[q] = lane == w16 + q ? 1.0 : 0.0;
+    for (int q = 0; q < NQ; ++q) x[q] = lane == w0 + q ? 1.0 : 0.0;
     if (normal) {
-        for (int i = w16 + 15; i >= 0; --i) {
+        for (int i = w0 + NQ - 1; i >= 0; --i) {
             const double d = L[i][i], rd = readlane(rdiag, i), u = lane < i ? -L[i][lane] : 0.0;
-            double v[16], xi[16];
+            double t[NQ], xi[NQ];
 #pragma unroll
-            for (int q = 0; q < 16; ++q) v[q] = readlane(x[q], i);
+            for (int q = 0; q < NQ; ++q) t[q] = readlane(x[q], i);
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const double v0 = v[q] * rd, v1 = fma(fma(-v0, d, v[q]), rd, v0);
-                xi[q] = v1 == v1 ? v1 : v0;            // v not finite
+            for (int q = 0; q < NQ; ++q) {
+                const double v0 = t[q] * rd, v1 = fma(fma(-v0, d, t[q]), rd, v0);
+                xi[q] = v1 == v1 ? v1 : v0;            // t not finite
             }
 #pragma unroll
-            for (int q = 0; q < 16; ++q) x[q] = lane < i ? fma(u, xi[q], x[q]) : (lane == i ? xi[q] : x[q]);
+            for (int q = 0; q < NQ; ++q) x[q] = lane < i ? fma(u, xi[q], x[q]) : (lane == i ? xi[q] : x[q]);
         }
     } else {
-        for (int i = w16 + 15; i >= 0; --i) {
+        for (int i = w0 + NQ - 1; i >= 0; --i) {
             const double d = L[i][i], u = lane < i ? -L[i][lane] : 0.0;
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
+            for (int q = 0; q < NQ; ++q) {
                 const double xi = readlane(x[q], i) / d;
                 x[q] = lane < i ? fma(u, xi, x[q]) : (lane == i ? xi : x[q]);
             }
         }
     }
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int j = w16 + q;
+    for (int q = 0; q < NQ; ++q) {
+        const int j = w0 + q;
         if (j < jb && lane < jb) X[(int64_t) (j0 + j) * ldx + j0 + lane] = lane <= j ? x[q] : 0.0;
     }
 }
@@ -490,7 +520,7 @@ int hip_dtrtri_upper(const int n, const double *R, const int ldR, double *X, con
     const bool dtl = ca3::gemm::dtl_ld_ok(ldR) && ca3::gemm::dtl_ld_ok(ldX) &&
                      ca3::gemm::load_mode() == ca3::gemm::kLoads16;
     hipStream_t st = ca3::stream();
-    trtri_diag_kernel<<<(n + kPb - 1) / kPb, 256, 0, st>>>(R, ldR, X, ldX, n);
+    trtri_diag_kernel<<<(n + kPb - 1) / kPb, 64 * kPb / 8, 0, st>>>(R, ldR, X, ldX, n);
     for (int s = kPb; s < n; s *= 2) {
         // blocks of s joined in pairs; the last block may be alone or short
         const int pairs = (n - s + 2 * s - 1) / (2 * s), tiles = s / 32;
