@@ -310,11 +310,15 @@ TileChoice tile_choice()
 // stage: a is what the stage's latency leaves exposed, b the MFMAs of one tile
 // (measured at 64 x 64 x 2000 to 8192^3; the sum is within a few percent of
 // the runs below).  A smaller tile spreads a small product over more CUs and
-// wastes less on edges and on the last round, but moves more bytes per flop,
-// so it has to be 8 % better to be taken.  Microseconds, 128 / 64 / 32 wide:
-//   600^3  78 / 26 / 16.5    1000^3  125 / 41 / 42    1000 x 2000 x 1000
-//   125 / 71.8 / 76.8    2000^3  247 / 263 / 287    3000^3  1053 / 868 / 976
-//   10000 x 10000 x 500  1515 / 1737 / 1826    8192^3  15150 / 18830 / 21150
+// wastes less on edges and on the last round, but moves more bytes per flop:
+// up to 32 workgroups per CU that hardly shows and it is taken where it is 3 %
+// better by the sum, beyond that (where it costs up to a fifth) 20 %.
+// Microseconds, 128 / 64 / 32 wide:
+//   600^3  89 / 36 / 28    1000^3  138 / 50 / 53    1000 x 2000 x 1000
+//   138 / 80 / 85    2000^3  267 / 262 / 288    2500^3  598 / 543 / 577
+//   3000^3  1070 / 851 / 960    4000^3  1869 / 1951 / 2205    5000 x 5000 x 300
+//   276 / 259 / 284    20000 x 300 x 300  91 / 84 / 83    10000 x 10000 x 500
+//   1515 / 1737 / 1826    8192^3  15150 / 18830 / 21150
 //
 // Splits are tried at 1, 2, 4 and 8 workgroups per CU, each split at least
 // four stages long and all partial products within the buffer; one costs a
@@ -327,6 +331,9 @@ struct TileCost {
 };
 constexpr TileCost kTileCosts[] = {
     {kTile128, 128, 0.15, 1.80}, {kTile64, 64, 0.20, 0.47}, {kTile32, 32, 0.09, 0.135}};
+
+// What a smaller tile's cost has to be below, as a part of the larger one's.
+double smaller_tile_margin(int64_t wgs, int64_t cus) { return wgs <= 32 * cus ? 0.97 : 0.8; }
 
 struct Cut {
     TileChoice tile;
@@ -343,7 +350,7 @@ Cut pick_cut(int64_t M, int64_t N, int64_t K, bool may_split)
     for (const TileCost &c : kTileCosts) {
         const int64_t wgs = ((M + c.bm - 1) / c.bm) * ((N + c.bm - 1) / c.bm);
         const double us = (double) stages * (c.a + c.b * (double) ((wgs + cus - 1) / cus));
-        if (c.tile == kTile128 || us < 0.92 * t) {
+        if (c.tile == kTile128 || us < smaller_tile_margin(wgs, cus) * t) {
             best.tile = c.tile;
             t = us;
         }
@@ -556,7 +563,7 @@ int build_batch(const std::vector<Problem> &probs, bool per_segment, BatchPlan *
         const double us = wgs ? (double) work / (double) wgs *
                                     (c.a + c.b * (double) ((wgs + ca3::cu_count() - 1) / ca3::cu_count()))
                               : 0.0;
-        if (c.tile != kTile128 && !(all_dtl && us < 0.92 * best)) continue;
+        if (c.tile != kTile128 && !(all_dtl && us < smaller_tile_margin(wgs, ca3::cu_count()) * best)) continue;
         tile = c.tile;
         best = us;
         base = 0;
