@@ -1172,32 +1172,83 @@ __device__ __forceinline__ void spread_reduce_store(const double v[7], double *_
     if (threadIdx.x < 7) out[threadIdx.x] = red[threadIdx.x][0];
 }
 
+__device__ __forceinline__ uint32_t sample_row(int s, int m)
+{
+    return (uint32_t) ((((uint64_t) s * 2654435761ull + 2135587861ull) & 0xffffffffull) % (uint64_t) m);
+}
+__device__ __forceinline__ uint32_t sample_col(int s, int n)
+{
+    return (uint32_t) ((((uint64_t) s * 2246822519ull + 3266489917ull) & 0xffffffffull) % (uint64_t) n);
+}
+
+// order := the samples in buckets of neighbouring rows (COL: columns), by a
+// counting sort in LDS: 64 samples in a row then lie in a few cache lines of
+// an operand that is contiguous along m (n).  The order inside a bucket is
+// free: a sample's statistics do not depend on its place.
+template <bool COL>
+__global__ __launch_bounds__(1024) void ozaki_sample_order_kernel(int dim, int *__restrict__ order)
+{
+    constexpr int S = kSpreadSamples, PER = S / 1024;
+    __shared__ int count[S], sums[1024];
+    const int t = threadIdx.x;
+    uint32_t bucket[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) count[t + 1024 * q] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int s = t + 1024 * q;
+        bucket[q] = (uint32_t) ((uint64_t) (COL ? sample_col(s, dim) : sample_row(s, dim)) * S / (uint32_t) dim);
+        atomicAdd(&count[bucket[q]], 1);
+    }
+    __syncthreads();
+    int own = 0, before[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        before[q] = own;
+        own += count[PER * t + q];
+    }
+    sums[t] = own;
+    __syncthreads();
+    for (int w = 1; w < 1024; w *= 2) {
+        const int v = t >= w ? sums[t - w] : 0;
+        __syncthreads();
+        sums[t] += v;
+        __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < PER; ++q) count[PER * t + q] = sums[t] - own + before[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PER; ++q) order[atomicAdd(&count[bucket[q]], 1)] = t + 1024 * q;
+}
+
 // The statistics over one range of k, lane = sample, 256 samples per
 // workgroup.  An operand that is contiguous along m or n gives a lane one
 // double of a cache line per k, and the lines of one k are shared by all
 // samples: workgroup b runs on XCD b % 8, which takes all samples of a k
-// range together, so that its L2 serves the rest of a line.  (A workgroup per
+// range together, so that its L2 serves the rest of a line; one such operand's
+// lines are also shared inside a wave (order, see above).  (A workgroup per
 // sample, threads along k, fetched a line per double: at 5000 x 3001 x 4001
 // with both operands so 528 us and 230 KB for the host to take logarithms of;
-// now 158 and, for the exponents, 16.)  An operand contiguous along k (AK, BK) is read
-// a line at a time by its lane.  Partials: part[(range 7 + statistic) samples
-// + sample].
+// in the samples' own order 158, so 118, and 16 for the exponents.)  An operand
+// contiguous along k (AK, BK) is read a line at a time by its lane.
+// Partials: part[(range 7 + statistic) samples + place in order].
 template <bool AK, bool BK>
 __global__ __launch_bounds__(256) void ozaki_spread_kernel(const double *__restrict__ A, int64_t a_sl, int64_t a_sk,
                                                             int m, const double *__restrict__ B, int64_t b_sl,
                                                             int64_t b_sk, int n, int k, int kstep,
-                                                            double *__restrict__ part)
+                                                            const int *__restrict__ order, double *__restrict__ part)
 {
     constexpr int GROUPS = kSpreadSamples / 256, U = 8;
     const int e = (int) (blockIdx.x >> 3), range = (e / GROUPS) * 8 + (int) (blockIdx.x & 7);
-    const int s = (e % GROUPS) * 256 + (int) threadIdx.x;
+    const int place = (e % GROUPS) * 256 + (int) threadIdx.x;
     const int k0 = range * kstep, k1 = min(k, k0 + kstep);
     if (k0 >= k) return;
-    const uint64_t i = (((uint64_t) s * 2654435761ull + 2135587861ull) & 0xffffffffull) % (uint64_t) m;
-    const uint64_t j = (((uint64_t) s * 2246822519ull + 3266489917ull) & 0xffffffffull) % (uint64_t) n;
+    const int s = order ? order[place] : place;
     const int64_t ak = AK ? 1 : a_sk, bk = BK ? 1 : b_sk;
-    const double *a = A + (int64_t) i * a_sl + k0 * ak;
-    const double *b = B + (int64_t) j * b_sl + k0 * bk;
+    const double *a = A + (int64_t) sample_row(s, m) * a_sl + k0 * ak;
+    const double *b = B + (int64_t) sample_col(s, n) * b_sl + k0 * bk;
     double v[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     int l = k0;
     for (; l + U <= k1; l += U, a += U * ak, b += U * bk) {
@@ -1212,7 +1263,7 @@ __global__ __launch_bounds__(256) void ozaki_spread_kernel(const double *__restr
     }
     for (; l < k1; ++l, a += ak, b += bk) spread_accumulate(fabs(*a), fabs(*b), v);
 #pragma unroll
-    for (int q = 0; q < 7; ++q) part[((int64_t) range * 7 + q) * kSpreadSamples + s] = v[q];
+    for (int q = 0; q < 7; ++q) part[((int64_t) range * 7 + q) * kSpreadSamples + place] = v[q];
 }
 
 // The exponents L and Ls of spread_exponents over 64 samples per workgroup
@@ -2702,16 +2753,29 @@ int hip_ozaki_choose(hip_proxy_enum_t transA, hip_proxy_enum_t transB, const int
     const int ranges = (k + kstep - 1) / kstep, blocks = kSpreadSamples / 64;
     const size_t words = (size_t) kSpreadSamples * 7 * ranges;
     int rc = 0;
-    double *d = (double *) workspace((words + 2 * blocks) * sizeof(double), &rc);
+    double *d = (double *) workspace((words + 2 * blocks) * sizeof(double) + kSpreadSamples * sizeof(int), &rc);
     if (rc) return rc;
+    int *order = (int *) (d + words + 2 * blocks);
     const int64_t a_sl = ta ? ldA : 1, a_sk = ta ? 1 : ldA;
     const int64_t b_sl = tb ? 1 : ldB, b_sk = tb ? ldB : 1;
     hipStream_t st = ca3::stream();
     const int grid = (ranges + 7) / 8 * 8 * (kSpreadSamples / 256);
-    if (ta && tb) ozaki_spread_kernel<true, false><<<grid, 256, 0, st>>>(A, a_sl, a_sk, m, B, b_sl, b_sk, n, k, kstep, d);
-    else if (ta) ozaki_spread_kernel<true, true><<<grid, 256, 0, st>>>(A, a_sl, a_sk, m, B, b_sl, b_sk, n, k, kstep, d);
-    else if (tb) ozaki_spread_kernel<false, false><<<grid, 256, 0, st>>>(A, a_sl, a_sk, m, B, b_sl, b_sk, n, k, kstep, d);
-    else ozaki_spread_kernel<false, true><<<grid, 256, 0, st>>>(A, a_sl, a_sk, m, B, b_sl, b_sk, n, k, kstep, d);
+    // by rows for an A contiguous along m (both operands so: A's lines are
+    // shared, B's come one by one), else by columns for such a B; not where the
+    // 7 us of the sort are more than it saves (10 ns per k, and a short column
+    // stays in the L1)
+    if (k < 1024 || (ta ? n : m) < 1024) order = nullptr;
+    else if (!ta) ozaki_sample_order_kernel<false><<<1, 1024, 0, st>>>(m, order);
+    else if (tb) ozaki_sample_order_kernel<true><<<1, 1024, 0, st>>>(n, order);
+    else order = nullptr;
+    auto spread = [&](auto AK, auto BK) {
+        ozaki_spread_kernel<decltype(AK)::value, decltype(BK)::value><<<grid, 256, 0, st>>>(
+            A, a_sl, a_sk, m, B, b_sl, b_sk, n, k, kstep, order, d);
+    };
+    if (ta && tb) spread(std::true_type{}, std::false_type{});
+    else if (ta) spread(std::true_type{}, std::true_type{});
+    else if (tb) spread(std::false_type{}, std::false_type{});
+    else spread(std::false_type{}, std::true_type{});
     ozaki_spread_exponents_kernel<<<blocks, 256, 0, st>>>(d, ranges, d + words);
     double h[2 * (kSpreadSamples / 64)];
     hipError_t e = hipMemcpyAsync(h, d + words, sizeof(h), hipMemcpyDeviceToHost, st);
