@@ -12,7 +12,7 @@
 //   G  += s I  (shifted passes only) s = 11 (m n + n (n + 1)) u ||Q||_F^2,
 //                                    ||Q||_F^2 = trace(G), u = 2^-53
 //   R_p = chol(G) 'U'                hip_dpotrf, strictly lower part zeroed
-//   Q   = Q R_p^{-1}                 hip_dtrsm
+//   Q   = Q R_p^{-1}                 trsm_right_upper_out (hip_dtrsm in place)
 //   R   = R_p R                      hip_dgemm
 // The shift is the one of Fukaya, Kannan, Nakatsukasa, Yamamoto, Yanagisawa,
 // "Shifted Cholesky QR for computing the QR factorization of ill-conditioned

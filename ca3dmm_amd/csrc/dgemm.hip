@@ -10,7 +10,7 @@
 // Design (MI355X / CDNA4):
 //  * v_mfma_f64_16x16x4_f64.  A workgroup of 8 wave64s owns a 128x128 tile
 //    of C, each wave 64x32 = 4x2 MFMA blocks; smaller products take 64x64 or
-//    32x32 tiles (pick_tile).
+//    32x32 tiles (pick_cut).
 //  * K advances in stages of 16, loaded direct-to-LDS into a double buffer:
 //    the next stage's loads are issued before the current stage's MFMAs, one
 //    barrier per stage.  Operands that cannot be loaded so are staged through

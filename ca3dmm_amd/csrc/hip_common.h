@@ -31,8 +31,8 @@ int finish();
 int cu_count();
 
 // X := B R^{-1} (B, X m x n, R n x n upper triangular, non-unit) with X not
-// overlapping B: R^{-1} and one FP64 MFMA DGEMM per 128-column block of X
-// straight into X (the in-place hip_dtrsm needs a copy per block).
+// overlapping B: R^{-1} and one launch for all 128-column blocks of X (the
+// in-place hip_dtrsm needs a product and a copy per block).
 int trsm_right_upper_out(int m, int n, const double *R, int ldR, const double *B, int ldB, double *X, int ldX);
 
 // FP64 multiply and add rounded separately.  hipcc contracts a * b + c into
