@@ -443,19 +443,29 @@ __global__ __launch_bounds__(512, 4) void trmm_kernel(ca3::gemm::GemmArgs g)
     epilogue<TL>(g, m0, n0, acc, dtl_shift<1, 4>(mn));
 }
 
+// The scratch of the solves, one buffer per device (R_jj and info of a
+// factorization, R^{-1} of a right solve).  A call holds the device's mutex
+// from before scratch() until its last launch is enqueued (hip_dpotrf until
+// info is read back), so that calls of several threads, which share the
+// device's stream, neither mix their launches nor free the buffer under each
+// other.
 struct Ws {
     void *p = nullptr;
     size_t bytes = 0;
+    std::mutex mu;
 };
 Ws g_ws[16];
-std::mutex g_mu;
 
-void *scratch(size_t bytes, int *rc)
+Ws &device_ws()
 {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    Ws &w = g_ws[dev & 15];
-    std::lock_guard<std::mutex> lk(g_mu);
+    return g_ws[dev & 15];
+}
+
+// At least `bytes` of w, whose mutex the caller holds.
+void *scratch(Ws &w, size_t bytes, int *rc)
+{
     *rc = 0;
     if (w.bytes < bytes) {
         if (w.p) {
@@ -483,7 +493,9 @@ int hip_dpotrf(const char uplo, const int n, double *A, const int ldA)
     if (n > kMaxN) return ca3::fail_msg(HIP_PROXY_ERR_UNSUPP, "dpotrf: n > %d", kMaxN);
     if (n == 0) return 0;
     int rc = 0;
-    int *dinfo = (int *) scratch(256 + sizeof(double) * kPb * kPb, &rc);
+    Ws &ws = device_ws();
+    std::lock_guard<std::mutex> lk(ws.mu);
+    int *dinfo = (int *) scratch(ws, 256 + sizeof(double) * kPb * kPb, &rc);
     if (rc) return rc;
     double *Rjj = (double *) ((char *) dinfo + 256);
     const bool dtl = ca3::gemm::dtl_ld_ok(ldA) && ca3::gemm::load_mode() == ca3::gemm::kLoads16;
@@ -552,10 +564,12 @@ int hip_dtrsm(hip_proxy_enum_t side, hip_proxy_enum_t uplo, hip_proxy_enum_t tra
     const int wcols = std::min(n, nb);
     int rc = 0;
     const size_t rinv_bytes = sizeof(double) * (size_t) n * n;
-    char *ws = (char *) scratch(rinv_bytes + sizeof(double) * (size_t) m * wcols + 256, &rc);
+    Ws &ws = device_ws();
+    std::unique_lock<std::mutex> lk(ws.mu);
+    char *buf = (char *) scratch(ws, rinv_bytes + sizeof(double) * (size_t) m * wcols + 256, &rc);
     if (rc) return rc;
-    double *Rinv = (double *) ws;
-    double *T = (double *) (ws + ((rinv_bytes + 255) / 256) * 256);
+    double *Rinv = (double *) buf;
+    double *T = (double *) (buf + ((rinv_bytes + 255) / 256) * 256);
     const int save = ca3::sync_mode();
     hip_proxy_set_sync(0);
     rc = hip_dtrtri_upper(n, A, ldA, Rinv, n);
@@ -566,6 +580,7 @@ int hip_dtrsm(hip_proxy_enum_t side, hip_proxy_enum_t uplo, hip_proxy_enum_t tra
         if (!rc) rc = hip_copy_matrix_block(8, w, m, T, m, B + (size_t) j0 * ldB, ldB);
     }
     hip_proxy_set_sync(save);
+    lk.unlock();
     if (rc) return rc;
     return ca3::finish();
 }
@@ -579,7 +594,9 @@ int ca3::trsm_right_upper_out(int m, int n, const double *R, int ldR, const doub
     if (m == 0 || n == 0) return HIP_PROXY_OK;
     if (n > kMaxN) return ca3::fail_msg(HIP_PROXY_ERR_UNSUPP, "trsm_right_upper_out: n > %d", kMaxN);
     int rc = 0;
-    double *Rinv = (double *) scratch(sizeof(double) * (size_t) n * n, &rc);
+    Ws &ws = device_ws();
+    std::unique_lock<std::mutex> lk(ws.mu);
+    double *Rinv = (double *) scratch(ws, sizeof(double) * (size_t) n * n, &rc);
     if (rc) return rc;
     const int save = ca3::sync_mode();
     hip_proxy_set_sync(0);
@@ -595,6 +612,7 @@ int ca3::trsm_right_upper_out(int m, int n, const double *R, int ldR, const doub
         trmm_kernel<<<(unsigned) tiles, 512, 0, ca3::stream()>>>(g);
         hipError_t e = hipGetLastError();
         hip_proxy_set_sync(save);
+        lk.unlock();
         if (e != hipSuccess) return ca3::fail(e, "trmm_kernel");
         return ca3::finish();
     }
@@ -606,6 +624,7 @@ int ca3::trsm_right_upper_out(int m, int n, const double *R, int ldR, const doub
                        X + (size_t) j0 * ldX, ldX);
     }
     hip_proxy_set_sync(save);
+    lk.unlock();
     if (rc) return rc;
     return ca3::finish();
 }
