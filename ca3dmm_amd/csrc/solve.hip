@@ -124,8 +124,10 @@ __device__ __forceinline__ bool eliminate16(double (&d)[16], double (&r)[16], bo
 // below are updated by MFMAs.  The chain of 64 pivots (square root, quotient,
 // first update) bounds it.
 //
-// info: 0 written by the first block row; a later one does nothing once info
-// is set, and writes j0 + k + 1 when its pivot k is not > 0.
+// info: 0 written by the first block row; a later one does nothing once an
+// earlier one has set it, and writes j0 + k + 1 when its pivot k is not > 0.
+// Workgroup 0 may do so while waves of the same launch still read info: those
+// take a value above j0 for none, so that all of them go on alike.
 __global__ __launch_bounds__(256) void potrf_row_kernel(double *A, int64_t lda, int j0, int jb, int n, double *Rjj,
                                                         int *info)
 {
@@ -133,7 +135,7 @@ __global__ __launch_bounds__(256) void potrf_row_kernel(double *A, int64_t lda, 
     __shared__ double W[kPb][LD];           // W[i][j]: row i; columns j < 64 the diagonal block, then the 64 others
     __shared__ int bad, plain;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int failed = j0 > 0 ? *info : 0;   // looked at once the loads below are under way
+    const int seen = j0 > 0 ? *info : 0;     // looked at once the loads below are under way
     const int c0 = j0 + jb + (int) blockIdx.x * kPb, nc = min(kPb, n - c0);
     double *D = A + (int64_t) j0 * lda + j0, *S = A + (int64_t) c0 * lda + j0;
     if (t == 0) bad = plain = 0;
@@ -155,7 +157,7 @@ __global__ __launch_bounds__(256) void potrf_row_kernel(double *A, int64_t lda, 
         W[lane][j] = lane <= j && j < jb ? dv[q] : lane == j ? 1.0 : 0.0;
         W[lane][kPb + j] = lane < jb && j < nc ? sv[q] : 0.0;
     }
-    if (failed) return;
+    if (seen > 0 && seen <= j0) return;
     __syncthreads();
     for (int s = 0; s < kPb; s += 16) {
         double r[16], d[16];
