@@ -127,7 +127,9 @@ __device__ __forceinline__ bool eliminate16(double (&d)[16], double (&r)[16], bo
 // info: 0 written by the first block row; a later one does nothing once an
 // earlier one has set it, and writes j0 + k + 1 when its pivot k is not > 0.
 // Workgroup 0 may do so while waves of the same launch still read info: those
-// take a value above j0 for none, so that all of them go on alike.
+// take a value above j0 for none, so that all of them go on alike.  The block
+// is then left as LAPACK's: factor rows before the failing pivot, and in the
+// others what remains after those; the columns right of it stay as they are.
 __global__ __launch_bounds__(256) void potrf_row_kernel(double *A, int64_t lda, int j0, int jb, int n, double *Rjj,
                                                         int *info)
 {
@@ -196,7 +198,14 @@ __global__ __launch_bounds__(256) void potrf_row_kernel(double *A, int64_t lda, 
             for (int i = 0; i < 16; ++i) W[s + i][t] = r[i];
         }
         __syncthreads();
-        if (bad) break;
+        if (bad) {
+            // the rows behind these 16 take the steps before the failing one
+            if (t < kPb)
+                for (int i = s + 16; i < kPb; ++i)
+                    for (int k = s; k < bad - 1; ++k) W[i][t] = fma(-W[k][i], W[k][t], W[i][t]);
+            __syncthreads();
+            break;
+        }
         // rows below: W(i, j) -= W(s : s + 16, i)^T W(s : s + 16, j) for the
         // block rows bi and the blocks bj >= bi of each
         const int s16 = s / 16;
@@ -220,7 +229,7 @@ __global__ __launch_bounds__(256) void potrf_row_kernel(double *A, int64_t lda, 
     if (blockIdx.x == 0) {
         const bool last = nc <= 0;
         if (t == 0 && (j0 == 0 || bad)) *info = bad ? j0 + bad : 0;
-        for (int j = wave; !bad && j < jb; j += 4)
+        for (int j = wave; j < jb; j += 4)
             if (lane <= j) (last ? D : Rjj)[(int64_t) j * (last ? lda : kPb) + lane] = W[lane][j];
     }
     for (int j = wave; !bad && j < nc; j += 4)
@@ -230,10 +239,11 @@ __global__ __launch_bounds__(256) void potrf_row_kernel(double *A, int64_t lda, 
 // The trailing update behind a block row of 64: C(i, j) -= X(:, i)^T X(:, j)
 // for i <= j < n, X of 64 rows, one 64 x 64 tile per workgroup, tiles of the
 // upper triangle only, C loaded under the products.  Workgroup 0 also puts
-// the factored diagonal block in its place.
+// the factored diagonal block (up to a failing pivot of its own, info > j0) in
+// its place.
 template <bool DTL>
 __global__ __launch_bounds__(512, 4) void potrf_update_kernel(const double *X, double *C, int64_t lda, int n,
-                                                             const double *Rjj, double *D, const int *info)
+                                                             const double *Rjj, double *D, int j0, const int *info)
 {
     using namespace ca3::gemm;
     using TL = Tile64;
@@ -272,7 +282,7 @@ __global__ __launch_bounds__(512, 4) void potrf_update_kernel(const double *X, d
         lb.init(X, lda, n0, n);
         mainloop<TL>(la, lb, 0, kPb, m0 + TL::BM <= n && n0 + TL::BN <= n, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
     }
-    if (failed) return;
+    if (failed && failed <= j0) return;
 #pragma unroll
     for (int i = 0; i < TL::FI; ++i)
 #pragma unroll
@@ -280,7 +290,8 @@ __global__ __launch_bounds__(512, 4) void potrf_update_kernel(const double *X, d
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int row = row0 + 16 * i, col = col0 + 16 * j + 4 * r;
-                if (row <= col && col < n) C[(int64_t) col * lda + row] = ca3::add_rn(c[i][j][r], -acc[i][j][r]);
+                if (!failed && row <= col && col < n)
+                    C[(int64_t) col * lda + row] = ca3::add_rn(c[i][j][r], -acc[i][j][r]);
             }
     if (blockIdx.x == 0)
         for (int e = t; e < kPb * kPb; e += TL::THREADS)
@@ -512,8 +523,8 @@ int hip_dpotrf(const char uplo, const int n, double *A, const int ldA)
         // trailing upper triangle: A(r, r) -= X^T X, X = A(j0:j0+64, r)
         double *X = A + (int64_t) (j0 + jb) * ldA + j0, *D = A + (int64_t) j0 * ldA + j0;
         const int nt = (nr + kPb - 1) / kPb;
-        if (dtl) potrf_update_kernel<true><<<nt * (nt + 1) / 2, 512, 0, ca3::stream()>>>(X, X + jb, ldA, nr, Rjj, D, dinfo);
-        else potrf_update_kernel<false><<<nt * (nt + 1) / 2, 512, 0, ca3::stream()>>>(X, X + jb, ldA, nr, Rjj, D, dinfo);
+        if (dtl) potrf_update_kernel<true><<<nt * (nt + 1) / 2, 512, 0, ca3::stream()>>>(X, X + jb, ldA, nr, Rjj, D, j0, dinfo);
+        else potrf_update_kernel<false><<<nt * (nt + 1) / 2, 512, 0, ca3::stream()>>>(X, X + jb, ldA, nr, Rjj, D, j0, dinfo);
         e = hipGetLastError();
         if (e != hipSuccess) rc = ca3::fail(e, "potrf_update_kernel");
     }

@@ -37,3 +37,19 @@ def test_rows_from_the_failing_block_on_are_the_updated_rest(hip, n, k):
     for rows, cols in ((slice(j0, j0 + NB), slice(j0 + NB, n)), (slice(j0 + NB, n), slice(j0 + NB, n))):
         m = up[rows, cols]
         assert np.abs((got - rest)[rows, cols][m]).max(initial=0.0) <= tol
+
+
+@pytest.mark.parametrize("n,k", [(64, 63), (200, 70), (300, 47), (300, 17), (130, 129), (1000, 150), (90, 64)])
+def test_rows_before_the_failing_pivot_are_factor_rows(hip, n, k):
+    """Inside the failing block: rows of the factor before the pivot, and in
+    the others the block less those rows, as LAPACK's dpotf2 leaves it."""
+    S, R = _broken(n, k)
+    j0 = k // NB * NB
+    j1 = min(n, j0 + NB)
+    d = hip.DeviceArray.from_numpy(S)
+    assert hip.potrf_upper(n, d) == k + 1
+    got = d.numpy()[j0:j1, j0:j1]
+    rest = (S - R[:k].T @ R[:k])[j0:j1, j0:j1]
+    want = np.where(np.arange(j0, j1)[:, None] < k, R[j0:j1, j0:j1], rest)
+    up = np.triu(np.ones(want.shape, bool))
+    assert np.abs((got - want)[up]).max() <= 8 * (n + 2) * U * np.abs(S).max()
