@@ -900,17 +900,14 @@ void cannon_engine_print_stat(cannon_engine_p e)
 // =====================================================================
 namespace {
 
-// C := B^T B of one rank.  Up to 3968 columns through the Gram product, half
-// the flops (1000 x 200000: 3.1 ms, as a full product 6.7 ms), whose partial
-// tiles then fit its fixed 64 MiB; a wider B as a full product.  C may share
-// memory with B in the first case: it is written after all reads.
-constexpr int kGramMaxN = 3968;
+// B^T B of one rank up to 3968 columns goes through the Gram entry that
+// allocates nothing: half the flops (1000 x 200000: 3.1 ms, as a full product
+// 6.7 ms).  Its fixed 64 MiB come with the library's code, which the engine's
+// init has loaded; where there is no room for them, and for a wider B, the
+// full product runs.
+constexpr int kGramMaxN = 3968;                // the limit of hip_dsyrk_gram_noalloc
 
-int btb_product(int n, int k, const double *B, int ldB, double *C, int ldC)
-{
-    if (n <= kGramMaxN) return hip_dsyrk_gram(n, k, 1.0, B, ldB, 0.0, C, ldC, 1);
-    return hip_dgemm(HipTrans, HipNoTrans, n, n, k, 1.0, B, ldB, B, ldB, 0.0, C, ldC);
-}
+bool btb_by_gram(int n) { return n <= kGramMaxN && ca3::grouped::gram_ready(); }
 
 ca3dmm_engine_p init_single(int m, int n, int k, int tA, int tB, const Rect &sA, const Rect &sB,
                             const Rect *dC, const int *proc_grid, bool btb, ca3dmm_comm_t comm,
@@ -933,6 +930,7 @@ ca3dmm_engine_p init_single(int m, int n, int k, int tA, int tB, const Rect &sA,
     if (dC) P.dstC = {*dC};
     ca3dmm_engine_p e = build_rank(P, 0);
     if (!e) return nullptr;
+    if (btb) (void) btb_by_gram(n);            // loads it: exec allocates nothing
     const size_t bytes = total_bytes(e);
     if (workbuf_bytes) {
         e->alloc_workbuf = 0;
@@ -1056,9 +1054,12 @@ void ca3dmm_engine_exec(ca3dmm_engine_p e, const void *src_A, const int ldA, con
                r->src_scol == r->req_scol && r->src_nrow == r->req_nrow && r->src_ncol == r->req_ncol;
     };
     const bool directC = e->redist_C ? whole(e->redist_C) : false;
-    if (!force && (e->is_BTB ? n <= kGramMaxN : whole(e->redist_A)) && whole(e->redist_B) && directC) {
-        if (e->is_BTB)
-            rc = btb_product(n, k, (const double *) src_B, ldB, (double *) dst_C, ldC);
+    // (B^T B: by the Gram product, which writes C after all reads of B, so that
+    // the two may share memory)
+    const bool gram = e->is_BTB && btb_by_gram(n);
+    if (!force && (e->is_BTB ? gram : whole(e->redist_A)) && whole(e->redist_B) && directC) {
+        if (gram)
+            rc = hip_dsyrk_gram_noalloc(n, k, 1.0, (const double *) src_B, ldB, 0.0, (double *) dst_C, ldC, 1);
         else
             rc = hip_dgemm(e->trans_A ? HipTrans : HipNoTrans, e->trans_B ? HipTrans : HipNoTrans, m, n, k,
                            1.0, (const double *) src_A, ldA, (const double *) src_B, ldB, 0.0,
@@ -1105,7 +1106,10 @@ void ca3dmm_engine_exec(ca3dmm_engine_p e, const void *src_A, const int ldA, con
             } else {
                 // C = B^T B from the redistributed B block (ca3dmm.c:1172-1265,
                 // pair transpose fused into the loads)
-                rc = btb_product(n, k, (const double *) e->B_2dmm_d, e->B_2dmm_nrow, Cdst, e->C_2dmm_nrow);
+                const double *B = (const double *) e->B_2dmm_d;
+                const int ld = e->B_2dmm_nrow;
+                rc = gram ? hip_dsyrk_gram_noalloc(n, k, 1.0, B, ld, 0.0, Cdst, e->C_2dmm_nrow, 1)
+                          : hip_dgemm(HipTrans, HipNoTrans, n, n, k, 1.0, B, ld, B, ld, 0.0, Cdst, e->C_2dmm_nrow);
             }
         }
         hip_stream_sync(nullptr);

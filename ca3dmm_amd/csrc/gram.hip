@@ -16,6 +16,7 @@
 
 #include "ca3dmm_ext.h"
 #include "dgemm_tile.h"
+#include "grouped.h"
 #include "hip_common.h"
 
 // Partial tiles of hip_dsyrk_gram_noalloc: a fixed array in device memory,
@@ -232,6 +233,17 @@ std::mutex g_gram_mu;
 constexpr int kScratchTiles = 512;   // partial 128 x 128 tiles the allocation-free entry can hold
 double *g_scratch_ptr[16];          // device address of `scratch` per device (0: not looked up yet)
 
+// Looks it up, once per device, with that device current and g_gram_mu held:
+// the host-side name `scratch` is not a device address.  The first lookup
+// loads this file's code and the array with it.
+hipError_t find_scratch(int dev)
+{
+    void *q = nullptr;
+    const hipError_t e = hipGetSymbolAddress(&q, HIP_SYMBOL(scratch));
+    if (e == hipSuccess) g_scratch_ptr[dev] = (double *) q;
+    return e;
+}
+
 // Tile width and k ranges for n x n from k, by the cost of a single product's
 // rule: a CU that holds w workgroups takes a + b w us per 16-deep stage, a
 // diagonal tile f of that b; the second launch and the partials cost what the
@@ -327,6 +339,18 @@ int launch(const Plan &p, double alpha, double beta, double *C, int ldC, int mir
 
 }  // namespace
 
+bool ca3::grouped::gram_ready()
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) {
+        (void) hipGetLastError();
+        return false;
+    }
+    std::lock_guard<std::mutex> lk(g_gram_mu);
+    if (!g_scratch_ptr[dev] && find_scratch(dev) != hipSuccess) (void) hipGetLastError();
+    return g_scratch_ptr[dev] != nullptr;
+}
+
 extern "C" {
 
 int hip_dsyrk_gram(const int n, const int k, const double alpha, const double *A, const int ldA,
@@ -375,11 +399,8 @@ int hip_dsyrk_gram_noalloc(const int n, const int k, const double alpha, const d
     {
         std::lock_guard<std::mutex> lk(g_gram_mu);
         if (!g_scratch_ptr[dev]) {
-            // once per device, with that device current: the host-side name
-            // `scratch` is not a device address
-            void *q = nullptr;
-            CA3_CHECK(hipGetSymbolAddress(&q, HIP_SYMBOL(scratch)));
-            g_scratch_ptr[dev] = (double *) q;
+            const hipError_t e = find_scratch(dev);
+            if (e != hipSuccess) return ca3::fail(e, "hipGetSymbolAddress");
         }
         p.g.A = A; p.g.lda = ldA; p.g.P = g_scratch_ptr[dev];
         rc = launch(p, alpha, beta, C, ldC, mirror);

@@ -124,8 +124,13 @@ struct SeqGraph;
 int capture_sequence(SeqGraph **out, const std::function<int()> &body);
 // The library's sync mode (hip_proxy_set_sync), for code outside the HIP sources.
 bool sync_mode();
+
 int replay_sequence(SeqGraph *g);
 void destroy_sequence(SeqGraph *g);
+
+// Whether hip_dsyrk_gram_noalloc can run on the current device (gram.hip); the
+// first call loads its fixed array.
+bool gram_ready();
 
 }  // namespace grouped
 }  // namespace ca3
