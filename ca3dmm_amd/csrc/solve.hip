@@ -19,6 +19,7 @@
 //                   produced from the last to the first through a workspace,
 //                   so B can be overwritten in place.
 #include <algorithm>
+#include <cfloat>
 #include <climits>
 #include <cstring>
 #include <mutex>
@@ -301,7 +302,8 @@ __global__ __launch_bounds__(512, 4) void potrf_update_kernel(const double *X, d
 // X = R^{-1} on the 64 x 64 diagonal blocks (the last may be smaller), one
 // workgroup each, the zeros below the diagonal included.  A wave sweeps 8
 // columns from the bottom row up, lane = row, so that a step is 8 independent
-// quotients and updates.
+// quotients and updates.  (A column takes no step behind its own row: its zeros
+// there would turn an infinity or a zero pivot of a later column into NaN.)
 __global__ __launch_bounds__(64 * kPb / 8) void trtri_diag_kernel(const double *R, int64_t ldr, double *X, int64_t ldx, int n)
 {
     __shared__ double L[kPb][kPb + 1];     // L[j][i] = R(j0 + i, j0 + j), i <= j
@@ -339,7 +341,8 @@ __global__ __launch_bounds__(64 * kPb / 8) void trtri_diag_kernel(const double *
                 xi[q] = v1 == v1 ? v1 : v0;            // t not finite
             }
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) x[q] = lane < i ? fma(u, xi[q], x[q]) : (lane == i ? xi[q] : x[q]);
+            for (int q = 0; q < NQ; ++q)
+                if (i <= w0 + q) x[q] = lane < i ? fma(u, xi[q], x[q]) : (lane == i ? xi[q] : x[q]);
         }
     } else {
         for (int i = w0 + NQ - 1; i >= 0; --i) {
@@ -347,7 +350,7 @@ __global__ __launch_bounds__(64 * kPb / 8) void trtri_diag_kernel(const double *
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
                 const double xi = readlane(x[q], i) / d;
-                x[q] = lane < i ? fma(u, xi, x[q]) : (lane == i ? xi : x[q]);
+                if (i <= w0 + q) x[q] = lane < i ? fma(u, xi, x[q]) : (lane == i ? xi : x[q]);
             }
         }
     }
@@ -355,6 +358,27 @@ __global__ __launch_bounds__(64 * kPb / 8) void trtri_diag_kernel(const double *
     for (int q = 0; q < NQ; ++q) {
         const int j = w0 + q;
         if (j < jb && lane < jb) X[(int64_t) (j0 + j) * ldx + j0 + lane] = lane <= j ? x[q] : 0.0;
+    }
+}
+
+// A wave's 16 x 16 products of a join again, each over its own k alone (PART 0:
+// k <= its row of X22^T, PART 1: k >= its row of X11): where R holds an infinity
+// or a NaN, the zeros of the triangles that a tile multiplies with it would
+// carry it into entries that do not depend on it.  In the order of k, from
+// global memory: only waves whose products are not finite come here.
+template <int PART>
+__device__ __forceinline__ void join_one_by_one(const ca3::gemm::GemmArgs &g, int row, int n0, int ct0, int ns,
+                                                ca3::gemm::f64x4 &acc)
+{
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int ct = ct0 + 4 * r, col = n0 + ct - (ct == ns + 1);
+        double v = 0.0;
+        if (row < g.M && ct != ns && col < g.N)
+            for (int k = PART ? row : 0; k < (PART ? g.K : row + 1); ++k)
+                v = fma(g.A[PART ? row + (int64_t) k * g.lda : k + (int64_t) row * g.lda],
+                        g.B[col + (int64_t) k * g.ldb], v);
+        acc[r] = v;
     }
 }
 
@@ -406,15 +430,23 @@ __global__ __launch_bounds__(256, 4) void trtri_join_kernel(const double *R, int
         da.init(g.A, g.lda, m0, mn);
         db.init(g.B, g.ldb, n0, nn);
         mainloop_dtl<TL>(da, db, g.lda, g.ldb, kbeg, kend, A0, A1, B0, B1, acc);
-        epilogue<TL>(g, m0, n0, acc, dtl_shift<PART, 4>(mn), dtl_shift<1, 4>(nn));
     } else {
         OperandLoader<PART, TL::BM, TL::THREADS> la;
         OperandLoader<1, TL::BN, TL::THREADS> lb;
         la.init(g.A, g.lda, m0, g.M);
         lb.init(g.B, g.ldb, n0, g.N);
         mainloop<TL>(la, lb, kbeg, kend, mn == TL::BM && nn == TL::BN, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
-        epilogue<TL>(g, m0, n0, acc);
     }
+    const int ns = DTL ? dtl_shift<1, 4>(nn) : -2;              // (rows: contiguous along k, or an even count)
+    bool finite = true;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) finite = finite && fabs(acc[0][0][r]) <= DBL_MAX;
+    if (!__all(finite)) {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        join_one_by_one<PART>(g, m0 + block_row<TL>(wave % TL::WM, 0) + (lane & 15), n0,
+                              block_col<TL>(wave / TL::WM, 0) + (lane >> 4), ns, acc[0][0]);
+    }
+    epilogue<TL>(g, m0, n0, acc, -2, ns);
 }
 
 // The strictly lower 64 x 64 blocks of X := 0, one workgroup per column.
