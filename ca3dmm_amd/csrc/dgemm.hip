@@ -326,11 +326,15 @@ TileChoice tile_choice()
 // be 10 % better than none.
 struct TileCost {
     TileChoice tile;
-    int bm;
+    int bm, threads;
     double a, b;
 };
 constexpr TileCost kTileCosts[] = {
-    {kTile128, 128, 0.15, 1.80}, {kTile64, 64, 0.20, 0.47}, {kTile32, 32, 0.09, 0.135}};
+    {kTile128, 128, 512, 0.15, 1.80}, {kTile64, 64, 512, 0.20, 0.47}, {kTile32, 32, 256, 0.09, 0.135}};
+
+// A grid has fewer than 2^32 threads (2 x 2^29 from 16 has more 32-wide tiles
+// than that holds; beyond 2^23 128-wide ones the 4-wave form runs).
+bool grid_fits(int64_t wgs, int threads) { return (wgs + 7) / 8 * 8 * threads < (int64_t) 1 << 32; }
 
 // What a smaller tile's cost has to be below, as a part of the larger one's.
 double smaller_tile_margin(int64_t wgs, int64_t cus) { return wgs <= 32 * cus ? 0.97 : 0.8; }
@@ -349,6 +353,7 @@ Cut pick_cut(int64_t M, int64_t N, int64_t K, bool may_split)
     double t = 0.0, ts = 0.0;
     for (const TileCost &c : kTileCosts) {
         const int64_t wgs = ((M + c.bm - 1) / c.bm) * ((N + c.bm - 1) / c.bm);
+        if (c.tile != kTile128 && !grid_fits(wgs, c.threads)) continue;
         const double us = (double) stages * (c.a + c.b * (double) ((wgs + cus - 1) / cus));
         if (c.tile == kTile128 || us < smaller_tile_margin(wgs, cus) * t) {
             best.tile = c.tile;
@@ -428,7 +433,7 @@ int launch(const GemmArgs &g, TileChoice best)
     const int wa = dtl_words(g.A, g.lda, !TA, mode), wb = dtl_words(g.B, g.ldb, TB, mode);
     // a single row (column) contiguous along m (n) has no pair to load
     const bool edges = (TA || wa == 1 || g.M > 1) && (!TB || wb == 1 || g.N > 1);
-    if (!reg_tile && wa && wb && edges && g.K >= kBK) {
+    if (!reg_tile && wa && wb && edges && g.K >= kBK && grid_fits(grid_of<Tile128w8>(g), Tile128w8::THREADS)) {
         if (wa == 4 && wb == 4) {
             switch (tc == kTileAuto ? best : tc) {
             case kTile64: return launch_dtl<TA, TB, 4, 4, Tile64, 4>(g);
@@ -567,6 +572,8 @@ int build_batch(const std::vector<Problem> &probs, bool per_segment, BatchPlan *
         const double us = wgs ? (double) work / (double) wgs *
                                     (c.a + c.b * (double) ((wgs + ca3::cu_count() - 1) / ca3::cu_count()))
                               : 0.0;
+        if (c.tile == kTile128) all_dtl = all_dtl && grid_fits(wgs, c.threads);
+        else if (!grid_fits(wgs, c.threads)) continue;
         if (c.tile != kTile128 && !(all_dtl && us < smaller_tile_margin(wgs, ca3::cu_count()) * best)) continue;
         tile = c.tile;
         best = us;
