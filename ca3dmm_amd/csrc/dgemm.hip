@@ -60,7 +60,7 @@ __device__ __forceinline__ bool locate(const GemmArgs &g, int *m0, int *n0, int 
     *n0 = __builtin_amdgcn_readfirstlane(tn * TL::BN);
     *split = __builtin_amdgcn_readfirstlane(s);
     *kbeg = *split * g.kstep;
-    *kend = min(g.K, *kbeg + g.kstep);
+    *kend = g.K - *kbeg < g.kstep ? g.K : *kbeg + g.kstep;      // (the sum may pass 2^31)
     return true;
 }
 
@@ -491,7 +491,7 @@ int run(hip_proxy_enum_t transA, hip_proxy_enum_t transB, int m, int n, int k, d
         if (!g.part) cut = pick_cut(m, n, k, false);
     }
     g.ksplit = cut.ksplit;
-    g.kstep = std::max(1, cut.stages) * kBK;
+    g.kstep = (int) std::min<int64_t>((int64_t) std::max(1, cut.stages) * kBK, INT_MAX);
     int rc;
     if (!ta && !tb) rc = launch<0, 0>(g, cut.tile);
     else if (!ta && tb) rc = launch<0, 1>(g, cut.tile);

@@ -1,5 +1,5 @@
-"""GPU: products with so many columns that their small tiles would need a grid
-of 2^32 threads or more."""
+"""GPU: products whose number of columns or length of k nears 2^31: grids of
+2^32 threads or more, ends of k ranges beyond the largest int."""
 
 import numpy as np
 import pytest
@@ -25,3 +25,16 @@ def test_two_rows_times_very_many_columns(hip):
     for i in (0, 1):
         lo, hi = got[i].min(), got[i].max()
         assert want[i] - tol[i] <= lo and hi <= want[i] + tol[i]
+
+
+@pytest.mark.parametrize("k", [2 ** 31 - 8, 2 ** 31 - 10 ** 6])
+def test_k_up_to_the_largest_int(hip, k):
+    """C = A B^T of 2 x 2 from k with entries all alike (two operands of 34 GB):
+    k equal products, summed in some order."""
+    dA = hip.DeviceArray.filled((2, k), 0x3F)
+    dB = hip.DeviceArray.filled((2, k), 0x3F)
+    dC = hip.DeviceArray.filled((2, 2), 0xFF)
+    print("[long]", k, flush=True)
+    hip.dgemm(0, 1, 2, 2, k, 1.0, dA, dB, 0.0, dC)
+    got = dC.numpy()
+    assert np.abs(got / (k * V * V) - 1.0).max() <= k * 2.0 ** -53
