@@ -210,8 +210,7 @@ int hip_cholesky_qr(const int m, const int n, double *A, const int ldA, double *
     double *W = (ip && !strcmp(ip, "1")) ? nullptr : qbuffer((size_t) m * n * sizeof(double));
     double *Q = A, *Qo = W ? W : A;
     int ldQ = ldA, ldQo = W ? m : ldA;
-    const int save = ca3::sync_mode();
-    hip_proxy_set_sync(0);
+    ca3::Unsynced unsynced;
     // plain passes still to do after the last shifted one; a plain pass
     // that breaks down is redone shifted when the variant allows it.  One
     // shifted pass divides kappa by about sqrt(11 (m n + n (n + 1)) u)
@@ -243,7 +242,7 @@ int hip_cholesky_qr(const int m, const int n, double *A, const int ldA, double *
     }
     // Q holds the last pass's result: in the buffer after an odd count
     if (!rc && Q != A) rc = hip_copy_matrix_block(8, n, m, Q, ldQ, A, ldA);
-    hip_proxy_set_sync(save);
+    unsynced.end();
     if (passes_run) *passes_run = passes;
     if (rc) return rc;
     return ca3::finish();

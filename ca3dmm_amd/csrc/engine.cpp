@@ -21,6 +21,7 @@
 #include "ca3dmm_ext.h"
 #include "ca3dmm_sim.h"
 #include "grouped.h"
+#include "unsynced.h"
 #include "hip_proxy.h"
 
 #define ENG_ERR(...) fprintf(stderr, "[ca3dmm_amd] " __VA_ARGS__)
@@ -1631,8 +1632,7 @@ int sim_exec(ca3dmm_sim *S, const void *const *src_A, const int *ldA, const void
         }
         if (rc) return rc;
     }
-    const bool save = ca3::grouped::sync_mode();
-    hip_proxy_set_sync(0);
+    ca3::Unsynced unsynced;
     const std::vector<uintptr_t> key = sequence_key(S, src_A, ldA, src_B, ldB, dst_C, ldC);
     if (!S->ozaki_auto) {
         rc = run_sequence(S, 0, key, [&]() { return sim_sequence(S, src_A, ldA, src_B, ldB, dst_C, ldC); });
@@ -1655,7 +1655,6 @@ int sim_exec(ca3dmm_sim *S, const void *const *src_A, const int *ldA, const void
             rc = run_sequence(S, 2, sequence_key(S, src_A, ldA, src_B, ldB, dst_C, ldC),
                               [&]() { return sim_products(S, dst_C, ldC); });
     }
-    hip_proxy_set_sync(save ? 1 : 0);
     if (rc) return rc;
     return hip_stream_sync(nullptr);
 }

@@ -122,9 +122,6 @@ int round_product(int m, int n, int k, const double *A, int lda, const double *B
 // synchronise, allocate or copy through the host while it is captured.
 struct SeqGraph;
 int capture_sequence(SeqGraph **out, const std::function<int()> &body);
-// The library's sync mode (hip_proxy_set_sync), for code outside the HIP sources.
-bool sync_mode();
-
 int replay_sequence(SeqGraph *g);
 void destroy_sequence(SeqGraph *g);
 

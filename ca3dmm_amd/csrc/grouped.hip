@@ -414,10 +414,9 @@ int run(Plan *p, bool use_graph)
         drop_graph(p);
     if (!p->exec) {
         CA3_CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        const bool sync_saved = ca3::sync_mode();
-        hip_proxy_set_sync(0);                    // no stream synchronisation inside the capture
+        ca3::Unsynced unsynced;                   // no stream synchronisation inside the capture
         int rc = launch(p, p->tune, st);
-        hip_proxy_set_sync(sync_saved ? 1 : 0);
+        unsynced.end();
         hipGraph_t g = nullptr;
         hipError_t e = hipStreamEndCapture(st, &g);
         if (rc) { if (g) (void) hipGraphDestroy(g); return rc; }
@@ -435,8 +434,7 @@ int autotune(Plan *p, int reps)
     static const int rows[] = {1, 4, 8, 16};
     hipStream_t st = ca3::stream();
     // the candidates are timed back to back: no synchronisation per launch
-    const bool sync_saved = ca3::sync_mode();
-    hip_proxy_set_sync(0);
+    ca3::Unsynced unsynced;
     hipEvent_t e0, e1;
     CA3_CHECK(hipEventCreate(&e0));
     CA3_CHECK(hipEventCreate(&e1));
@@ -464,7 +462,6 @@ int autotune(Plan *p, int reps)
     }
     (void) hipEventDestroy(e0);
     (void) hipEventDestroy(e1);
-    hip_proxy_set_sync(sync_saved ? 1 : 0);
     if (rc) return rc;
     p->tune = bt;
     store_tuning("fp64", p->signature, bt);
@@ -515,8 +512,6 @@ int capture_sequence(SeqGraph **out, const std::function<int()> &body)
     *out = sg;
     return 0;
 }
-
-bool sync_mode() { return ca3::sync_mode(); }
 
 int replay_sequence(SeqGraph *g)
 {

@@ -6,6 +6,7 @@
 #include <cstdio>
 
 #include "hip_proxy.h"
+#include "unsynced.h"
 
 namespace ca3 {
 
@@ -13,7 +14,8 @@ namespace ca3 {
 // priority, non-blocking with respect to the null stream).
 hipStream_t stream();
 
-// 1 when entry points synchronise the library stream before returning.
+// Whether entry points called by this thread synchronise the library stream
+// before returning.
 bool sync_mode();
 
 // Record a HIP failure (text kept for hip_proxy_last_error) and map it to a

@@ -19,6 +19,7 @@ hipEvent_t g_ev0[kMaxDev] = {}, g_ev1[kMaxDev] = {};
 int g_cus[kMaxDev] = {};
 std::mutex g_mu;
 bool g_sync = true;
+thread_local int g_unsynced = 0;
 thread_local char g_err[512] = "";
 
 int cur_dev()
@@ -42,7 +43,15 @@ hipStream_t stream()
     return g_stream[d];
 }
 
-bool sync_mode() { return g_sync; }
+bool sync_mode() { return g_sync && g_unsynced == 0; }
+
+Unsynced::Unsynced() { ++g_unsynced; }
+
+void Unsynced::end()
+{
+    if (on) --g_unsynced;
+    on = false;
+}
 
 int fail(hipError_t e, const char *what)
 {
@@ -67,7 +76,7 @@ int finish()
 {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(e, "kernel launch");
-    if (g_sync) {
+    if (sync_mode()) {
         e = hipStreamSynchronize(stream());
         if (e != hipSuccess) return fail(e, "hipStreamSynchronize");
     }

@@ -544,8 +544,6 @@ int hip_dpotrf(const char uplo, const int n, double *A, const int ldA)
     if (rc) return rc;
     double *Rjj = (double *) ((char *) dinfo + 256);
     const bool dtl = ca3::gemm::dtl_ld_ok(ldA) && ca3::gemm::load_mode() == ca3::gemm::kLoads16;
-    const int save = ca3::sync_mode();
-    hip_proxy_set_sync(0);
     for (int j0 = 0; j0 < n && !rc; j0 += kPb) {
         const int jb = std::min(kPb, n - j0), nr = n - j0 - jb;
         potrf_row_kernel<<<std::max(1, (nr + kPb - 1) / kPb), 256, 0, ca3::stream()>>>(A, ldA, j0, jb, n, Rjj, dinfo);
@@ -560,7 +558,6 @@ int hip_dpotrf(const char uplo, const int n, double *A, const int ldA)
         e = hipGetLastError();
         if (e != hipSuccess) rc = ca3::fail(e, "potrf_update_kernel");
     }
-    hip_proxy_set_sync(save);
     if (rc) return rc;
     int info = 0;
     CA3_CHECK(hipMemcpyAsync(&info, dinfo, sizeof(int), hipMemcpyDeviceToHost, ca3::stream()));
@@ -615,8 +612,7 @@ int hip_dtrsm(hip_proxy_enum_t side, hip_proxy_enum_t uplo, hip_proxy_enum_t tra
     if (rc) return rc;
     double *Rinv = (double *) buf;
     double *T = (double *) (buf + ((rinv_bytes + 255) / 256) * 256);
-    const int save = ca3::sync_mode();
-    hip_proxy_set_sync(0);
+    ca3::Unsynced unsynced;
     rc = hip_dtrtri_upper(n, A, ldA, Rinv, n);
     // column block jb of X = B R^{-1} needs rows 0 .. end(jb) of R^{-1}
     for (int j0 = ((n - 1) / nb) * nb; !rc && j0 >= 0; j0 -= nb) {
@@ -624,7 +620,7 @@ int hip_dtrsm(hip_proxy_enum_t side, hip_proxy_enum_t uplo, hip_proxy_enum_t tra
         rc = hip_dgemm(HipNoTrans, HipNoTrans, m, w, kk, alpha, B, ldB, Rinv + (size_t) j0 * n, n, 0.0, T, m);
         if (!rc) rc = hip_copy_matrix_block(8, w, m, T, m, B + (size_t) j0 * ldB, ldB);
     }
-    hip_proxy_set_sync(save);
+    unsynced.end();
     lk.unlock();
     if (rc) return rc;
     return ca3::finish();
@@ -643,8 +639,7 @@ int ca3::trsm_right_upper_out(int m, int n, const double *R, int ldR, const doub
     std::unique_lock<std::mutex> lk(ws.mu);
     double *Rinv = (double *) scratch(ws, sizeof(double) * (size_t) n * n, &rc);
     if (rc) return rc;
-    const int save = ca3::sync_mode();
-    hip_proxy_set_sync(0);
+    ca3::Unsynced unsynced;
     rc = hip_dtrtri_upper(n, R, ldR, Rinv, n);
     const int64_t tiles = (int64_t) ((m + 127) / 128 + 7) / 8 * 8 * ((n + 127) / 128);
     if (!rc && m > 1 && n >= gemm::kBK && tiles <= INT_MAX && gemm::dtl_ld_ok(ldB) && ((uintptr_t) B % 8) == 0 &&
@@ -656,7 +651,7 @@ int ca3::trsm_right_upper_out(int m, int n, const double *R, int ldR, const doub
         g.A = B; g.lda = ldB; g.B = Rinv; g.ldb = n; g.C = X; g.ldc = ldX;
         trmm_kernel<<<(unsigned) tiles, 512, 0, ca3::stream()>>>(g);
         hipError_t e = hipGetLastError();
-        hip_proxy_set_sync(save);
+        unsynced.end();
         lk.unlock();
         if (e != hipSuccess) return ca3::fail(e, "trmm_kernel");
         return ca3::finish();
@@ -668,7 +663,7 @@ int ca3::trsm_right_upper_out(int m, int n, const double *R, int ldR, const doub
         rc = hip_dgemm(HipNoTrans, HipNoTrans, m, w, kk, 1.0, B, ldB, Rinv + (size_t) j0 * n, n, 0.0,
                        X + (size_t) j0 * ldX, ldX);
     }
-    hip_proxy_set_sync(save);
+    unsynced.end();
     lk.unlock();
     if (rc) return rc;
     return ca3::finish();
