@@ -87,15 +87,22 @@ struct Ws {
     void *p = nullptr;
     size_t bytes = 0;
 };
-Ws g_ws[16];
-std::mutex g_mu;
+// G, R_p R and the diagonal's range, and the out-of-place Q: one buffer each
+// per device, which a call uses from its first launch to its last one; the
+// device's mutex is held that long.
+Ws g_ws[16], g_qbuf[16];
+std::mutex g_mu[16];
 
-double *workspace(size_t bytes, int *rc)
+int device_index()
 {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    Ws &w = g_ws[dev & 15];
-    std::lock_guard<std::mutex> lk(g_mu);
+    return dev & 15;
+}
+
+// At least `bytes` of w, whose device's mutex the caller holds.
+double *workspace(Ws &w, size_t bytes, int *rc)
+{
     *rc = 0;
     if (w.bytes < bytes) {
         if (w.p) {
@@ -157,14 +164,8 @@ int one_pass(int m, int n, double *Q, int ldQ, double *Qo, int ldQo, double *G, 
 
 // The out-of-place Q buffer: cached like the workspace; nullptr (and the
 // in-place solve) when it cannot be allocated.
-Ws g_qbuf[16];
-
-double *qbuffer(size_t bytes)
+double *qbuffer(Ws &w, size_t bytes)
 {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    Ws &w = g_qbuf[dev & 15];
-    std::lock_guard<std::mutex> lk(g_mu);
     if (w.bytes < bytes) {
         if (w.p) {
             (void) hipStreamSynchronize(ca3::stream());
@@ -200,14 +201,16 @@ int hip_cholesky_qr(const int m, const int n, double *A, const int ldA, double *
     if (n == 0) return HIP_PROXY_OK;
     int rc = 0;
     const size_t nn = (size_t) n * n;
-    double *G = workspace((2 * nn + 2) * sizeof(double), &rc);
+    const int dev = device_index();
+    std::unique_lock<std::mutex> lk(g_mu[dev]);
+    double *G = workspace(g_ws[dev], (2 * nn + 2) * sizeof(double), &rc);
     if (rc) return rc;
     double *T = G + nn, *dscal = T + nn;
     // an m x n buffer (when the device has room for it) lets each pass write
     // its Q out of place: the passes alternate between A and the buffer, and
     // an odd count ends with one copy back into A
     const char *ip = getenv("CA3DMM_CHOLQR_INPLACE");
-    double *W = (ip && !strcmp(ip, "1")) ? nullptr : qbuffer((size_t) m * n * sizeof(double));
+    double *W = (ip && !strcmp(ip, "1")) ? nullptr : qbuffer(g_qbuf[dev], (size_t) m * n * sizeof(double));
     double *Q = A, *Qo = W ? W : A;
     int ldQ = ldA, ldQo = W ? m : ldA;
     ca3::Unsynced unsynced;
@@ -243,6 +246,7 @@ int hip_cholesky_qr(const int m, const int n, double *A, const int ldA, double *
     // Q holds the last pass's result: in the buffer after an odd count
     if (!rc && Q != A) rc = hip_copy_matrix_block(8, n, m, Q, ldQ, A, ldA);
     unsynced.end();
+    lk.unlock();
     if (passes_run) *passes_run = passes;
     if (rc) return rc;
     return ca3::finish();
