@@ -1923,20 +1923,27 @@ __global__ __launch_bounds__(256) void ozaki_fold_kernel(const int *__restrict__
 }
 
 // Library-owned, grow-only workspace for the planes and exponents.
+// One workspace per device.  A call holds its mutex from before workspace() to
+// its last launch (or, where it reads something back, to that), so that calls
+// of several threads, which share the device's stream, neither mix their
+// launches nor free the buffer under each other.
 struct Workspace {
     void *p = nullptr;
     size_t bytes = 0;
-    int dev = -1;
+    std::mutex mu;
 };
 Workspace g_ws[16];
-std::mutex g_ws_mu;
 
-void *workspace(size_t bytes, int *rc)
+Workspace &device_workspace()
 {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) dev = 0;
-    Workspace &w = g_ws[dev & 15];
-    std::lock_guard<std::mutex> lk(g_ws_mu);
+    return g_ws[dev & 15];
+}
+
+// At least `bytes` of w, whose mutex the caller holds.
+void *workspace(Workspace &w, size_t bytes, int *rc)
+{
     if (w.bytes < bytes) {
         if (w.p) {
             (void) hipStreamSynchronize(ca3::stream());
@@ -2038,7 +2045,9 @@ int ozaki_core(int ta, int tb, int m, int n, int k, double alpha, const double *
     const OzPlan pl = oz_plan(m, n, k, s, gram);
     const int Mp = pl.Mp, Np = pl.Np, Kp = pl.Kp;
     int rc = 0;
-    char *ws = (char *) workspace(pl.total, &rc);
+    Workspace &wsp = device_workspace();
+    std::lock_guard<std::mutex> lk(wsp.mu);
+    char *ws = (char *) workspace(wsp, pl.total, &rc);
     if (rc) return rc;
     int8_t *PA = (int8_t *) ws;
     int8_t *PB = gram ? PA : PA + pl.planesA;
@@ -2199,7 +2208,9 @@ int ozaki2_core(int ta, int tb, int m, int n, int k, double alpha, const double 
     const Oz2Plan pl = oz2_plan(m, n, k, nmod);
     const int Mp = pl.Mp, Np = pl.Np, Kp = pl.Kp;
     int rc = 0;
-    char *ws = (char *) workspace(pl.total, &rc);
+    Workspace &wsp = device_workspace();
+    std::lock_guard<std::mutex> lk(wsp.mu);
+    char *ws = (char *) workspace(wsp, pl.total, &rc);
     if (rc) return rc;
     int8_t *PA = (int8_t *) ws;
     int8_t *PB = PA + pl.planesA;
@@ -2666,7 +2677,9 @@ int choose_moduli(const std::vector<Problem> &probs, const std::vector<int> &sam
         const size_t tb = (tab.size() * sizeof(SpreadProb) + 255) / 256 * 256;
         const size_t sb = ((size_t) ns * 3 * sizeof(int) + 255) / 256 * 256;
         int rc = 0;
-        char *w = (char *) workspace(tb + sb + (size_t) ns * 7 * sizeof(double), &rc);
+        Workspace &wsp = device_workspace();
+        std::lock_guard<std::mutex> lk(wsp.mu);
+        char *w = (char *) workspace(wsp, tb + sb + (size_t) ns * 7 * sizeof(double), &rc);
         if (rc) return rc;
         hipStream_t st = ca3::stream();
         std::vector<double> h((size_t) ns * 7);
@@ -2753,7 +2766,9 @@ int hip_ozaki_choose(hip_proxy_enum_t transA, hip_proxy_enum_t transB, const int
     const int ranges = (k + kstep - 1) / kstep, blocks = kSpreadSamples / 64;
     const size_t words = (size_t) kSpreadSamples * 7 * ranges;
     int rc = 0;
-    double *d = (double *) workspace((words + 2 * blocks) * sizeof(double) + kSpreadSamples * sizeof(int), &rc);
+    Workspace &wsp = device_workspace();
+    std::lock_guard<std::mutex> lk(wsp.mu);
+    double *d = (double *) workspace(wsp, (words + 2 * blocks) * sizeof(double) + kSpreadSamples * sizeof(int), &rc);
     if (rc) return rc;
     int *order = (int *) (d + words + 2 * blocks);
     const int64_t a_sl = ta ? ldA : 1, a_sk = ta ? 1 : ldA;
