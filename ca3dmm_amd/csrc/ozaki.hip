@@ -1243,15 +1243,16 @@ __global__ __launch_bounds__(256) void ozaki_spread_kernel(const double *__restr
     constexpr int GROUPS = kSpreadSamples / 256, U = 8;
     const int e = (int) (blockIdx.x >> 3), range = (e / GROUPS) * 8 + (int) (blockIdx.x & 7);
     const int place = (e % GROUPS) * 256 + (int) threadIdx.x;
-    const int k0 = range * kstep, k1 = min(k, k0 + kstep);
-    if (k0 >= k) return;
+    const int64_t first = (int64_t) range * kstep;
+    if (first >= k) return;
+    const int k0 = (int) first, k1 = k - k0 < kstep ? k : k0 + kstep;      // (their sum may pass 2^31)
     const int s = order ? order[place] : place;
     const int64_t ak = AK ? 1 : a_sk, bk = BK ? 1 : b_sk;
     const double *a = A + (int64_t) sample_row(s, m) * a_sl + k0 * ak;
     const double *b = B + (int64_t) sample_col(s, n) * b_sl + k0 * bk;
     double v[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     int l = k0;
-    for (; l + U <= k1; l += U, a += U * ak, b += U * bk) {
+    for (; k1 - l >= U; l += U, a += U * ak, b += U * bk) {
         double x[U], y[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -2762,8 +2763,8 @@ int hip_ozaki_choose(hip_proxy_enum_t transA, hip_proxy_enum_t transB, const int
     if (!A || ldA < std::max(1, ta ? k : m)) return ca3::fail_msg(HIP_PROXY_ERR_ARG, "ozaki_choose: bad A / ldA");
     if (!B || ldB < std::max(1, tb ? n : k)) return ca3::fail_msg(HIP_PROXY_ERR_ARG, "ozaki_choose: bad B / ldB");
     // k ranges of at least 8, at most 128 of them: 2048 workgroups
-    int kstep = (std::max(8, (k + 127) / 128) + 7) / 8 * 8;
-    const int ranges = (k + kstep - 1) / kstep, blocks = kSpreadSamples / 64;
+    const int kstep = (int) ((std::max<int64_t>(8, ((int64_t) k + 127) / 128) + 7) / 8 * 8);
+    const int ranges = (int) (((int64_t) k + kstep - 1) / kstep), blocks = kSpreadSamples / 64;
     const size_t words = (size_t) kSpreadSamples * 7 * ranges;
     int rc = 0;
     Workspace &wsp = device_workspace();
