@@ -55,7 +55,7 @@ __device__ __forceinline__ bool locate(const GemmArgs &g, int *m0, int *n0, int 
     if (t >= tiles * g.ksplit) return false;
     const int s = g.ksplit > 1 ? t / tiles : 0;
     int tm, tn;
-    tile_coords<TL>(t - s * tiles, 1, g.M, g.N, &tm, &tn, g.group);    // nb = 1: no XCD remap here
+    tile_coords<TL>(t - s * tiles, g.M, g.N, &tm, &tn, g.group);
     *m0 = __builtin_amdgcn_readfirstlane(tm * TL::BM);
     *n0 = __builtin_amdgcn_readfirstlane(tn * TL::BN);
     *split = __builtin_amdgcn_readfirstlane(s);
@@ -99,8 +99,8 @@ __global__ __launch_bounds__(TL::THREADS, TL::MIN_BLOCKS) void dgemm_kernel(Gemm
     store_split<TL>(g, split, m0, n0, acc);
 }
 
-// The same product with direct-to-LDS stages; needs k >= 16 and edges that
-// can be loaded so (dtl_edge_ok).  WA / WB: 4 for 16-byte loads of an operand,
+// The same product with direct-to-LDS stages; needs k >= 16, and 16-byte loads
+// of an operand contiguous along m (n) more than one row (column).  WA / WB: 4 for 16-byte loads of an operand,
 // 1 for 4-byte loads.  The same products in the same order as dgemm_kernel,
 // whatever the tile.  WPE: waves per SIMD to leave registers for.
 template <int TA, int TB, int WA, int WB, class TL, int WPE>
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(TL::THREADS, WPE) void dgemm_batch_kernel(const Bat
     }
     const BatchProb &P = probs[lo];
     int tm, tn;
-    tile_coords<TL>((int) (t - P.base), 1, P.M, P.N, &tm, &tn, group);   // nb = 1: no XCD remap here
+    tile_coords<TL>((int) (t - P.base), P.M, P.N, &tm, &tn, group);
     const int m0 = __builtin_amdgcn_readfirstlane(tm * TL::BM), n0 = __builtin_amdgcn_readfirstlane(tn * TL::BN);
     const int mn = min(TL::BM, P.M - m0), nn = min(TL::BN, P.N - n0);
 

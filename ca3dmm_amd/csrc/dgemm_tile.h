@@ -23,14 +23,17 @@ namespace gemm {
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) double gdouble;     // in global memory (a pointer read from a table is generic)
 
-constexpr int kBM = 128, kBN = 128, kBK = 16, kThreads = 256;
+constexpr int kBM = 128, kBN = 128, kBK = 16;
 constexpr int kMaxFoldSrc = 8;
+
+template <int XC, int W = 128, int T = 256>
+struct OperandLoader;
 
 // Workgroup tile BM x BN of C: WM x WN waves along m and n, each of FI x FJ
 // MFMA blocks.  Register-staged kernels: 128 x 128 with 4 waves of 64 x 64
 // (two workgroups per CU), 256 x 128 and 128 x 256 with 8 waves (one per CU).
-// Direct-to-LDS kernels: Tile128w8, 8 waves of 64 x 32, whose 122 vector
-// registers leave room for four waves per SIMD (8192^3 TN 15.1 ms; the 4
+// Direct-to-LDS kernels: Tile128w8, 8 waves of 64 x 32, whose 117 to
+// 124 vector registers leave room for four waves per SIMD (8192^3 TN 15.1 ms; the 4
 // waves of 64 x 64, two per SIMD, 15.45 ms; 10000 x 10000 x 500 1.52 / 1.59
 // ms); Tile64 (8 waves of 32 x 16) and Tile32 (4 waves of 16 x 16) for
 // products whose 128 x 128 tiles leave CUs idle.  IL (Tile128e): a wave's
@@ -45,6 +48,9 @@ struct TileShape {
     static constexpr int FI = BM / WM / 16, FJ = BN / WN / 16;
     static constexpr int NW = WM * WN, THREADS = 64 * NW;
     static constexpr int MIN_BLOCKS = THREADS == 256 ? 2 : 1;     // per CU, for __launch_bounds__
+    // the register-staged loader of either operand of a square tile
+    template <int XC>
+    using OperandLoader = std::enable_if_t<BM_ == BN_, gemm::OperandLoader<XC, BM_, 64 * WM_ * WN_>>;
 };
 using Tile128 = TileShape<128, 128>;
 using Tile256x128 = TileShape<256, 128>;
@@ -94,20 +100,17 @@ __device__ __forceinline__ int swz(int kk, int x)
     return x ^ (((kk & 1) << 4) | ((kk >> 1) & 7));
 }
 
-// Linear workgroup id -> (tile row, tile col): XCD-contiguous ranges, then
-// groups of G tile-rows (16 unless CA3DMM_DGEMM_GROUP says otherwise)
-// walked column by column.
-template <class TL = Tile128>
-__device__ __forceinline__ void tile_coords(int bid, int nb, int M, int N, int *tm, int *tn, int G = 16)
+// Linear tile index -> (tile row, tile col): groups of G tile-rows (16 unless
+// CA3DMM_DGEMM_GROUP says otherwise) walked column by column.
+template <class TL>
+__device__ __forceinline__ void tile_coords(int t, int M, int N, int *tm, int *tn, int G)
 {
     const int tiles_m = (M + TL::BM - 1) / TL::BM, tiles_n = (N + TL::BN - 1) / TL::BN;
-    (void) tiles_n;
-    if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
     const int per = G * tiles_n;
-    const int grp = bid / per;
+    const int grp = t / per;
     const int first = grp * G;
     const int gsz = min(tiles_m - first, G);
-    const int r = bid - grp * per;
+    const int r = t - grp * per;
     *tm = first + r % gsz;
     *tn = r / gsz;
 }
@@ -117,7 +120,7 @@ __device__ __forceinline__ void tile_coords(int bid, int nb, int M, int N, int *
 // the operand is contiguous along x (m or n); XC = 0: contiguous along k.
 // Out-of-range elements read as 0.  Each thread holds P = 16 W / T elements:
 // XC = 1 at k rows kk0, kk0 + T/W, ...; XC = 0 at columns x, x + T/16, ...
-template <int XC, int W = 128, int T = 256>
+template <int XC, int W, int T>
 struct OperandLoader {
     static constexpr int P = W * kBK / T;
     static constexpr int KSTEP = T / W;         // XC: k rows per pass of the workgroup
@@ -340,13 +343,6 @@ __device__ __forceinline__ int dtl_index(int k, int x)
 // (global_load_lds_dword, lane l of load q lands at M0 + 256 q + 4 l), for
 // any xn, every x in its own slot; otherwise the same LDS image.
 __host__ __device__ constexpr bool dtl_ld_ok(int64_t ld) { return ld >= 0 && ld <= (int64_t) 1 << 26; }
-
-// Whether a tile edge of xn existing x from x0 can be loaded.
-template <int XC, int WORDS>
-__device__ __forceinline__ bool dtl_edge_ok(int x0, int xn)
-{
-    return !XC || WORDS == 1 || xn > 1 || x0 > 0;
-}
 
 // The x of the tile whose products appear one row (column) further on (see
 // above), or -2 for none.

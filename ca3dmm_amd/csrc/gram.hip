@@ -131,14 +131,6 @@ struct DiagTile {
     }
 };
 
-// The register-staged loader of a square tile, for either panel.
-template <class TL>
-struct Staged {
-    static_assert(TL::BM == TL::BN, "square tile");
-    template <int XC>
-    using OperandLoader = ca3::gemm::OperandLoader<XC, TL::BM, TL::THREADS>;
-};
-
 // One partial tile per workgroup.  DTL: 16-byte direct-to-LDS stages in 8-wave
 // workgroups; otherwise register-staged (both panels are k-contiguous, where
 // 4-byte direct-to-LDS loads lose to register staging), the same products in
@@ -188,7 +180,7 @@ __global__ __launch_bounds__(TL::THREADS, DTL ? 4 : 2) void gram_partial_kernel(
         mainloop_dtl<TL>(da, db, g.lda, g.lda, kbeg, kend, A0, A1, B0, B1, acc);
         store_tile<TL>(out, acc);
     } else {
-        typename Staged<TL>::template OperandLoader<0> la, lb;
+        typename TL::template OperandLoader<0> la, lb;
         la.init(g.A, g.lda, m0, g.n);
         lb.init(g.A, g.lda, n0, g.n);
         f64x4 acc[TL::FI][TL::FJ];

@@ -278,7 +278,7 @@ __global__ __launch_bounds__(512, 4) void potrf_update_kernel(const double *X, d
         db.init(X, lda, n0, min(TL::BN, n - n0));
         mainloop_dtl<TL>(da, db, lda, lda, 0, kPb, A0, A1, B0, B1, acc);
     } else {
-        OperandLoader<0, TL::BM, TL::THREADS> la, lb;
+        TL::OperandLoader<0> la, lb;
         la.init(X, lda, m0, n);
         lb.init(X, lda, n0, n);
         mainloop<TL>(la, lb, 0, kPb, m0 + TL::BM <= n && n0 + TL::BN <= n, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
@@ -431,8 +431,8 @@ __global__ __launch_bounds__(256, 4) void trtri_join_kernel(const double *R, int
         db.init(g.B, g.ldb, n0, nn);
         mainloop_dtl<TL>(da, db, g.lda, g.ldb, kbeg, kend, A0, A1, B0, B1, acc);
     } else {
-        OperandLoader<PART, TL::BM, TL::THREADS> la;
-        OperandLoader<1, TL::BN, TL::THREADS> lb;
+        TL::OperandLoader<PART> la;
+        TL::OperandLoader<1> lb;
         la.init(g.A, g.lda, m0, g.M);
         lb.init(g.B, g.ldb, n0, g.N);
         mainloop<TL>(la, lb, kbeg, kend, mn == TL::BM && nn == TL::BN, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
