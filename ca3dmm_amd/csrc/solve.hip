@@ -283,18 +283,18 @@ __global__ __launch_bounds__(512, 4) void potrf_update_kernel(const double *X, d
         lb.init(X, lda, n0, n);
         mainloop<TL>(la, lb, 0, kPb, m0 + TL::BM <= n && n0 + TL::BN <= n, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
     }
-    if (failed && failed <= j0) return;
+    if (!failed) {
 #pragma unroll
-    for (int i = 0; i < TL::FI; ++i)
+        for (int i = 0; i < TL::FI; ++i)
 #pragma unroll
-        for (int j = 0; j < TL::FJ; ++j)
+            for (int j = 0; j < TL::FJ; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = row0 + 16 * i, col = col0 + 16 * j + 4 * r;
-                if (!failed && row <= col && col < n)
-                    C[(int64_t) col * lda + row] = ca3::add_rn(c[i][j][r], -acc[i][j][r]);
-            }
-    if (blockIdx.x == 0)
+                for (int r = 0; r < 4; ++r) {
+                    const int row = row0 + 16 * i, col = col0 + 16 * j + 4 * r;
+                    if (row <= col && col < n) C[(int64_t) col * lda + row] = ca3::add_rn(c[i][j][r], -acc[i][j][r]);
+                }
+    }
+    if (blockIdx.x == 0 && (!failed || failed > j0))
         for (int e = t; e < kPb * kPb; e += TL::THREADS)
             if (e % kPb <= e / kPb) D[(int64_t) (e / kPb) * lda + e % kPb] = Rjj[e];
 }
