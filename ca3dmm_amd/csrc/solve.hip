@@ -330,7 +330,7 @@ __global__ __launch_bounds__(64 * kPb / 8) void trtri_diag_kernel(const double *
 #pragma unroll
     for (int q = 0; q < NQ; ++q) x[q] = lane == w0 + q ? 1.0 : 0.0;
     if (normal) {
-        for (int i = w0 + NQ - 1; i >= 0; --i) {
+        auto step = [&](int i, auto own) __attribute__((always_inline)) {       // own: one of the wave's rows
             const double d = L[i][i], rd = readlane(rdiag, i), u = lane < i ? -L[i][lane] : 0.0;
             double t[NQ], xi[NQ];
 #pragma unroll
@@ -342,8 +342,11 @@ __global__ __launch_bounds__(64 * kPb / 8) void trtri_diag_kernel(const double *
             }
 #pragma unroll
             for (int q = 0; q < NQ; ++q)
-                if (i <= w0 + q) x[q] = lane < i ? fma(u, xi[q], x[q]) : (lane == i ? xi[q] : x[q]);
-        }
+                if (!decltype(own)::value || i <= w0 + q)
+                    x[q] = lane < i ? fma(u, xi[q], x[q]) : (lane == i ? xi[q] : x[q]);
+        };
+        for (int i = w0 + NQ - 1; i > w0; --i) step(i, std::true_type{});
+        for (int i = w0; i >= 0; --i) step(i, std::false_type{});
     } else {
         for (int i = w0 + NQ - 1; i >= 0; --i) {
             const double d = L[i][i], u = lane < i ? -L[i][lane] : 0.0;
