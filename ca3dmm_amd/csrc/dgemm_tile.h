@@ -611,20 +611,28 @@ __device__ __forceinline__ void mainloop_edge(const LA &la, const LB &lb, int64_
     else run(two, one);
 }
 
-// The whole tile of acc to out, column by column (rows fastest).
+// The whole tile of acc to out, column by column (rows fastest), or added to
+// what it stored there before.
 template <class TL>
-__device__ __forceinline__ void store_tile(double *out, const f64x4 (&acc)[TL::FI][TL::FJ])
+__device__ __forceinline__ void store_tile(double *out, const f64x4 (&acc)[TL::FI][TL::FJ], bool add = false)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));                // no address is computed before the main loop
+    const int lane = tid & 63, wave = tid >> 6;
     const int wm = wave % TL::WM, wn = wave / TL::WM;
 #pragma unroll
     for (int i = 0; i < TL::FI; ++i)
 #pragma unroll
-        for (int j = 0; j < TL::FJ; ++j)
+        for (int j = 0; j < TL::FJ; ++j) {
+            double *o = out + (block_col<TL>(wn, j) + (lane >> 4)) * TL::BM + block_row<TL>(wm, i) + (lane & 15);
+            double x[4] = {0.0, 0.0, 0.0, 0.0};  // (acc, from +0 on, is never -0)
+            if (add) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                out[(block_col<TL>(wn, j) + 4 * r + (lane >> 4)) * TL::BM + block_row<TL>(wm, i) + (lane & 15)] =
-                    acc[i][j][r];
+                for (int r = 0; r < 4; ++r) x[r] = o[4 * r * TL::BM];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[4 * r * TL::BM] = ca3::add_rn(x[r], acc[i][j][r]);
+        }
 }
 
 // C := fold(P) + (alpha*acc + beta*C) for the tile at (m0, n0), with the

@@ -32,8 +32,10 @@ using namespace ca3::gemm;
 // Tile pairs (ti < tj) take k in ranges of step1, s1 of them, the tiles on the
 // diagonal ranges of step2, s2 of them.  Partials in P: pair p and range ks at
 // (ks noff + p), diagonal tile t at (noff s1 + ks ntile + t), in tiles.
+// A workgroup sums its range in chains of at most chain1 (chain2) k and adds
+// them up in its partial tile.
 struct GramArgs {
-    int n, k, ntile, noff, s1, step1, s2, step2;
+    int n, k, ntile, noff, s1, step1, s2, step2, chain1, chain2;
     const double *A;
     int64_t lda;
     double *P;
@@ -116,17 +118,24 @@ struct DiagTile {
             dtl_publish();
             mfma<true>(nfull & 1 ? S1 : S0, kBK - rem);
         }
+        __syncthreads();
     }
 
-    __device__ __forceinline__ void store(double *out) const
+    __device__ __forceinline__ void store(double *out, bool add) const
     {
-        const int lane = threadIdx.x & 63;
+        int lane = threadIdx.x & 63;
+        asm volatile("" : "+v"(lane));               // no address is computed before the main loop
 #pragma unroll
         for (int q = 0; q < MOST; ++q) {
             if (q >= count) continue;
+            double *o = out + (bj[q] * 16 + (lane >> 4)) * TL::BM + bi[q] * 16 + (lane & 15);
+            double x[4] = {0.0, 0.0, 0.0, 0.0};      // (acc, from +0 on, is never -0)
+            if (add) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                out[(bj[q] * 16 + 4 * r + (lane >> 4)) * TL::BM + bi[q] * 16 + (lane & 15)] = acc[q][r];
+                for (int r = 0; r < 4; ++r) x[r] = o[4 * r * TL::BM];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[4 * r * TL::BM] = ca3::add_rn(x[r], acc[q][r]);
         }
     }
 };
@@ -155,39 +164,58 @@ __global__ __launch_bounds__(TL::THREADS, DTL ? 4 : 2) void gram_partial_kernel(
         ks = bid / g.noff;
         pair_of(bid - ks * g.noff, g.ntile, &ti, &tj);
     }
-    const int step = diag ? g.step2 : g.step1;
+    const int step = diag ? g.step2 : g.step1, chain = diag ? g.chain2 : g.chain1;
     const int kbeg = __builtin_amdgcn_readfirstlane(ks * step);
-    const int kend = __builtin_amdgcn_readfirstlane(min(g.k, kbeg + step));
+    const int kend = __builtin_amdgcn_readfirstlane(g.k - kbeg < step ? g.k : kbeg + step);
     const int m0 = __builtin_amdgcn_readfirstlane(ti * TL::BM), n0 = __builtin_amdgcn_readfirstlane(tj * TL::BN);
+    // sum(first k, end, whether to add, m0, n0); the tile's origin is opaque in
+    // each chain, so that no address is held in registers across the main loop
+    auto chains = [&](auto sum) __attribute__((always_inline)) {
+        int k0 = kbeg;
+        do {
+            int sm0 = m0, sn0 = n0;
+            asm volatile("" : "+s"(sm0), "+s"(sn0));
+            const int k1 = __builtin_amdgcn_readfirstlane(kend - k0 < chain ? kend : k0 + chain);
+            sum(k0, k1, k0 > kbeg, sm0, sn0);
+            k0 = k1;
+        } while (k0 < kend);
+    };
     double *out = g.P + (int64_t) bid * (TL::BM * TL::BN);
     // op(A) = A^T and op(B) = A: both panels are contiguous along k.  The
     // splits start at multiples of 16, so the panels keep A's alignment; edge
     // tiles load copies of their last line in place of the missing ones.
     if constexpr (DTL) {
         DtlLoader<0, 4, TL::BM, TL::NW> da;
-        da.init(g.A, g.lda, m0, min(TL::BM, g.n - m0));
         if (diag) {
-            DiagTile<TL> tile;
-            tile.init();
-            tile.run(da, kbeg, kend, A0, A1);
-            tile.store(out);
+            chains([&](int k0, int k1, bool add, int m0, int) __attribute__((always_inline)) {
+                da.init(g.A, g.lda, m0, min(TL::BM, g.n - m0));
+                DiagTile<TL> tile;
+                tile.init();
+                tile.run(da, k0, k1, A0, A1);
+                tile.store(out, add);
+            });
             return;
         }
         DtlLoader<0, 4, TL::BN, TL::NW> db;
-        db.init(g.A, g.lda, n0, min(TL::BN, g.n - n0));
-        f64x4 acc[TL::FI][TL::FJ];
-        zero(acc);
-        mainloop_dtl<TL>(da, db, g.lda, g.lda, kbeg, kend, A0, A1, B0, B1, acc);
-        store_tile<TL>(out, acc);
+        chains([&](int k0, int k1, bool add, int m0, int n0) __attribute__((always_inline)) {
+            da.init(g.A, g.lda, m0, min(TL::BM, g.n - m0));
+            db.init(g.A, g.lda, n0, min(TL::BN, g.n - n0));
+            f64x4 acc[TL::FI][TL::FJ];
+            zero(acc);
+            mainloop_dtl<TL>(da, db, g.lda, g.lda, k0, k1, A0, A1, B0, B1, acc);
+            store_tile<TL>(out, acc, add);
+        });
     } else {
         typename TL::template OperandLoader<0> la, lb;
-        la.init(g.A, g.lda, m0, g.n);
-        lb.init(g.A, g.lda, n0, g.n);
-        f64x4 acc[TL::FI][TL::FJ];
-        zero(acc);
-        mainloop<TL>(la, lb, kbeg, kend, m0 + TL::BM <= g.n && n0 + TL::BN <= g.n, LdsPair{A0, A1}, LdsPair{B0, B1},
-                     acc);
-        store_tile<TL>(out, acc);
+        chains([&](int k0, int k1, bool add, int m0, int n0) __attribute__((always_inline)) {
+            la.init(g.A, g.lda, m0, g.n);
+            lb.init(g.A, g.lda, n0, g.n);
+            f64x4 acc[TL::FI][TL::FJ];
+            zero(acc);
+            mainloop<TL>(la, lb, k0, k1, m0 + TL::BM <= g.n && n0 + TL::BN <= g.n, LdsPair{A0, A1}, LdsPair{B0, B1},
+                         acc);
+            store_tile<TL>(out, acc, add);
+        });
     }
 }
 
@@ -205,9 +233,15 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(GramArgs g, double alp
     const int ksplit = diag ? g.s2 : g.s1;
     const int64_t step = (int64_t) (diag ? g.ntile : g.noff) * (BM * BM);
     const double *q = g.P + (diag ? (int64_t) g.noff * g.s1 + ti : (int64_t) p) * (BM * BM) + e;
-    double s = *q;
+    // sixteen ranges at a time: up to a thousand of them in one chain would cost
+    // the accuracy that short ranges give
+    double s = 0.0;
+    for (int k0 = 0; k0 < ksplit; k0 += 16) {
+        double t = q[k0 * step];
 #pragma unroll 8
-    for (int ks = 1; ks < ksplit; ++ks) s = ca3::add_rn(s, q[ks * step]);
+        for (int ks = k0 + 1; ks < min(ksplit, k0 + 16); ++ks) t = ca3::add_rn(t, q[ks * step]);
+        s = k0 ? ca3::add_rn(s, t) : t;
+    }
     double *c = C + (int64_t) gj * ldc + gi;
     double v = ca3::mul_rn(alpha, s);
     if (beta != 0.0) v = ca3::add_rn(v, ca3::mul_rn(beta, *c));
@@ -289,6 +323,19 @@ Plan plan(int n, int k)
             }
         }
     }
+    // Chains no longer than equal ranges of all 128-wide tiles in one round of
+    // the chip (of about 1024 k or more): an entry on the diagonal is a sum of
+    // squares, whose error grows with the root of the chain (1000 from 100000,
+    // rms of the relative error: in one chain per range 1.0e-15, so 4.2e-16).
+    const int64_t nt = (n + 127) / 128, pairs = nt * (nt + 1) / 2;
+    const int equal = (int) std::max<int64_t>(1, std::min<int64_t>(2 * cus / pairs, ((int64_t) k + 1023) / 1024));
+    const int most = (stages + equal - 1) / equal;
+    auto chain = [&](int step) {
+        const int len = step / kBK, parts = std::max(1, (len + most - 1) / std::max(1, most));
+        return std::max(1, (len + parts - 1) / parts) * kBK;
+    };
+    best.g.chain1 = chain(best.g.step1);
+    best.g.chain2 = chain(best.g.step2);
     return best;
 }
 
