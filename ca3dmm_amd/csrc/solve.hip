@@ -12,7 +12,8 @@
 //                   pivot k is not > 0).
 //   hip_dtrtri_upper  R^{-1} for upper-triangular R: the 64 x 64 diagonal
 //                   blocks in one launch, then pairs of inverted blocks
-//                   joined by FP64 MFMA products, the block size doubling.
+//                   joined by FP64 MFMA products and corrected once, the
+//                   block size doubling.
 //   hip_dtrsm(R,U,N,N)  B := alpha * B * R^{-1}: R^{-1} (trtri) followed by
 //                   one FP64 MFMA DGEMM per column block of the result, each
 //                   reading only the non-zero rows of R^{-1}; blocks are
@@ -364,12 +365,12 @@ __global__ __launch_bounds__(64 * kPb / 8) void trtri_diag_kernel(const double *
     }
 }
 
-// A wave's 16 x 16 products of a join again, each over its own k alone (PART 0:
-// k <= its row of X22^T, PART 1: k >= its row of X11): where R holds an infinity
+// A wave's 16 x 16 products of a join again, each over its own k alone (k <= its
+// row of X22^T, or, MUL, k >= its row of X11): where R holds an infinity
 // or a NaN, the zeros of the triangles that a tile multiplies with it would
 // carry it into entries that do not depend on it.  In the order of k, from
 // global memory: only waves whose products are not finite come here.
-template <int PART>
+template <bool MUL>
 __device__ __forceinline__ void join_one_by_one(const ca3::gemm::GemmArgs &g, int row, int n0, int ct0, int ns,
                                                 ca3::gemm::f64x4 &acc)
 {
@@ -378,11 +379,36 @@ __device__ __forceinline__ void join_one_by_one(const ca3::gemm::GemmArgs &g, in
         const int ct = ct0 + 4 * r, col = n0 + ct - (ct == ns + 1);
         double v = 0.0;
         if (row < g.M && ct != ns && col < g.N)
-            for (int k = PART ? row : 0; k < (PART ? g.K : row + 1); ++k)
-                v = fma(g.A[PART ? row + (int64_t) k * g.lda : k + (int64_t) row * g.lda],
+            for (int k = MUL ? row : 0; k < (MUL ? g.K : row + 1); ++k)
+                v = fma(g.A[MUL ? row + (int64_t) k * g.lda : k + (int64_t) row * g.lda],
                         g.B[col + (int64_t) k * g.ldb], v);
         acc[r] = v;
     }
+}
+
+// The products of a tile of X12^T with R11^T for k in [n0, n0 + 32), where R11
+// counts as zero below its diagonal: through registers into the LDS images of
+// two direct-to-LDS stages.
+__device__ __forceinline__ void join_triangle(const ca3::gemm::GemmArgs &g, int m0, int mn, int n0, double *A0,
+                                              double *A1, double *B0, double *B1, ca3::gemm::f64x4 (&acc)[1][1])
+{
+    using namespace ca3::gemm;
+    double a[4], b[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int e = (int) threadIdx.x + 256 * q, lo = e & 31, hi = e >> 5;
+        a[q] = g.A[(int64_t) (m0 + min(hi, mn - 1)) * g.lda + n0 + lo];          // k = lo, x = hi
+        b[q] = g.B[(int64_t) (n0 + hi) * g.ldb + n0 + lo];                       // k = hi, x = lo
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int e = (int) threadIdx.x + 256 * q, lo = e & 31, hi = e >> 5;
+        (lo < kBK ? A0 : A1)[dtl_index<0, 32>(lo % kBK, hi)] = a[q];
+        (hi < kBK ? B0 : B1)[dtl_index<1, 32>(hi % kBK, lo)] = lo <= hi ? b[q] : 0.0;
+    }
+    __syncthreads();
+    stage_mfma_dtl<0, 1, Tile32, 1, 1>(A0, B0, acc);
+    stage_mfma_dtl<0, 1, Tile32, 1, 1>(A1, B1, acc);
 }
 
 // Joins pairs of inverted blocks: with R11 (s x s, at o = 2 s blockIdx.y) and
@@ -393,6 +419,13 @@ __device__ __forceinline__ void join_one_by_one(const ca3::gemm::GemmArgs &g, in
 // row (last column), which passes over them and over the zeros.  With fewer
 // than 16 k the one stage starts before the block (o + s >= 64, so inside X
 // and R) and counts what it reads there as zero.
+//
+// X11 is a rounded inverse, so that R11 X12 differs from -T by some u |R11|
+// |X11| |T|, where a back substitution leaves u |R11| |X12|: at kappa(R) = 1e6
+// six times the residual R X - I, and with it 1.3 times that of a solve.  PART
+// 2 forms the transpose of what is missing, E = -T - R11 X12, in the place of
+// T, and PART 3 adds X11 E to X12, which brings both residuals back to the
+// back substitution's.  (Entries that are not finite are left as they are.)
 template <int PART, bool DTL>
 __global__ __launch_bounds__(256, 4) void trtri_join_kernel(const double *R, int64_t ldr, double *X, int64_t ldx,
                                                            int n, int s)
@@ -403,19 +436,19 @@ __global__ __launch_bounds__(256, 4) void trtri_join_kernel(const double *R, int
     __shared__ __attribute__((aligned(1024))) double B0[kBK * TL::BN], B1[kBK * TL::BN];
     const int o = 2 * s * (int) blockIdx.y, w = min(s, n - o - s);
     GemmArgs g;
-    g.M = PART ? s : w;
-    g.N = PART ? w : s;
-    g.K = g.M;
+    constexpr bool MUL = PART & 1;              // by X11
+    g.M = MUL ? s : w;
+    g.N = MUL ? w : s;
+    g.K = PART == 0 ? w : s;
     g.nsrc = 0;
-    g.alpha = PART ? -1.0 : 1.0;
-    g.beta = 0.0;
-    double *const X11 = X + (int64_t) o * ldx + o, *const X21 = X11 + s;
-    const double *const X22 = X11 + (int64_t) s * ldx + s;
-    g.A = PART ? X11 : X22;
+    g.alpha = PART == 1 || PART == 2 ? -1.0 : 1.0;
+    g.beta = PART < 2 ? 0.0 : g.alpha;
+    double *const X11 = X + (int64_t) o * ldx + o, *const X21 = X11 + s, *const X12 = X11 + (int64_t) s * ldx;
+    g.A = MUL ? X11 : PART == 0 ? X12 + s : X12;
     g.lda = ldx;
-    g.B = PART ? X21 : R + (int64_t) (o + s) * ldr + o;
-    g.ldb = PART ? ldx : ldr;
-    g.C = PART ? X11 + (int64_t) s * ldx : X21;
+    g.B = MUL ? X21 : R + (int64_t) (PART == 0 ? o + s : o) * ldr + o;
+    g.ldb = MUL ? ldx : ldr;
+    g.C = MUL ? X12 : X21;
     g.ldc = ldx;
     const int tiles_m = (g.M + TL::BM - 1) / TL::BM, tiles_n = (g.N + TL::BN - 1) / TL::BN;
     if ((int) blockIdx.x >= tiles_m * tiles_n) return;
@@ -423,30 +456,34 @@ __global__ __launch_bounds__(256, 4) void trtri_join_kernel(const double *R, int
     const int tm = (int) blockIdx.x / tiles_n;
     const int m0 = __builtin_amdgcn_readfirstlane((PART ? tm : tiles_m - 1 - tm) * TL::BM);
     const int n0 = __builtin_amdgcn_readfirstlane(((int) blockIdx.x % tiles_n) * TL::BN);
-    const int kbeg = PART ? m0 : 0, kend = PART ? s : min(w, m0 + TL::BM);
+    const int kbeg = MUL ? m0 : PART == 0 ? 0 : n0 + TL::BN, kend = PART ? s : min(w, m0 + TL::BM);
     const int mn = min(TL::BM, g.M - m0), nn = min(TL::BN, g.N - n0);
     f64x4 acc[TL::FI][TL::FJ];
     zero(acc);
     if constexpr (DTL) {
-        DtlLoader<PART, 4, TL::BM, TL::NW> da;
+        DtlLoader<MUL, 4, TL::BM, TL::NW> da;
         DtlLoader<1, 4, TL::BN, TL::NW> db;
         da.init(g.A, g.lda, m0, mn);
         db.init(g.B, g.ldb, n0, nn);
         mainloop_dtl<TL>(da, db, g.lda, g.ldb, kbeg, kend, A0, A1, B0, B1, acc);
     } else {
-        TL::OperandLoader<PART> la;
+        TL::OperandLoader<MUL> la;
         TL::OperandLoader<1> lb;
         la.init(g.A, g.lda, m0, g.M);
         lb.init(g.B, g.ldb, n0, g.N);
         mainloop<TL>(la, lb, kbeg, kend, mn == TL::BM && nn == TL::BN, LdsPair{A0, A1}, LdsPair{B0, B1}, acc);
     }
+    if constexpr (PART == 2) join_triangle(g, m0, mn, n0, A0, A1, B0, B1, acc);
     const int ns = DTL ? dtl_shift<1, 4>(nn) : -2;              // (rows: contiguous along k, or an even count)
     bool finite = true;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) finite = finite && fabs(acc[0][0][r]) <= DBL_MAX;
-    if (!__all(finite)) {
+    for (int r = 0; r < 4; ++r) {
+        finite = finite && fabs(acc[0][0][r]) <= DBL_MAX;
+        if (PART == 3 && !(fabs(acc[0][0][r]) <= DBL_MAX)) acc[0][0][r] = 0.0;
+    }
+    if (PART < 2 && !__all(finite)) {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        join_one_by_one<PART>(g, m0 + block_row<TL>(wave % TL::WM, 0) + (lane & 15), n0,
+        join_one_by_one<MUL>(g, m0 + block_row<TL>(wave % TL::WM, 0) + (lane & 15), n0,
                               block_col<TL>(wave / TL::WM, 0) + (lane >> 4), ns, acc[0][0]);
     }
     epilogue<TL>(g, m0, n0, acc, -2, ns);
@@ -582,13 +619,15 @@ int hip_dtrtri_upper(const int n, const double *R, const int ldR, double *X, con
         // blocks of s joined in pairs; the last block may be alone or short
         const int pairs = (n - s + 2 * s - 1) / (2 * s), tiles = s / 32;
         const dim3 grid((unsigned) (tiles * tiles), (unsigned) pairs);
-        if (dtl) {
-            trtri_join_kernel<0, true><<<grid, 256, 0, st>>>(R, ldR, X, ldX, n, s);
-            trtri_join_kernel<1, true><<<grid, 256, 0, st>>>(R, ldR, X, ldX, n, s);
-        } else {
-            trtri_join_kernel<0, false><<<grid, 256, 0, st>>>(R, ldR, X, ldX, n, s);
-            trtri_join_kernel<1, false><<<grid, 256, 0, st>>>(R, ldR, X, ldX, n, s);
-        }
+        auto join = [&](auto PART) {
+            constexpr int P = decltype(PART)::value;
+            if (dtl) trtri_join_kernel<P, true><<<grid, 256, 0, st>>>(R, ldR, X, ldX, n, s);
+            else trtri_join_kernel<P, false><<<grid, 256, 0, st>>>(R, ldR, X, ldX, n, s);
+        };
+        join(std::integral_constant<int, 0>{});
+        join(std::integral_constant<int, 1>{});
+        join(std::integral_constant<int, 2>{});
+        join(std::integral_constant<int, 3>{});
     }
     if (n > kPb) trtri_zero_kernel<<<n, 256, 0, st>>>(X, ldX, n);
     return ca3::finish();

@@ -125,17 +125,36 @@ def test_join_reads_stay_inside_both_matrices(n):
             assert w > 0
             x11, x22 = o * ld + o, (o + s) * ld + o + s
             x21, r12 = x11 + s, (o + s) * ld + o
-            for part in (0, 1):
-                M, N = (s, w) if part else (w, s)
+            x12 = x11 + s * ld
+            for part in (0, 1, 2):                    # (3 reads what 1 does)
+                M, N = (s, w) if part == 1 else (w, s)
+                org_a, org_b = ((x22, r12), (x11, x21), (x12, o * ld + o))[part]
                 for m0 in range(0, M, 32):
-                    kbeg, kend = (m0, s) if part else (0, min(w, m0 + 32))
                     for n0 in range(0, N, 32):
+                        kbeg, kend = ((0, min(w, m0 + 32)), (m0, s), (n0 + 32, s))[part]
                         mn, nn = min(32, M - m0), min(32, N - n0)
                         for k0, _ in (stages(kbeg, kend) if kend >= BK else [(kend - BK, BK - kend)]):
-                            for xc, org, x0, xn in ((part, x11 if part else x22, m0, mn), (1, x21 if part else r12, n0, nn)):
+                            for xc, org, x0, xn in ((part == 1, org_a, m0, mn), (1, org_b, n0, nn)):
                                 img = dtl_stage(xc, 32, 4, ld, x0, xn, k0)
                                 assert 0 <= org + min(img.values()) and org + max(img.values()) <= last
+                        if part == 2:                 # join_triangle: k in [n0, n0 + 32)
+                            assert n0 + 32 <= s and nn == 32
+                            reads = [org_a + (m0 + min(x, mn - 1)) * ld + n0 + k for x in range(32) for k in range(32)]
+                            reads += [org_b + (n0 + k) * ld + n0 + x for x in range(32) for k in range(32)]
+                            assert min(reads) >= 0 and max(reads) <= last
         s *= 2
+
+
+def test_join_triangle_fills_both_stages():
+    for xc in (0, 1):
+        seen = {}
+        for e in range(1024):
+            lo, hi = e & 31, e >> 5
+            k, x = (hi, lo) if xc else (lo, hi)
+            slot = (k >= BK, dtl_index(xc, 32, k % BK, x))
+            assert slot not in seen and slot[1] < 512
+            seen[slot] = (k, x)
+        assert len(seen) == 1024
 
 
 def tile_coords(t, M, N, W, G):
