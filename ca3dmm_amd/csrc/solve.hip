@@ -64,52 +64,43 @@ __device__ __forceinline__ void unrolled(const F &f)
 // 16 steps of the factorization of the 16 x 16 block d, held by every row of
 // 16 lanes (lane = column, register = row), and of the columns r.  False if a
 // pivot is outside [2^-900, 2^900] (not positive ones among them): r is then
-// of no use.  The steps eliminate with p_k = d_kk itself, d_i -= (d_k / p_k)_i
-// d_k, and the rows are divided by sqrt(p_k) at the end: a step's chain is then
-// a reciprocal (two Newton iterations) and a product, and the 16 square roots
-// (Goldschmidt's iteration) overlap.  Rounding: a multiplier carries 1.5 ulp at
-// most, where two rows divided by a rounded root carry two between them; the
-// final quotients are corrected to what the division would round them to.
+// of no use.  The square root comes from Goldschmidt's iteration, the quotients
+// from its reciprocal and one correction, which leaves them as the division
+// would round them, and the steps eliminate with these rounded rows: what they
+// round off comes back in the rows below.  (Eliminating with d_k / p_k and
+// taking all roots at the end leaves up to four times the backward error for
+// n <= 32, and is no shorter: 18.3 us a block row, 17.4 so.)
 __device__ __forceinline__ bool eliminate16(double (&d)[16], double (&r)[16], bool first, int col)
 {
     bool ok = true;
     unrolled<0, 16>([&](auto K) {
         constexpr int k = decltype(K)::value;
-        const double p = row_lane<k>(d[k]);
-        ok = ok && p >= 0x1p-900 && p <= 0x1p900;
-        double y = __builtin_amdgcn_rcp(p);
-        y = fma(fma(-p, y, 1.0), y, y);
-        y = fma(fma(-p, y, 1.0), y, y);
-        const double w = d[k] * y;
-        unrolled<k + 1, 16>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            const double f = -row_lane<i>(w);
-            d[i] = fma(f, d[k], d[i]);
-            r[i] = fma(f, r[k], r[i]);
-        });
-        // r keeps pace with d: left to itself the compiler runs all of d first
-        // and holds 120 multipliers for r
-        unrolled<k + 1, 16>([&](auto I) {
-            double &ri = r[decltype(I)::value];
-            asm volatile("" : "+v"(ri));
-        });
-        double &dl = d[15];
-        asm volatile("" : "+v"(dl));
-    });
-    unrolled<0, 16>([&](auto K) {
-        constexpr int k = decltype(K)::value;
         const double p = row_lane<k>(d[k]), y = __builtin_amdgcn_rsq(p);
+        ok = ok && p >= 0x1p-900 && p <= 0x1p900;
         double g = p * y, h = 0.5 * y, e = fma(-h, g, 0.5);
         g = fma(g, e, g);
         h = fma(h, e, h);
         e = fma(-h, g, 0.5);
         g = fma(g, e, g);
         h = fma(h, e, h);
-        const double piv = fma(fma(-g, g, p), h, g);
-        double inv = h + h;
-        inv = fma(fma(-inv, piv, 1.0), inv, inv);
-        const double q = r[k] * inv;
-        r[k] = first && col == k ? piv : fma(fma(-q, piv, r[k]), inv, q);
+        const double piv = fma(fma(-g, g, p), h, g), inv = h + h;
+        const double qd = d[k] * inv, qr = r[k] * inv;
+        const double dk = fma(fma(-qd, piv, d[k]), inv, qd), rk = fma(fma(-qr, piv, r[k]), inv, qr);
+        unrolled<k + 1, 16>([&](auto I) {
+            constexpr int i = decltype(I)::value;
+            const double f = -row_lane<i>(dk);
+            d[i] = fma(f, dk, d[i]);
+            r[i] = fma(f, rk, r[i]);
+        });
+        r[k] = first && col == k ? piv : rk;
+        // r keeps pace with d: left to itself the compiler runs all of d first
+        // and holds 120 multipliers for r
+        unrolled<k, 16>([&](auto I) {
+            double &ri = r[decltype(I)::value];
+            asm volatile("" : "+v"(ri));
+        });
+        double &dl = d[15];
+        asm volatile("" : "+v"(dl));
     });
     return ok;
 }
