@@ -303,8 +303,8 @@ TileChoice tile_choice()
     return kTileAuto;
 }
 
-// How an M x N product from K is cut: the direct-to-LDS tile, and the number
-// of ranges its k is split into.
+// How an M x N product from K is cut: the tile, and the number of ranges its k
+// is split into.
 //
 // A CU that holds w workgroups takes about a + b w microseconds per 16-deep
 // stage: a is what the stage's latency leaves exposed, b the MFMAs of one tile
@@ -319,6 +319,8 @@ TileChoice tile_choice()
 //   3000^3  1070 / 851 / 960    4000^3  1869 / 1951 / 2205    5000 x 5000 x 300
 //   276 / 259 / 284    20000 x 300 x 300  91 / 84 / 83    10000 x 10000 x 500
 //   1515 / 1737 / 1826    8192^3  15150 / 18830 / 21150
+// Register-staged products (below 16 k, single rows) take the same tile: 3 x 12
+// from 1 18.6 / - / 13.2, 1 x 1138 from 16 18.4 / - / 14.4.
 //
 // Splits are tried at 1, 2, 4 and 8 workgroups per CU, each split at least
 // four stages long and all partial products within the buffer; one costs a
@@ -447,9 +449,11 @@ int launch(const GemmArgs &g, TileChoice best)
         if (wb == 4) return launch_dtl<TA, TB, 1, 4, Tile128, 2>(g);
         return launch_dtl<TA, TB, 1, 1, Tile128, 2>(g);
     }
-    switch (tc) {
+    switch (tc == kTileAuto ? best : tc) {
     case kTile256x128: return launch_tile<TA, TB, Tile256x128>(g);
     case kTile128x256: return launch_tile<TA, TB, Tile128x256>(g);
+    case kTile64: return launch_tile<TA, TB, Tile64>(g);
+    case kTile32: return launch_tile<TA, TB, Tile32>(g);
     default: return launch_tile<TA, TB, Tile128>(g);
     }
 }
