@@ -155,7 +155,7 @@ __global__ __launch_bounds__(256) void potrf_row_kernel(double *A, int64_t lda, 
     }
     if (seen > 0 && seen <= j0) return;
     __syncthreads();
-    for (int s = 0; s < kPb; s += 16) {
+    for (int s = 0; s < jb; s += 16) {       // (beyond jb the identity)
         double r[16], d[16];
         bool ok = true;
         if (wave < 2) {
