@@ -63,7 +63,8 @@ __device__ __forceinline__ void unrolled(const F &f)
 }
 
 // 16 steps of the factorization of the 16 x 16 block d, held by every row of
-// 16 lanes (lane = column, register = row), and of the columns r.  False if a
+// 16 lanes (lane = column, register = row), and of the columns r; 8 where no
+// more than 8 rows are not the identity's.  False if a
 // pivot is outside [2^-900, 2^900] (not positive ones among them): r is then
 // of no use.  The square root comes from Goldschmidt's iteration, the quotients
 // from its reciprocal and one correction, which leaves them as the division
@@ -71,10 +72,10 @@ __device__ __forceinline__ void unrolled(const F &f)
 // round off comes back in the rows below.  (Eliminating with d_k / p_k and
 // taking all roots at the end leaves up to four times the backward error for
 // n <= 32, and is no shorter: 18.3 us a block row, 17.4 so.)
-__device__ __forceinline__ bool eliminate16(double (&d)[16], double (&r)[16], bool first, int col)
+__device__ __forceinline__ bool eliminate16(double (&d)[16], double (&r)[16], int rows, bool first, int col)
 {
     bool ok = true;
-    unrolled<0, 16>([&](auto K) {
+    auto step = [&](auto K) __attribute__((always_inline)) {
         constexpr int k = decltype(K)::value;
         const double p = row_lane<k>(d[k]), y = __builtin_amdgcn_rsq(p);
         ok = ok && p >= 0x1p-900 && p <= 0x1p900;
@@ -102,7 +103,9 @@ __device__ __forceinline__ bool eliminate16(double (&d)[16], double (&r)[16], bo
         });
         double &dl = d[15];
         asm volatile("" : "+v"(dl));
-    });
+    };
+    unrolled<0, 8>(step);
+    if (rows > 8) unrolled<8, 16>(step);
     return ok;
 }
 
@@ -139,13 +142,18 @@ __global__ __launch_bounds__(256) void potrf_row_kernel(double *A, int64_t lda, 
     // from clamped places and selected afterwards: a load under a condition
     // would be waited for by itself)
     double dv[kPb / 4], sv[kPb / 4];
-    const double *Sc = nc > 0 ? S : D;
-    const int ri = min(lane, jb - 1), nl = max(nc, 1) - 1;
+    const int ri = min(lane, jb - 1);
 #pragma unroll
     for (int q = 0; q < kPb / 4; ++q) {
         const int j = wave + 4 * q;
         dv[q] = D[(int64_t) min(j, jb - 1) * lda + ri];
-        sv[q] = Sc[(int64_t) min(j, nl) * lda + ri];
+    }
+    if (nc > 0) {
+#pragma unroll
+        for (int q = 0; q < kPb / 4; ++q) sv[q] = S[(int64_t) min(wave + 4 * q, nc - 1) * lda + ri];
+    } else {
+#pragma unroll
+        for (int q = 0; q < kPb / 4; ++q) sv[q] = 0.0;
     }
 #pragma unroll
     for (int q = 0; q < kPb / 4; ++q) {
@@ -164,7 +172,7 @@ __global__ __launch_bounds__(256) void potrf_row_kernel(double *A, int64_t lda, 
                 r[i] = W[s + i][t];
                 d[i] = W[s + i][s + (lane & 15)];
             }
-            ok = eliminate16(d, r, (t & ~15) == s, lane & 15);
+            ok = eliminate16(d, r, jb - s, (t & ~15) == s, lane & 15);
             if (t == 0 && !ok) plain = 1;
         }
         __syncthreads();                   // both waves have read the diagonal block before one stores it
@@ -200,6 +208,7 @@ __global__ __launch_bounds__(256) void potrf_row_kernel(double *A, int64_t lda, 
             __syncthreads();
             break;
         }
+        if (s + 16 >= jb) break;
         // rows below: W(i, j) -= W(s : s + 16, i)^T W(s : s + 16, j) for the
         // block rows bi and the blocks bj >= bi of each
         const int s16 = s / 16;
