@@ -233,14 +233,24 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(GramArgs g, double alp
     const int ksplit = diag ? g.s2 : g.s1;
     const int64_t step = (int64_t) (diag ? g.ntile : g.noff) * (BM * BM);
     const double *q = g.P + (diag ? (int64_t) g.noff * g.s1 + ti : (int64_t) p) * (BM * BM) + e;
-    // sixteen ranges at a time: up to a thousand of them in one chain would cost
-    // the accuracy that short ranges give
+    // sixteen ranges at a time, their loads in flight together: up to a thousand
+    // of them in one chain would cost the accuracy that short ranges give
+    constexpr int U = 16;
     double s = 0.0;
-    for (int k0 = 0; k0 < ksplit; k0 += 16) {
+    int k0 = 0;
+    for (; k0 + U <= ksplit; k0 += U) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = q[(k0 + u) * step];
+#pragma unroll
+        for (int u = 1; u < U; ++u) v[0] = ca3::add_rn(v[0], v[u]);
+        s = ca3::add_rn(s, v[0]);
+    }
+    if (k0 < ksplit) {
         double t = q[k0 * step];
 #pragma unroll 8
-        for (int ks = k0 + 1; ks < min(ksplit, k0 + 16); ++ks) t = ca3::add_rn(t, q[ks * step]);
-        s = k0 ? ca3::add_rn(s, t) : t;
+        for (int ks = k0 + 1; ks < ksplit; ++ks) t = ca3::add_rn(t, q[ks * step]);
+        s = ca3::add_rn(s, t);
     }
     double *c = C + (int64_t) gj * ldc + gi;
     double v = ca3::mul_rn(alpha, s);
