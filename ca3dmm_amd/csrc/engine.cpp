@@ -1277,14 +1277,14 @@ int build_ozaki(ca3dmm_sim *S)
 }
 
 // The per-rank Cannon rounds (step 3 below) as one batched launch unless
-// CA3DMM_SIM_BATCH=0 asks for one hip_dgemm launch per rank and round.
+// CA3DMM_SIM_BATCH=0 asks for one launch (round_product) per rank and round.
 bool batch_on()
 {
     const char *v = getenv("CA3DMM_SIM_BATCH");
     return !(v && !strcmp(v, "0"));
 }
 
-// The problems of the batched launch: exactly the hip_dgemm calls of the
+// The problems of the batched launch: exactly the products of the
 // per-rank rounds, one problem per rank with its q rounds as segments in
 // round order (rounds with k = 0 included).
 int build_batch(ca3dmm_sim *S)

@@ -40,8 +40,8 @@ struct Fold {                 // k-layer reduction of the C blocks of kp problem
 
 struct Tuning {
     int tile = 0;             // workgroup tile: 0 = 128 x 128, 1 = 256 x 128, 2 = 128 x 256 (persistent,
-                              // register-staged); 3 = one batched direct-to-LDS launch of 128 x 128
-                              // tiles (rounds in registers), then the folds as separate launches
+                              // register-staged); 3 = one batched direct-to-LDS launch (128 x 128 or
+                              // smaller tiles, rounds in registers), then the folds as separate launches
     int group_rows = 8;       // tile rows walked together in the queue order
     int wg_per_cu = 2;        // persistent workgroups per CU (1 for the 8-wave tiles)
 };

@@ -125,8 +125,9 @@ int hip_ozaki_gram(const int n, const int k, const double alpha, const double *A
  * ca3dmm_engine_init_BTB (src/ca3dmm.c:1172-1265) and of CholeskyQR
  * (examples/example_CholeskyQR.c:109-117).  Only the upper triangle is
  * computed (n(n+1)k flops); mirror != 0 also writes the lower triangle as an
- * exact copy.  k is split across workgroups and the partials are added in a
- * fixed order, so results are reproducible. */
+ * exact copy.  k is split across workgroups, whose longer ranges are summed in
+ * several chains, and the partials are added in a fixed order, so results are
+ * reproducible. */
 int hip_dsyrk_gram(const int n, const int k, const double alpha, const double *A, const int ldA,
                    const double beta, double *C, const int ldC, int mirror);
 
@@ -138,9 +139,11 @@ int hip_dsyrk_gram(const int n, const int k, const double alpha, const double *A
  * tiles of 128 x 128 doubles, one per GPU the library runs on, held until
  * the process ends) instead of a library allocation.  Shapes needing more
  * than 512 partial tiles (n > 3968 on a 256-CU MI355X) are refused with
- * HIP_PROXY_ERR_ARG.  Every call on a GPU shares that GPU's array: calls that
- * overlap in time on one GPU (two streams, two host threads) race.  Each
- * call writes every partial tile it reads, so nothing needs clearing. */
+ * HIP_PROXY_ERR_ARG.  Every call on a GPU shares that GPU's array, and so does
+ * a single rank's B^T B engine up to that size: calls of several host threads
+ * take it in turn, on the library's stream, but a captured call that is
+ * replayed on another stream races with any that runs meanwhile.  Each call
+ * writes every partial tile it reads, so nothing needs clearing. */
 int hip_dsyrk_gram_noalloc(const int n, const int k, const double alpha, const double *A, const int ldA,
                            const double beta, double *C, const int ldC, int mirror);
 
@@ -174,7 +177,8 @@ int hip_dtrtri_upper(const int n, const double *R, const int ldR, double *X, con
  * *passes_run (may be NULL) receives the number of completed passes.
  * When it can, the call holds a device buffer of m x n doubles (cached
  * across calls) so that each pass writes Q out of place; otherwise, or with
- * CA3DMM_CHOLQR_INPLACE=1, the passes solve in place (same result).
+ * CA3DMM_CHOLQR_INPLACE=1, the passes solve in place (the same up to rounding:
+ * its products may split k, see hip_dgemm).
  * Synchronous (one read-back of the Cholesky's info per pass).  The
  * reference runs one pass and only prints a warning on breakdown
  * (examples/example_CholeskyQR.c:125-129). */

@@ -70,8 +70,8 @@ int ca3dmm_sim_set_mode(ca3dmm_sim_p sim, int grouped, int use_graph);
 
 /* Time the grouped launch over its tunings -- tile 0, 1, 2: the persistent
  * register-staged kernel with workgroup tile 128 x 128 (4 waves), 256 x 128
- * or 128 x 256 (8 waves); tile 3: one batched direct-to-LDS launch of
- * 128 x 128 tiles with the rounds accumulated in registers, then the fold
+ * or 128 x 256 (8 waves); tile 3: one batched direct-to-LDS launch of 128 x
+ * 128 or smaller tiles with the rounds accumulated in registers, then the fold
  * launches (the same bits); tile rows walked together: 1, 4, 8, 16;
  * persistent workgroups per CU: 1, 2 (tile 0 only) -- keep the fastest for
  * this grid's shape signature, in memory and in the tuning table on disk

@@ -9,10 +9,12 @@
  *     (reference: src/cuda_utils.h:23-35);
  *   - all kernels are this library's own HIP kernels; no vendor BLAS,
  *     solver or random-number library is called;
- *   - work runs on one library-owned stream per device (default priority).
- *     By default each entry synchronises that stream before returning, as
+ *   - work runs on one library-owned stream per device (default priority);
+ *     entries may be called from several threads, which share that stream and
+ *     the library's buffers in turn;
+ *   - by default each entry synchronises that stream before returning, as
  *     the reference's BLAS proxies do (cuda_proxy.cu:184,229); after
- *     hip_proxy_set_sync(0) entries return as soon as the work is queued and
+ *     hip_proxy_set_sync(0), for the whole process, entries return as soon as the work is queued and
  *     hip_stream_sync(NULL) waits for it.
  * Pointers are plain device (or pinned host) addresses; sizes are in
  * elements unless named *bytes.
@@ -105,11 +107,12 @@ int hip_dcopy(const int n, const double *x, const int incx, double *y, const int
 
 /* cuda_proxy.h:92-97 (cuda_cublas_dgemm, cuda_proxy.cu:211-230):
  * column-major C := alpha*op(A)*op(B) + beta*C, FP64 MFMA, all four
- * transA/transB cases (HipNoTrans / HipTrans).  The sums run in a fixed order
- * that depends on m, n and k alone.  Where C is small and k long, k is split
- * over workgroups, whose partial sums pass through a device buffer of 64 MiB
- * that the library allocates once and keeps; without it, and under stream
- * capture, the same product runs unsplit. */
+ * transA/transB cases (HipNoTrans / HipTrans).  Where C is small and k long, k
+ * is split over workgroups, whose partial sums pass through a device buffer of
+ * 64 MiB that the library allocates at the first such call and keeps.  The sums
+ * run in an order that is fixed for given m, n and k on a device (its number of
+ * CUs decides the split); without that buffer, and under stream capture, the
+ * product runs unsplit, whose last bits differ. */
 int hip_dgemm(hip_proxy_enum_t transA, hip_proxy_enum_t transB,
               const int m, const int n, const int k, const double alpha,
               const double *A, const int ldA, const double *B, const int ldB,
@@ -136,7 +139,10 @@ int hip_dtrsm(hip_proxy_enum_t side, hip_proxy_enum_t uplo,
 /* cuda_proxy.h:117 (cuda_cusolver_dpotrf): Cholesky A = R^T R in place,
  * uplo 'U' (the strictly lower part is not referenced).  Returns LAPACK's
  * info: 0 on success, i > 0 when the leading minor of order i is not
- * positive definite, < 0 on an argument or runtime error.  n <= 8192. */
+ * positive definite, < 0 on an argument or runtime error.  After a breakdown
+ * the whole blocks of 64 rows before the failing one are the factor's, and so
+ * are, within its 64 columns, the failing block's rows before the pivot; the
+ * rest of the upper triangle is what remains of A after those.  n <= 8192. */
 int hip_dpotrf(const char uplo, const int n, double *A, const int ldA);
 
 #ifdef __cplusplus
